@@ -107,10 +107,10 @@ def _mix_shapes(case):
 
 
 def _matrix(gen, rows, cols, dtype, dist="uniform"):
-    if dist == "wide":
-        e = torch.randint(-20, 21, (rows, cols), generator=gen, device="cuda", dtype=torch.int32)
-        s = torch.randint(0, 2, (rows, cols), generator=gen, device="cuda", dtype=torch.int32) * 2 - 1
-        return torch.ldexp(s.to(dtype), e)
+    if dist == "wide":  # sign * 2^e from its FP64 bits, so that every value is exact
+        e = torch.randint(-20, 21, (rows, cols), generator=gen, device="cuda")
+        s = torch.randint(0, 2, (rows, cols), generator=gen, device="cuda")
+        return ((s << 63) | ((e + 1023) << 52)).view(torch.float64).to(dtype)
     return torch.empty((rows, cols), dtype=dtype, device="cuda").uniform_(-1.0, 1.0, generator=gen)
 
 
