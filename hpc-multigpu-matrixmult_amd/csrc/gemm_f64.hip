@@ -1,12 +1,13 @@
-// FP64 GEMM on gfx950 matrix cores: C += A*B, grouped and persistent.
+// FP64 GEMM on gfx950 matrix cores: C += A*B, one launch for any number of GEMMs.
 //
 // Replaces the reference's gemm_kernel (src/phpc_gemm.cu:6-57). The reference gives
 // each thread one output and walks the K dimension in T-wide shared-memory phases.
 // Here a workgroup owns a BM x BN macro tile, its waves own 16x16 MFMA sub-tiles
-// (v_mfma_f64_16x16x4f64), operands are staged through LDS in BK=16 slabs with
-// double buffering, and the workgroups form a persistent grid that walks a flat list
-// of tiles covering any number of GEMMs (one launch for all SUMMA ranks, or for a
-// batch of unrelated GEMMs).
+// (v_mfma_f64_16x16x4f64), operands are staged through LDS in slabs of k, and the
+// workgroups share a flat list of tiles covering any number of GEMMs (one launch for all
+// SUMMA ranks, or for a batch of unrelated GEMMs). Two kernels: f64_rm_kernel copies slabs
+// HBM -> LDS directly and runs everything the planner picks; f64_gemm_kernel stages them
+// through registers and is kept as the fixed configurations that it is compared with.
 //
 // Arithmetic. v_mfma_f64_16x16x4f64 computes, per output, the FMA chain
 // d = fma(a3,b3, fma(a2,b2, fma(a1,b1, fma(a0,b0,c)))) in k order (measured on the
@@ -16,14 +17,15 @@
 // (src/phpc_gemm.cu:32,50-51,55). Zero padding of partial slabs adds fma(0,0,c) = c,
 // as the reference's own tile padding does (:38-46).
 //
-// Layout. Row-major, arbitrary leading dimensions. LDS holds A transposed
-// (At[k][m]) and B as is (Bs[k][n]) so each MFMA operand fetch is 16 consecutive
-// doubles per lane group.
+// Layout. Row-major, arbitrary leading dimensions. The register-staged kernel's LDS holds A
+// transposed (At[k][m]) and B as is (Bs[k][n]) so each MFMA operand fetch is 16 consecutive
+// doubles per lane group; the direct kernel's layout is described with it.
 #include "phpc_internal.h"
 
 #include <algorithm>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 typedef double d4 __attribute__((ext_vector_type(4)));
@@ -31,12 +33,13 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 namespace {
 
 struct GemmBatch {
-  const GemmDesc *descs;  // device array (ndesc > 1)
+  const GemmDesc *descs;  // device array (ndesc > 2)
   int ndesc;
   int total_tiles;
   int group_m;            // tile-row swizzle width
   int xcd_remap;          // 1: contiguous tile runs per XCD
-  GemmDesc d0;            // inline copy when ndesc == 1
+  int tail_start;         // row-major kernels: tiles from here on have the tail's shape
+  GemmDesc d0, d1;        // inline copies when there are at most two (ndesc <= 2)
 };
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
@@ -109,7 +112,7 @@ __device__ __forceinline__ T *uni(T *p) {
 
 // Decode global tile id -> (descriptor, tile row, tile col).
 __device__ __forceinline__ const GemmDesc *find_desc(const GemmBatch &b, int t) {
-  if (b.ndesc == 1) return &b.d0;
+  if (b.ndesc <= 2) return b.ndesc == 2 && t >= b.d1.tile_start ? &b.d1 : &b.d0;
   int lo = 0, hi = b.ndesc - 1;
   while (lo < hi) {
     int mid = (lo + hi + 1) >> 1;
@@ -340,23 +343,6 @@ __global__ __launch_bounds__(WM *WN * 64) __attribute__((amdgpu_waves_per_eu(2))
   }
 }
 
-// ---------------------------------------------------------------------------
-// Direct-to-LDS variant (16-byte aligned operands, even k and n).
-//
-// Slabs are copied HBM -> LDS by buffer_load_dwordx4 ... lds: each wave instruction
-// fills one contiguous 1 KiB LDS block, lane p writing bytes [16p, 16p+16). Which
-// global 16-byte chunk each lane fetches is free, so the lane -> address map sets
-// the LDS layout. No registers stage the data, so STAGES slabs can be in flight.
-//
-// LDS layout of one stage, in 16-byte chunks:
-//   A: BM rows x 16 doubles. Rows go in pairs of 17 chunks (8 + 8 + 1 pad), row r at
-//      chunk (r/2)*17 + (r%2)*8. A 16-lane MFMA operand read (16 rows, one k) then
-//      touches 16 distinct 8-byte bank slots, and k steps are plain address offsets.
-//   B: 16 rows x BN doubles, row k at chunk k*BN/2, chunk c at slot c ^ ((k&1)<<3), so
-//      the two 16-lane groups of a half-wave (rows k, k+1) use opposite bank halves.
-// Blocks of a stage are dealt to waves round-robin; pad chunks are fetched with an
-// out-of-range offset (zero) and never read.
-// ---------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) void lds_void;
 
 // s_waitcnt vmcnt(N) leaving expcnt and lgkmcnt unconstrained (gfx9 encoding: vmcnt
@@ -376,91 +362,123 @@ __device__ __forceinline__ void wait_vm_c() {
 // from moving memory operations across it.
 __device__ __forceinline__ void slab_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
-template <int BM, int BN_, int WM, int WN, int STAGES, bool MP>
-struct F64Lds {
-  static constexpr int BK = 16;
-  static constexpr int BN = BN_;
-  static constexpr int NT = WM * WN * 64;
+// ---------------------------------------------------------------------------
+// Row-major direct-to-LDS kernels: A and B are read where they lie, any leading dimension
+// and any (8-byte) alignment. Slabs are copied HBM -> LDS by 16-byte buffer loads, which
+// need 4-byte aligned addresses only: each wave instruction fills one contiguous 1 KiB LDS
+// block, lane p writing bytes [16p, 16p+16), and the lane -> address map sets the layout.
+//
+// LDS layout of one stage, in 16-byte chunks:
+//   A: BM rows x BK doubles, CPR = BK/2 chunks per row, chunk c of row r at slot
+//      c ^ sw(r), sw(r) = (r * CPR / 16) mod CPR: the 32 lanes of a half-wave of an MFMA
+//      operand read (16 rows, one chunk, both halves) cover all 64 banks once.
+//   B: BK rows x BN doubles, chunk c of row k at slot c ^ ((k & 1) << 3), so the two
+//      16-lane groups of a half-wave (rows k, k+1) use opposite bank halves.
+// A slab with fewer than BK k rows (the end of a panel) takes 4-byte loads into the same
+// layout, each checked against k, rows and columns, so padding is exact zeros in both
+// operands. So does the last slab of a GEMM with an odd n whose B rows are not 16-byte
+// aligned: there a 16-byte load of the last column would read past the last row's end.
+//
+// What bounds it. An FP64 MFMA holds its SIMD's vector pipe for 64 cycles, and a vector
+// instruction of any kind waits for the MFMA before it to leave: one address addition per
+// MFMA makes 64 cycles 99 (measured on one wave), while LDS reads, loads to LDS and scalar
+// instructions issue beside it for nothing. So the loop over full slabs holds MFMAs, LDS
+// reads at a lane's constant address plus an immediate, loads at a lane's constant offset
+// plus a scalar one, and nothing vector: every stage of the ring has its own copy of the code.
+// Operands are read ahead of their MFMAs and across the slab barrier (the barrier of slab s
+// waits for slab s + 1), since in a small problem one wave per SIMD has nothing else to hide
+// LDS latency with. At the full MFMA rate a CU on 256x128 tiles loads 14 GB/s, one on 32x32
+// tiles 74, half of what its loads to LDS reach from L2 (150): hence large tiles where there
+// are enough of them.
+//
+// Measured (MI355X, whole call, before -> after; before: A staged transposed by a kernel of
+// its own, or the address arithmetic in the loop):
+//   N = 256     16.0 -> 6.2 us          N = 1024     68 -> 41 us
+//   N = 2048     277 -> 240 us          N = 4096   2.05 -> 1.88 ms (73 TFLOP/s)
+//   N = 16384  123.8 -> 117.5 ms (74.8 TFLOP/s, 95% of the FP64 peak)
+// ---------------------------------------------------------------------------
+template <int BM, int BN, int WM, int WN, int BK_, int STAGES_>
+struct F64Rm {
+  static constexpr int BK = BK_;
+  static constexpr int STAGES = STAGES_;
   static constexpr int NW = WM * WN;
-  static constexpr int WTM = BM / WM;
-  static constexpr int WTN = BN_ / WN;
-  static constexpr int TM = WTM / 16;
-  static constexpr int TN = WTN / 16;
-  static constexpr int A_CHUNKS = (BM / 2) * 17;
-  static constexpr int A_BLOCKS = (A_CHUNKS + 63) / 64;
-  static constexpr int A_BYTES = A_BLOCKS * 1024;
-  static constexpr int B_BLOCKS = BK * BN_ * 8 / 1024;
-  static constexpr int B_BYTES = B_BLOCKS * 1024;
-  static constexpr int STAGE_BYTES = A_BYTES + B_BYTES;
-  static constexpr int BLOCKS = A_BLOCKS + B_BLOCKS;
-  static constexpr int PER_LO = BLOCKS / NW;                  // blocks per wave (low)
-  static constexpr int PER_HI = (BLOCKS + NW - 1) / NW;       // blocks per wave (high)
-  static_assert(BN_ % 32 == 0 && BM % 32 == 0, "tile shape");
-  static_assert(STAGES >= 2 && STAGES <= 4, "pipeline depth");
-  static_assert(STAGES * STAGE_BYTES <= 160 * 1024, "LDS budget");
+  static constexpr int WTM = BM / WM, WTN = BN / WN;
+  static constexpr int TM = WTM / 16, TN = WTN / 16;
+  static constexpr int CPR = BK / 2, CPB = BN / 2;       // chunks per A row, per B row
+  static constexpr int ARB = 64 / CPR, BRB = 64 / CPB;   // A rows, B rows per 1 KiB block
+  static constexpr int A_BYTES = BM * BK * 8, B_BYTES = BK * BN * 8;  // of a stage; A's stages, then B's
+  static constexpr int B_BASE = STAGES * A_BYTES;
+  static constexpr int LDS_BYTES = STAGES * (A_BYTES + B_BYTES);
+  static constexpr int PA = A_BYTES / 1024 / NW, PB = B_BYTES / 1024 / NW;  // 1 KiB blocks per wave
+  static constexpr int PER = PA + PB;
+  static constexpr int KSTEPS = BK / 4;
+  static_assert(CPR == 8 || CPR == 16, "slab depth");
+  static_assert(CPB >= 16 && CPB <= 64 && BM % (NW * ARB) == 0 && BK % (NW * BRB) == 0, "blocks split evenly");
+  static_assert((NW * ARB) % 16 == 0 && (NW * BRB) % 2 == 0, "a wave's blocks share their swizzle");
+  static_assert(TM >= 1 && TN >= 1, "wave tile");
+  // Operand sets in registers: set kk % RING holds k step kk, and behind step kk's MFMAs the
+  // set of step kk - 1 is refilled with step kk + RING - 1. The fewer MFMAs a k step has, the
+  // further ahead its operands are read. Two stages leave no slab to read ahead from: the
+  // operands of a slab are read after its own barrier.
+  static constexpr bool AHEAD = STAGES >= 3;
+  static constexpr int RING = TM * TN >= 4 ? 2 : TM * TN == 2 ? 4 : KSTEPS;
+  static_assert(KSTEPS % RING == 0, "operand ring");
+  static_assert(STAGES >= 2 && (STAGES + 1) * PER < 64 && LDS_BYTES <= 160 * 1024, "pipeline depth");
 };
 
-// wait until at most `n` vector-memory operations of this thread are outstanding,
-// n = later * per with per in {PER_LO, PER_HI} and later <= STAGES-2
-template <int LO, int HI>
-__device__ __forceinline__ void wait_outstanding(int later, int per) {
-  const int n = later * per;
-  if (n <= 0) { wait_vm_c<0>(); return; }
-  if (n == LO) { wait_vm_c<LO>(); return; }
-  if (n == HI) { wait_vm_c<HI>(); return; }
-  if (n == 2 * LO) { wait_vm_c<2 * LO>(); return; }
-  if (n == 2 * HI) { wait_vm_c<2 * HI>(); return; }
-  wait_vm_c<0>();
+// wait until at most `units` * PER vector-memory operations are outstanding (units <= MAX)
+template <int PER, int MAX>
+__device__ __forceinline__ void wait_units(int units) {
+  if constexpr (MAX == 0) {
+    wait_vm_c<0>();
+  } else {
+    if (units >= MAX)
+      wait_vm_c<MAX * PER>();
+    else
+      wait_units<PER, MAX - 1>(units);
+  }
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES, bool MP>
-__global__ __launch_bounds__(WM *WN * 64) __attribute__((amdgpu_waves_per_eu(2))) void f64_lds_kernel(
-    GemmBatch batch) {
-  using K = F64Lds<BM, BN, WM, WN, STAGES, MP>;
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
+// f(integral_constant 0), ..., f(integral_constant N - 1)
+template <int N, class F>
+__device__ __forceinline__ void for_stages(const F &f) {
+  if constexpr (N > 0) {
+    for_stages<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
+}
 
+// One BM x BN tile at (row0, col0) of GEMM d, all of them uniform.
+template <int BM, int BN, int WM, int WN, int BK, int STAGES, bool MP>
+__device__ __forceinline__ void f64_rm_tile(const GemmDesc &d, int row0, int col0) {
+  using K = F64Rm<BM, BN, WM, WN, BK, STAGES>;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int tid = threadIdx.x;
-  const int wave = uni(tid >> 6);  // wave-uniform: keeps LDS block bases scalar
+  const int wave = uni(tid >> 6);
   const int lane = tid & 63;
   const int g = lane >> 4;
   const int li = lane & 15;
+  // waves 0, 4, 8, ... share a SIMD: the column index is rotated so that the waves of one tile
+  // row or column, all that is left of a tile at the matrix edge, lie on different SIMDs
   const int wm = wave / WN;
-  const int wn = wave % WN;
-  // blocks owned by this wave: wave, wave + NW, ... (uniform per wave)
-  const int my_blocks = (K::BLOCKS - wave + K::NW - 1) / K::NW;
+  const int wn = (wave + (WN % 4 == 0 ? wm : wave / 4)) % WN;
+  auto swz = [](int r) { return (r * K::CPR / 16) & (K::CPR - 1); };
 
-  // per-lane LDS read offsets (bytes, stage-relative); k steps add constants
-  int a_off[K::TM], b_off[K::TN];
+  // LDS operand offsets of this lane (stage-relative bytes); blocks of 16 rows, and the k
+  // steps of B, add constants
+  int a_off[K::KSTEPS], b_off[K::TN];
 #pragma unroll
-  for (int i = 0; i < K::TM; ++i) {
-    const int r = wm * K::WTM + i * 16 + li;
-    a_off[i] = ((r >> 1) * 17 + (r & 1) * 8) * 16 + g * 8;
-  }
+  for (int kk = 0; kk < K::KSTEPS; ++kk)
+    a_off[kk] = (wm * K::WTM + li) * BK * 8 + (((2 * kk + (g >> 1)) ^ swz(li)) << 4) + (g & 1) * 8;
 #pragma unroll
   for (int j = 0; j < K::TN; ++j) {
     const int col = wn * K::WTN + j * 16 + li;
-    b_off[j] = K::A_BYTES + g * K::BN * 8 + ((((col >> 1) ^ ((g & 1) << 3))) << 4) + (col & 1) * 8;
+    b_off[j] = K::B_BASE + g * BN * 8 + (((col >> 1) ^ ((g & 1) << 3)) << 4) + (col & 1) * 8;
   }
-
-  const int G = gridDim.x;
-  const int bid = blockIdx.x;
-  const bool xcd_remap = batch.xcd_remap && (G % 8) == 0;
-  const int slot = uni(xcd_remap ? (bid % 8) * (G / 8) + bid / 8 : bid);
-
-  for (int round = 0;; ++round) {
-    const int t = round * G + slot;
-    if (t >= batch.total_tiles) break;
-    const GemmDesc d = uniform_desc(batch, uni(t));
-    const int lt = t - d.tile_start;
-    const int tiles_n = d.tiles_n;
-    const int tiles_m = (d.m + BM - 1) / BM;
-    const int gm = batch.group_m;
-    const int grp = lt / (gm * tiles_n);
-    const int first_m = grp * gm;
-    const int gsz = min(tiles_m - first_m, gm);
-    const int in_grp = lt - grp * gm * tiles_n;
-    const int row0 = (first_m + in_grp % gsz) * BM;
-    const int col0 = (in_grp / gsz) * BN;
+  // this lane's row and chunk in the wave's first A block and first B block
+  const int ar = wave * K::ARB + lane / K::CPR, ac = (lane % K::CPR) ^ swz(ar);
+  const int br = wave * K::BRB + lane / K::CPB, bc = (lane % K::CPB) ^ ((br & 1) << 3);
+  {
     const int m_rem = uni(d.m - row0);
     const int n_rem = uni(d.n - col0);
     const long lda = uni(d.lda), ldb = uni(d.ldb), ldc = uni(d.ldc);
@@ -469,291 +487,160 @@ __global__ __launch_bounds__(WM *WN * 64) __attribute__((amdgpu_waves_per_eu(2))
     gdouble *Cg = (gdouble *)(uni(d.C) + (long)row0 * ldc + col0);
     const int Kdim = uni(d.k);
     const int dpanel = uni(d.panel);
-    const int w = dpanel > 0 && dpanel < Kdim ? dpanel : Kdim;
-    const rsrc_t rA = make_rsrc(Ag, (long)min(m_rem, BM) * lda * 8);
+    const int w = MP && dpanel > 0 && dpanel < Kdim ? dpanel : Kdim;
+    const int spp = (w + BK - 1) / BK;  // slabs per full panel
+    const int full_panels = MP ? Kdim / w : 1;
+    const int nslab = MP ? uni(full_panels * spp + (Kdim - full_panels * w + BK - 1) / BK) : spp;
+    const int last_panel = MP && Kdim % w ? Kdim % w : w;
+    const bool exact_last = (d.n & 1) && (((reinterpret_cast<uintptr_t>(Bg) >> 3) | ldb) & 1);
 
-    // Per-lane global offsets of this wave's blocks for a full slab starting at k = 0
-    // (A: add kb*8 through soffset; B: the descriptor base moves to row kb). For a
-    // partial slab the k bound is applied on top (kcol < krem).
-    uint32_t goff[K::PER_HI];
-    int gk[K::PER_HI];  // k column (A) or k row (B) of the chunk; -1 for pad chunks
+    // Every 1 KiB block is addressed from its own first row (ARB or BRB rows, uniform), so one
+    // lane offset serves all of an operand's blocks. A rows past m_rem lie at or beyond
+    // num_records and read zero (k rides in the scalar offset, which the range check leaves
+    // out); B chunks past n_rem go out of range here.
+    rsrc_t rA[K::PA];
 #pragma unroll
-    for (int u = 0; u < K::PER_HI; ++u) {
-      const int blk = wave + u * K::NW;
-      goff[u] = kOOB;
-      gk[u] = 1 << 30;
-      if (blk < K::A_BLOCKS) {
-        const int q = blk * 64 + lane;  // chunk slot in the A region
-        const int pr = q / 17, pc = q % 17;
-        const int row = 2 * pr + (pc >= 8 ? 1 : 0);
-        const int c = pc >= 8 ? pc - 8 : pc;
-        if (pc < 16 && q < K::A_CHUNKS && row < m_rem) {
-          goff[u] = (uint32_t)(((long)row * lda + 2 * c) * 8);
-          gk[u] = 2 * c;
-        }
-      } else if (blk < K::BLOCKS) {
-        const int q = (blk - K::A_BLOCKS) * 64 + lane;
-        const int kr = q / (BN / 2);
-        const int c = (q % (BN / 2)) ^ ((kr & 1) << 3);
-        if (2 * c < n_rem) {
-          goff[u] = (uint32_t)(((long)kr * ldb + 2 * c) * 8);
-          gk[u] = kr;
-        }
-      }
+    for (int u = 0; u < K::PA; ++u) {
+      const int r0 = (wave + u * K::NW) * K::ARB;
+      rA[u] = make_rsrc(Ag + (long)r0 * lda, (long)min(m_rem - r0, K::ARB) * lda * 8);
     }
+    const uint32_t ga = (uint32_t)(((long)(lane / K::CPR) * lda + 2 * ac) * 8);
+    const uint32_t gb = 2 * bc < n_rem ? (uint32_t)(((long)(lane / K::CPB) * ldb + 2 * bc) * 8) : kOOB;
 
-    d4 acc[K::TM][K::TN];
-    d4 creg[MP ? K::TM : 1][MP ? K::TN : 1];
-#pragma unroll
-    for (int i = 0; i < K::TM; ++i)
-#pragma unroll
-      for (int j = 0; j < K::TN; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-    if constexpr (MP) {
-#pragma unroll
-      for (int i = 0; i < K::TM; ++i)
-#pragma unroll
-        for (int j = 0; j < K::TN; ++j) {
-          const int cc = wn * K::WTN + j * 16 + li;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int rr = wm * K::WTM + i * 16 + 4 * r + g;
-            creg[i][j][r] = (rr < m_rem && cc < n_rem) ? Cg[(long)rr * ldc + cc] : 0.0;
-          }
-        }
-    }
-
-    const int spp = (w + K::BK - 1) / K::BK;  // slabs per full panel
-    const int full_panels = Kdim / w;
-    const int tail = Kdim - full_panels * w;
-    const int nslab = full_panels * spp + (tail + K::BK - 1) / K::BK;
-
-    auto issue = [&](int sidx) {
-      const int p = sidx / spp;
-      const int kb = p * w + (sidx - p * spp) * K::BK;
-      const int krem = min(min(kb + K::BK, p * w + w), Kdim) - kb;
-      char *stage = smem + (sidx % STAGES) * K::STAGE_BYTES;
-      const rsrc_t rB = make_rsrc(Bg + (long)kb * ldb, (long)krem * ldb * 8);
-#pragma unroll
-      for (int u = 0; u < K::PER_HI; ++u) {
-        const int blk = wave + u * K::NW;
-        if (u < K::PER_LO || blk < K::BLOCKS) {
-          const uint32_t off = gk[u] < krem ? goff[u] : kOOB;
-          if (blk < K::A_BLOCKS)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, (lds_void *)(stage + blk * 1024), 16, off, kb * 8, 0, 0);
-          else
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, (lds_void *)(stage + blk * 1024), 16, off, 0, 0, 0);
-        }
-      }
+    // the next slab to issue: its first k row, the end of its panel, its stage
+    int ikb = 0, ipe = min(w, Kdim), istage = 0;
+    const double *iB = Bg;
+    auto rsrc_b = [&](int u) {
+      return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(iB + (long)(wave + u * K::NW) * K::BRB * ldb),
+                                               (short)0, 0x7fffffff, 0x00020000);
     };
-
-    auto mfma_step = [&](const char *stage, int kk) {
-      double a[K::TM], b[K::TN];
+    // block u of a full slab: A's, then B's
+    auto load_block = [&](int u, int q) {
+      if (u < K::PA)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rA[u], (lds_void *)(smem + q * K::A_BYTES + (wave + u * K::NW) * 1024), 16, ga,
+                                                  ikb * 8, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rsrc_b(u - K::PA), (lds_void *)(smem + K::B_BASE + q * K::B_BYTES + (wave + (u - K::PA) * K::NW) * 1024),
+            16, gb, 0, 0, 0);
+    };
+    auto advance = [&](int rows) {
+      ikb += rows;
+      iB += rows * ldb;
+    };
+    auto issue = [&]() {
+      const int krem = min(BK, ipe - ikb);
+      if (krem == BK && !(exact_last && ikb + BK >= Kdim)) {
 #pragma unroll
-      for (int i = 0; i < K::TM; ++i) a[i] = *reinterpret_cast<const double *>(stage + a_off[i] + kk * 32);
+        for (int u = 0; u < K::PER; ++u) load_block(u, istage);
+      } else {
 #pragma unroll
-      for (int j = 0; j < K::TN; ++j)
-        b[j] = *reinterpret_cast<const double *>(stage + b_off[j] + kk * 4 * K::BN * 8);
+        for (int u = 0; u < K::PA; ++u)
+#pragma unroll 1
+          for (int v = 0; v < 4; ++v) {
+            const int pos = v * 16 + (lane >> 2), r0 = (wave + u * K::NW) * K::ARB, r = pos / K::CPR;
+            const int c = (pos % K::CPR) ^ swz(r0 + r);
+            const uint32_t off = r0 + r < m_rem && 2 * c + ((lane >> 1) & 1) < krem
+                                     ? (uint32_t)((long)r * lda * 8 + c * 16 + (lane & 3) * 4)
+                                     : kOOB;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rA[u], (lds_void *)(smem + istage * K::A_BYTES + (wave + u * K::NW) * 1024 + v * 256), 4, off,
+                ikb * 8, 0, 0);
+          }
 #pragma unroll
-      for (int i = 0; i < K::TM; ++i)
-#pragma unroll
-        for (int j = 0; j < K::TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+        for (int u = 0; u < K::PB; ++u)
+#pragma unroll 1
+          for (int v = 0; v < 4; ++v) {
+            const int pos = v * 16 + (lane >> 2), r0 = (wave + u * K::NW) * K::BRB, r = pos / K::CPB;
+            const int c = (pos % K::CPB) ^ (((r0 + r) & 1) << 3);
+            const uint32_t off = r0 + r < krem && 2 * c + ((lane >> 1) & 1) < n_rem
+                                     ? (uint32_t)((long)r * ldb * 8 + c * 16 + (lane & 3) * 4)
+                                     : kOOB;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rsrc_b(u), (lds_void *)(smem + K::B_BASE + istage * K::B_BYTES + (wave + u * K::NW) * 1024 + v * 256), 4,
+                off, 0, 0, 0);
+          }
+      }
+      advance(krem);
+      istage = istage + 1 == STAGES ? 0 : istage + 1;
+      if (MP && ikb == ipe) ipe = min(ipe + w, Kdim);
     };
 
     // every wave must be done reading the previous tile's stages before refilling them
     slab_barrier();
-#pragma unroll
-    for (int s0 = 0; s0 < STAGES - 1; ++s0)
-      if (s0 < nslab) issue(s0);
+    const int last_units = last_panel % BK || exact_last ? 3 : 0;  // extra loads of a last slab in 4-byte pieces
+#pragma unroll 1
+    for (int s0 = 0; s0 < STAGES - 1 && s0 < nslab; ++s0) issue();
 
-    for (int sidx = 0; sidx < nslab; ++sidx) {
-      // loads of slab sidx are complete once at most the later slabs' are in flight
-      wait_outstanding<K::PER_LO, K::PER_HI>(min(STAGES - 2, nslab - 1 - sidx), my_blocks);
-      slab_barrier();
-      if (sidx + STAGES - 1 < nslab) issue(sidx + STAGES - 1);
-      const int p = sidx / spp;
-      const int j = sidx - p * spp;
-      const int kb = p * w + j * K::BK;
-      const int pe = min(p * w + w, Kdim);
-      const int klen = min(kb + K::BK, pe) - kb;
-      const char *stage = smem + (sidx % STAGES) * K::STAGE_BYTES;
-      // k beyond the slab reads as zero (out-of-range loads), so a partial slab simply
-      // adds fma(0, 0, c) = c terms, like the reference kernel's own tile padding
-#pragma unroll
-      for (int kk = 0; kk < K::BK / 4; ++kk) mfma_step(stage, kk);
-      if constexpr (MP) {
-        if (kb + klen == pe) {
-#pragma unroll
-          for (int i = 0; i < K::TM; ++i)
-#pragma unroll
-            for (int jj = 0; jj < K::TN; ++jj) {
-              creg[i][jj] = creg[i][jj] + acc[i][jj];
-              acc[i][jj] = d4{0.0, 0.0, 0.0, 0.0};
+    int issued = min(STAGES - 1, nslab);
+    // slab t has landed once the slabs issued after it are all that is outstanding
+    auto wait_slab = [&](int t) {
+      const int later = issued - 1 - t;
+      wait_units<K::PER, STAGES + 1>(later > 0 && issued == nslab ? later + last_units : later);
+    };
+    const int k16 = Kdim - (exact_last ? 1 : 0);  // a slab that ends past it takes 4-byte loads
+    // walk the slabs, STAGES at a time while the slabs that they issue are full ones of one
+    // panel; compute(stage, steady) is a slab's work behind its barrier
+    auto walk = [&](auto compute) {
+      int t = 0;  // the slab, in stage 0 at the head of this loop
+#pragma unroll 1
+      while (t < nslab) {
+#pragma unroll 1
+        while (ikb + STAGES * BK <= min(ipe, k16)) {
+          for_stages<STAGES>([&](auto qc) { compute(qc, std::true_type{}); });
+          t += STAGES;
+          if (MP && ikb == ipe) ipe = min(ipe + w, Kdim);
+        }
+        istage = STAGES - 1;  // slab t + STAGES - 1's
+        for_stages<STAGES>([&](auto qc) {
+          if (t < nslab) {
+            if (!K::AHEAD || t + 1 < nslab) wait_slab(K::AHEAD ? t + 1 : t);
+            slab_barrier();
+            if (issued < nslab) {
+              issue();
+              ++issued;
             }
-        }
-      }
-    }
-
-#pragma unroll
-    for (int i = 0; i < K::TM; ++i)
-#pragma unroll
-      for (int jj = 0; jj < K::TN; ++jj) {
-        const int cc = wn * K::WTN + jj * 16 + li;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int rr = wm * K::WTM + i * 16 + 4 * r + g;
-          if (rr < m_rem && cc < n_rem) {
-            gdouble *pc = Cg + (long)rr * ldc + cc;
-            if constexpr (MP)
-              *pc = creg[i][jj][r];
-            else
-              *pc = *pc + acc[i][jj][r];
+            compute(qc, std::false_type{});
+            ++t;
           }
-        }
+        });
       }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Transposed-A direct-to-LDS variant. The caller stores A transposed (At[k][m], row
-// pitch = the descriptor's lda, 16-byte aligned rows, pad columns zero), so both
-// operand slabs are k-row-major and are copied HBM -> LDS by 16-byte buffer loads
-// with no register staging and no LDS write instructions: each wave instruction fills
-// one contiguous 1 KiB piece of a k row. LDS rows are padded by 64 bytes. The MFMA
-// operand reads are the register-staged kernel's (16 consecutive doubles per lane
-// group), so the arithmetic is identical. STAGES slabs of BK k rows ring through LDS:
-// slab s + STAGES - 1 is issued while slab s is computed (two stages: a slab's loads land
-// while the previous slab is computed). MP: k is walked in panels, each panel's sum starts
-// from zero and is added to the C value carried in registers (as the register-staged MP
-// kernels).
-// ---------------------------------------------------------------------------
-template <int BM, int BN, int WM, int WN, int STAGES_ = 2, int BK_ = 16>
-struct F64At {
-  static constexpr int BK = BK_;
-  static constexpr int STAGES = STAGES_;
-  static constexpr int NW = WM * WN;
-  static constexpr int WTM = BM / WM, WTN = BN / WN;
-  static constexpr int TM = WTM / 16, TN = WTN / 16;
-  static constexpr int AP = BM + 8, BP = BN + 8;  // LDS row pitches (doubles)
-  static constexpr int A_BYTES = BK * AP * 8;
-  static constexpr int STAGE_BYTES = A_BYTES + BK * BP * 8;
-  static constexpr int A_PIECES = BM / 128, B_PIECES = BN / 128;  // 1 KiB pieces per k row
-  static constexpr int A_BLOCKS = BK * A_PIECES, BLOCKS = A_BLOCKS + BK * B_PIECES;
-  static constexpr int PER = BLOCKS / NW;
-  static_assert(BM % 128 == 0 && BN % 128 == 0 && BLOCKS % NW == 0, "tile shape");
-  static_assert(STAGES * STAGE_BYTES <= 160 * 1024, "LDS budget");
-  static_assert(STAGES >= 2 && (STAGES - 2) * PER < 64 && BK % 4 == 0, "pipeline depth");
-};
-
-template <int BM, int BN, int WM, int WN, bool MP, int STAGES = 2, int BK = 16>
-__device__ __forceinline__ void f64_at_body(const GemmBatch &batch) {
-  using K = F64At<BM, BN, WM, WN, STAGES, BK>;
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int tid = threadIdx.x;
-  const int wave = uni(tid >> 6);
-  const int lane = tid & 63;
-  const int g = lane >> 4;
-  const int li = lane & 15;
-  const int wm = wave / WN;
-  const int wn = wave % WN;
-
-  const int G = gridDim.x;
-  const int bid = blockIdx.x;
-  const bool xcd_remap = batch.xcd_remap && (G % 8) == 0;
-  const int slot = uni(xcd_remap ? (bid % 8) * (G / 8) + bid / 8 : bid);
-
-  for (int round = 0;; ++round) {
-    const int t = round * G + slot;
-    if (t >= batch.total_tiles) break;
-    const GemmDesc d = uniform_desc(batch, uni(t));
-    const int lt = t - d.tile_start;
-    const int tiles_n = d.tiles_n;
-    const int tiles_m = (d.m + BM - 1) / BM;
-    const int gm = batch.group_m;
-    const int grp = lt / (gm * tiles_n);
-    const int first_m = grp * gm;
-    const int gsz = min(tiles_m - first_m, gm);
-    const int in_grp = lt - grp * gm * tiles_n;
-    const int row0 = uni((first_m + in_grp % gsz) * BM);
-    const int col0 = uni((in_grp / gsz) * BN);
-    const int m_rem = uni(d.m - row0);
-    const int n_rem = uni(d.n - col0);
-    // single-panel kernels skip the MFMAs of waves with no output rows or columns; the
-    // panel kernels run them (skipping measured slower there: it costs the carried-C loop
-    // more than the few edge tiles give back)
-    const bool wave_live = MP || (wm * K::WTM < m_rem && wn * K::WTN < n_rem);
-    const long ldat = uni(d.lda), ldb = uni(d.ldb), ldc = uni(d.ldc);
-    const double *At_g = uni(d.A);
-    const double *Bg = uni(d.B) + col0;
-    gdouble *Cg = (gdouble *)(uni(d.C) + (long)row0 * ldc + col0);
-    const int Kdim = uni(d.k);
-    const int dpanel = uni(d.panel);
-    const int w = MP && dpanel > 0 && dpanel < Kdim ? dpanel : Kdim;
-    const int spp = (w + K::BK - 1) / K::BK;  // slabs per full panel
-    const int full_panels = Kdim / w;
-    const int tail = Kdim - full_panels * w;
-    const int nslab = full_panels * spp + (tail + K::BK - 1) / K::BK;
-
-    // lane offsets of this wave's pieces within a slab (k row kr, columns c, c+1);
-    // columns past the tile's edge read zero
-    uint32_t goff[K::PER];
-    int loff[K::PER];
+    };
+    // a full slab's turn: its successor has landed (two stages: it has itself), and every
+    // wave is done with the stage that is filled next
+    auto turn = [&]() {
+      wait_vm_c<(K::AHEAD ? STAGES - 3 : 0) * K::PER>();
+      slab_barrier();
+    };
+    if (wm * K::WTM >= m_rem || wn * K::WTN >= n_rem) {
+      // all of this wave's rows or columns lie past the matrix edge: it only loads its share
+      // of the slabs and keeps the barriers
+      if constexpr (K::AHEAD) {
+        wait_slab(0);
+        slab_barrier();
+      }
+      walk([&](auto stage, auto steady) {
+        if constexpr (decltype(steady)::value) {
+          turn();
 #pragma unroll
-    for (int u = 0; u < K::PER; ++u) {
-      const int blk = wave + u * K::NW;
-      if (blk < K::A_BLOCKS) {
-        const int kr = blk / K::A_PIECES;
-        const int c = (blk % K::A_PIECES) * 128 + 2 * lane;
-        goff[u] = c < m_rem ? (uint32_t)(((long)kr * ldat + row0 + c) * 8) : kOOB;
-        loff[u] = kr * K::AP * 8 + (blk % K::A_PIECES) * 1024;
-      } else {
-        const int q = blk - K::A_BLOCKS;
-        const int kr = q / K::B_PIECES;
-        const int c = (q % K::B_PIECES) * 128 + 2 * lane;
-        goff[u] = c < n_rem ? (uint32_t)(((long)kr * ldb + c) * 8) : kOOB;
-        loff[u] = K::A_BYTES + kr * K::BP * 8 + (q % K::B_PIECES) * 1024;
-      }
+          for (int u = 0; u < K::PER; ++u) load_block(u, (decltype(stage)::value + STAGES - 1) % STAGES);
+          advance(BK);
+          ++issued;
+        }
+      });
+      return;
     }
 
-    // slab bases advance by BK rows; a slab's byte range is BK rows (fewer for the last
-    // slab, whose missing k rows then read zero). The launcher keeps BK rows < 2 GiB.
-    const int full_a = (int)(K::BK * ldat * 8), full_b = (int)(K::BK * ldb * 8);
-    // slab sidx: k rows [kb, kb + krem) of panel p (slabs never cross a panel's end)
-    auto slab_rows = [&](int sidx, int &kb, int &krem, int &pe) {
-      const int p = sidx / spp;
-      kb = p * w + (sidx - p * spp) * K::BK;
-      pe = min(p * w + w, Kdim);
-      krem = min(K::BK, pe - kb);
-    };
-    auto issue = [&](int sidx) {
-      int kb, krem, pe;
-      slab_rows(sidx, kb, krem, pe);
-      char *stage = smem + (sidx % K::STAGES) * K::STAGE_BYTES;
-      const int na = krem == K::BK ? full_a : krem * (int)ldat * 8;
-      const int nb = krem == K::BK ? full_b : krem * (int)ldb * 8;
-      const rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(At_g + (long)kb * ldat), (short)0, na,
-                                                          0x00020000);
-      const rsrc_t rB =
-          __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(Bg + (long)kb * ldb), (short)0, nb, 0x00020000);
-#pragma unroll
-      for (int u = 0; u < K::PER; ++u) {
-        const int blk = wave + u * K::NW;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(blk < K::A_BLOCKS ? rA : rB, (lds_void *)(stage + loff[u]), 16, goff[u],
-                                                  0, 0, 0);
-      }
-    };
-
-    d4 acc[K::TM][K::TN];
-    d4 creg[MP ? K::TM : 1][MP ? K::TN : 1];
+    // a small wave tile (and a panel kernel, which carries it) reads C first, so that its
+    // latency passes under the slabs'
+    constexpr bool CFIRST = MP || (K::TM * K::TN <= 4 && K::NW <= 8);
+    d4 acc[K::TM][K::TN], creg[CFIRST ? K::TM : 1][CFIRST ? K::TN : 1];
 #pragma unroll
     for (int i = 0; i < K::TM; ++i)
 #pragma unroll
-      for (int j = 0; j < K::TN; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-    if constexpr (MP) {
-#pragma unroll
-      for (int i = 0; i < K::TM; ++i)
-#pragma unroll
-        for (int j = 0; j < K::TN; ++j) {
+      for (int j = 0; j < K::TN; ++j) {
+        acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+        if constexpr (CFIRST) {
           const int cc = wn * K::WTN + j * 16 + li;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
@@ -761,60 +648,72 @@ __device__ __forceinline__ void f64_at_body(const GemmBatch &batch) {
             creg[i][j][r] = (rr < m_rem && cc < n_rem) ? Cg[(long)rr * ldc + cc] : 0.0;
           }
         }
-    }
-
-    // every wave must be done reading the previous tile's stages before refilling them;
-    // with more than two stages nothing older than the ring's loads may be outstanding,
-    // so that counting them (in issue order) tells which slabs have landed
-    if constexpr (K::STAGES > 2) wait_vm_c<0>();
-    slab_barrier();
-#pragma unroll
-    for (int s0 = 0; s0 < K::STAGES - 1; ++s0)
-      if (s0 < nslab) issue(s0);
-    for (int sidx = 0; sidx < nslab; ++sidx) {
-      // slabs issued after this one that may stay in flight
-      const int later = min(K::STAGES - 2, nslab - 1 - sidx);
-      if constexpr (K::STAGES == 2) {
-        wait_vm_c<0>();
-      } else {
-        if (later <= 0)
-          wait_vm_c<0>();
-        else if (later == 1)
-          wait_vm_c<K::PER>();
-        else
-          wait_vm_c<(K::STAGES - 2) * K::PER>();
       }
+
+    auto read_ops = [&](int q, int kk, double(&x)[K::TM], double(&y)[K::TN]) {
+#pragma unroll
+      for (int i = 0; i < K::TM; ++i)
+        x[i] = *reinterpret_cast<const double *>(smem + a_off[kk] + (q * K::A_BYTES + i * 16 * BK * 8));
+#pragma unroll
+      for (int j = 0; j < K::TN; ++j)
+        y[j] = *reinterpret_cast<const double *>(smem + b_off[j] + (q * K::B_BYTES + kk * 4 * BN * 8));
+    };
+    auto mfmas = [&](const double(&x)[K::TM], const double(&y)[K::TN]) {
+#pragma unroll
+      for (int i = 0; i < K::TM; ++i)
+#pragma unroll
+        for (int j = 0; j < K::TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i], y[j], acc[i][j], 0, 0, 0);
+    };
+    double a[K::RING][K::TM], b[K::RING][K::TN];
+    if constexpr (K::AHEAD) {
+      wait_slab(0);
       slab_barrier();
-      const char *stage = smem + (sidx % K::STAGES) * K::STAGE_BYTES;
-      const double *At = reinterpret_cast<const double *>(stage);
-      const double *Bs = reinterpret_cast<const double *>(stage + K::A_BYTES);
-      // k beyond the last slab's rows reads as zero: fma(0, 0, c) = c
-      auto kstep = [&](int kk) {
-        double a[K::TM], b[K::TN];
 #pragma unroll
-        for (int i = 0; i < K::TM; ++i) a[i] = At[(kk * 4 + g) * K::AP + wm * K::WTM + i * 16 + li];
+      for (int q = 0; q < K::RING - 1; ++q) {
+        read_ops(0, q, a[q], b[q]);
+        __builtin_amdgcn_sched_barrier(0);  // in the order of their use
+      }
+    }
+    int kend = min(w, Kdim), kb = 0;  // MP: the panel end that the slab works towards
+    walk([&](auto stage, auto steady) {
+      constexpr int Q = decltype(stage)::value;
+      constexpr bool STEADY = decltype(steady)::value;
+      constexpr int R = K::RING, D = R - 1;
+      if constexpr (STEADY && !K::AHEAD) turn();
 #pragma unroll
-        for (int j = 0; j < K::TN; ++j) b[j] = Bs[(kk * 4 + g) * K::BP + wn * K::WTN + j * 16 + li];
+      for (int kk = 0; kk < K::KSTEPS; ++kk) {
+        if (!K::AHEAD && kk == 0) {
 #pragma unroll
-        for (int i = 0; i < K::TM; ++i)
+          for (int q = 0; q < D; ++q) read_ops(Q, q, a[q], b[q]);
+        }
+        mfmas(a[kk % R], b[kk % R]);
+        if constexpr (STEADY) {
+          if (K::AHEAD && kk == 0) turn();
+          // the loads are spread behind the k steps' MFMAs (two stages: all behind the first,
+          // since the next slab waits for them)
 #pragma unroll
-          for (int j = 0; j < K::TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
-      };
-      // the first k step's LDS reads go out right after the barrier; the next slab's
-      // loads are issued behind its MFMAs. A wave whose rows or columns all lie past the
-      // tile's edge has no output: it only loads its share of the slabs and keeps the
-      // barriers.
-      if (wave_live) kstep(0);
-      if (sidx + K::STAGES - 1 < nslab) issue(sidx + K::STAGES - 1);
-      if (wave_live) {
-#pragma unroll
-        for (int kk = 1; kk < K::BK / 4; ++kk) kstep(kk);
+          for (int u = 0; u < K::PER; ++u)
+            if ((K::AHEAD ? u * K::KSTEPS / K::PER : 0) == kk)
+              load_block(u, (Q + STAGES - 1) % STAGES);
+          if (kk + 1 == K::KSTEPS) {
+            advance(BK);
+            ++issued;
+          }
+        }
+        // keep the reads behind these MFMAs and ahead of the next (the scheduler would sink
+        // them to their use)
+        __builtin_amdgcn_sched_barrier(0);
+        if (kk + D < K::KSTEPS)
+          read_ops(Q, kk + D, a[(kk + D) % R], b[(kk + D) % R]);
+        else if constexpr (K::AHEAD)  // past the last slab: read, not used
+          read_ops((Q + 1) % STAGES, kk + D - K::KSTEPS, a[(kk + D) % R], b[(kk + D) % R]);
+        __builtin_amdgcn_sched_barrier(0);
       }
       if constexpr (MP) {
-        int kb, krem, pe;
-        slab_rows(sidx, kb, krem, pe);
-        if (kb + krem == pe) {
+        kb = min(kb + BK, kend);
+        if (kb == kend) {
+          kend = min(kend + w, Kdim);
 #pragma unroll
           for (int i = 0; i < K::TM; ++i)
 #pragma unroll
@@ -824,209 +723,160 @@ __device__ __forceinline__ void f64_at_body(const GemmBatch &batch) {
             }
         }
       }
-    }
-
+    });
 #pragma unroll
     for (int i = 0; i < K::TM; ++i)
 #pragma unroll
-      for (int jj = 0; jj < K::TN; ++jj) {
-        const int cc = wn * K::WTN + jj * 16 + li;
+      for (int j = 0; j < K::TN; ++j) {
+        const int cc = wn * K::WTN + j * 16 + li;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int rr = wm * K::WTM + i * 16 + 4 * r + g;
           if (rr < m_rem && cc < n_rem) {
             gdouble *pc = Cg + (long)rr * ldc + cc;
             if constexpr (MP)
-              *pc = creg[i][jj][r];
+              *pc = creg[i][j][r];
+            else if constexpr (CFIRST)
+              *pc = creg[i][j][r] + acc[i][j][r];
             else
-              *pc = *pc + acc[i][jj][r];
+              *pc = *pc + acc[i][j][r];
           }
         }
       }
   }
 }
 
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void f64_at_256x128(GemmBatch batch) {
-  f64_at_body<256, 128, 4, 2, false>(batch);
-}
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f64_at_128x128(GemmBatch batch) {
-  f64_at_body<128, 128, 2, 2, false>(batch);
-}
-// 8 waves with 64x32 wave tiles, so the carried C fits beside the accumulators
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void f64_at_128x128_w8(GemmBatch batch) {
-  f64_at_body<128, 128, 2, 4, false>(batch);
-}
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void f64_at_128x128_w8_mp(GemmBatch batch) {
-  f64_at_body<128, 128, 2, 4, true>(batch);
-}
-// One workgroup per CU leaves LDS for a deeper ring: three or four 16-deep stages, or two
-// 32-deep ones (half the barriers per k)
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void f64_at_128x128_w8_s3(GemmBatch batch) {
-  f64_at_body<128, 128, 2, 4, false, 3>(batch);
-}
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void f64_at_128x128_w8_mp_s3(
-    GemmBatch batch) {
-  f64_at_body<128, 128, 2, 4, true, 3>(batch);
-}
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void f64_at_128x128_w8_s4(GemmBatch batch) {
-  f64_at_body<128, 128, 2, 4, false, 4>(batch);
-}
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void f64_at_128x128_w8_mp_s4(
-    GemmBatch batch) {
-  f64_at_body<128, 128, 2, 4, true, 4>(batch);
-}
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void f64_at_128x128_w8_k32(GemmBatch batch) {
-  f64_at_body<128, 128, 2, 4, false, 2, 32>(batch);
-}
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void f64_at_128x128_w8_mp_k32(
-    GemmBatch batch) {
-  f64_at_body<128, 128, 2, 4, true, 2, 32>(batch);
-}
-// 16 waves with 32x32 wave tiles: the carried C and the accumulators fit 4 waves per SIMD,
-// so each barrier has four waves per SIMD to hide behind (LDS reads: one per MFMA)
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void f64_at_128x128_w16_k32(
-    GemmBatch batch) {
-  f64_at_body<128, 128, 4, 4, false, 2, 32>(batch);
-}
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void f64_at_128x128_w16_mp_k32(
-    GemmBatch batch) {
-  f64_at_body<128, 128, 4, 4, true, 2, 32>(batch);
+template <int BM, int BN>
+__device__ __forceinline__ void tile_origin(const GemmDesc &d, int lt, int group_m, int &row0, int &col0) {
+  const int tiles_n = d.tiles_n;
+  const int tiles_m = (d.m + BM - 1) / BM;
+  const int grp = lt / (group_m * tiles_n);
+  const int first_m = grp * group_m;
+  const int gsz = min(tiles_m - first_m, group_m);
+  const int in_grp = lt - grp * group_m * tiles_n;
+  row0 = uni((first_m + in_grp % gsz) * BM);
+  col0 = uni((in_grp / gsz) * BN);
 }
 
-// At[k][m] = A[m][k] for m < M, k < K; At[k][m] = 0 for M <= m < ldat (row pitch ldat)
-__global__ __launch_bounds__(256) void f64_transpose_kernel(const double *__restrict__ A, long lda, int M, int Kd,
-                                                            double *__restrict__ At, long ldat) {
-  __shared__ double tile[32][33];
-  const int k0 = blockIdx.x * 32, m0 = blockIdx.y * 32;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  double v[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int m = m0 + ty + 8 * u, k = k0 + tx;
-    v[u] = load_or_zero(A, (long)m * lda + k, m < M && k < Kd);
+// A contiguous run of the `total` tiles per XCD (workgroup bid runs on XCD bid % 8)
+__device__ __forceinline__ int xcd_run(int bid, int total) {
+  return (bid % 8) * (total / 8) + min(bid % 8, total % 8) + bid / 8;
+}
+
+// Tiles of shape T, and, from tile batch.tail_start on, the smaller tiles of shape U: the part
+// of the work that would leave the last round of T tiles nearly empty.
+template <class T, class U>
+__device__ __forceinline__ void f64_rm_body(const GemmBatch &batch) {
+  const int G = gridDim.x;
+  const int bid = blockIdx.x;
+  const int total = batch.total_tiles, head = batch.tail_start;
+  int slot = bid;
+  if (batch.xcd_remap) {
+    if (G == total)
+      slot = bid < head ? xcd_run(bid, head) : head + xcd_run(bid - head, total - head);
+    else if (G % 8 == 0)
+      slot = (bid % 8) * (G / 8) + bid / 8;
   }
-#pragma unroll
-  for (int u = 0; u < 4; ++u) tile[ty + 8 * u][tx] = v[u];
-  __syncthreads();
-#pragma unroll
-  for (int r = ty; r < 32; r += 8) {
-    const int k = k0 + r, m = m0 + tx;
-    if (k < Kd && m < ldat) At[(long)k * ldat + m] = tile[tx][r];
+  slot = uni(slot);
+  for (int t = slot; t < total; t += G) {
+    int row0, col0;
+    const GemmDesc d = uniform_desc(batch, uni(t));
+    if (t < head) {
+      tile_origin<T::BM, T::BN>(d, t - d.tile_start, batch.group_m, row0, col0);
+      T::run(d, row0, col0);
+    } else {
+      tile_origin<U::BM, U::BN>(d, t - d.tile_start, batch.group_m, row0, col0);
+      U::run(d, row0, col0);
+    }
   }
 }
 
-// Bc[k][j] = B[k][j] for j < N, 0 for N <= j < ldbc (row pitch ldbc)
-__global__ __launch_bounds__(256) void f64_copy_pad_kernel(const double *__restrict__ B, long ldb, int Kd, int N,
-                                                           double *__restrict__ Bc, long ldbc) {
-  const int k = blockIdx.y;
-  for (long j = (long)blockIdx.x * blockDim.x + threadIdx.x; j < ldbc; j += (long)gridDim.x * blockDim.x)
-    Bc[(long)k * ldbc + j] = j < N ? B[(long)k * ldb + j] : 0.0;
+template <int BM_, int BN_, int WM, int WN, int BK, int STAGES, bool MP>
+struct RmTile {
+  using K = F64Rm<BM_, BN_, WM, WN, BK, STAGES>;
+  static constexpr int BM = BM_, BN = BN_, THREADS = WM * WN * 64;
+  static constexpr int LDS = K::LDS_BYTES, A_ROWS = K::ARB, B_ROWS = K::BRB;
+  static __device__ __forceinline__ void run(const GemmDesc &d, int row0, int col0) {
+    f64_rm_tile<BM, BN, WM, WN, BK, STAGES, MP>(d, row0, col0);
+  }
+};
+
+template <class T, class U>
+__global__ __launch_bounds__(T::THREADS) __attribute__((amdgpu_waves_per_eu(2))) void f64_rm_kernel(GemmBatch batch) {
+  static_assert(T::THREADS == U::THREADS, "one workgroup shape");
+  f64_rm_body<T, U>(batch);
 }
 
 typedef void (*KernelFn)(GemmBatch);
 
-// One tile configuration: kernels for [panel grouping][16-byte loads]. Direct-to-LDS
-// configs use f64_lds_kernel when 16-byte loads are legal and fall back to the
-// register-staged kernel with the same macro tile otherwise (same tiles, same
-// arithmetic, so the planner's tile list is valid for both).
+// One tile configuration: kernels for [panel grouping][16-byte loads]. The row-major kernels
+// take any alignment, so both slots hold the same one.
 struct ConfigEntry {
-  int bm, bn, threads, bk;
-  size_t lds_bytes[2];  // dynamic LDS for [vec1][vec2] kernels
+  int bm, bn, threads;
+  int a_rows, b_rows;   // rows of A, rows of B under one 32-bit buffer offset
+  size_t lds_bytes;     // dynamic LDS
   bool panels;          // panel-grouped variants fit without spills
   KernelFn fn[2][2];
-  bool trans_a = false;  // the 16-byte kernel reads A transposed (descriptor A = At, lda = its pitch)
+  int tail_bm, tail_bn;  // the tail's tile; 0: none
 };
 
 #define PHPC_V1(BM_, BN_, WM_, WN_, BK_, MP_, VEC_) f64_gemm_kernel<BM_, BN_, WM_, WN_, BK_, MP_, VEC_>
-#define PHPC_LDS(BM_, BN_, WM_, WN_, ST_, MP_) f64_lds_kernel<BM_, BN_, WM_, WN_, ST_, MP_>
-#define LDS_BYTES(BM_, BN_, ST_) ((size_t)(ST_) * (size_t)F64Lds<BM_, BN_, 2, 2, ST_, false>::STAGE_BYTES)
 
+// a row-major configuration: head tile T, tail tile U (the same type: no tail); SP: single
+// panel only
+template <template <bool> class T, template <bool> class U, bool SP = false>
+constexpr ConfigEntry rm_config() {
+  using T0 = T<false>;
+  using U0 = U<false>;
+  constexpr bool same = std::is_same<T0, U0>::value;
+  KernelFn one = f64_rm_kernel<T<false>, U<false>>;
+  KernelFn mp = f64_rm_kernel<T<!SP>, U<!SP>>;
+  return {T0::BM, T0::BN, T0::THREADS, std::max(T0::A_ROWS, U0::A_ROWS), std::max(T0::B_ROWS, U0::B_ROWS),
+          (size_t)std::max(T0::LDS, U0::LDS), !SP, {{one, one}, {mp, mp}}, same ? 0 : U0::BM, same ? 0 : U0::BN};
+}
+// waves x 16-deep slabs unless named otherwise
+template <bool MP> using T32 = RmTile<32, 32, 2, 2, 16, 4, MP>;         // 4 waves, 32 KiB: five workgroups per CU
+template <bool MP> using T32K32 = RmTile<32, 32, 2, 2, 32, 4, MP>;      // 4 waves, 32-deep slabs
+template <bool MP> using T64x32 = RmTile<64, 32, 2, 2, 16, 5, MP>;      // 4 waves
+template <bool MP> using T64 = RmTile<64, 64, 2, 2, 16, 4, MP>;         // 4 waves, 64 KiB: two workgroups per CU
+template <bool MP> using T64W8 = RmTile<64, 64, 2, 4, 16, 4, MP>;       // 8 waves
+template <bool MP> using T64W16 = RmTile<64, 64, 4, 4, 32, 4, MP>;      // 16 waves, 32-deep slabs
+template <bool MP> using T128x64 = RmTile<128, 64, 4, 2, 16, 3, MP>;    // 8 waves
+template <bool MP> using T128W8 = RmTile<128, 128, 2, 4, 16, 4, MP>;    // 8 waves
+template <bool MP> using T128K32 = RmTile<128, 128, 4, 4, 32, 2, MP>;   // 16 waves, two 32-deep stages
+template <bool MP> using T128 = RmTile<128, 128, 4, 4, 16, 4, MP>;      // 16 waves
+template <bool MP> using T256W8 = RmTile<256, 128, 4, 2, 16, 3, MP>;    // 8 waves
+template <bool MP> using T256 = RmTile<256, 128, 4, 4, 16, 3, MP>;      // 16 waves
+
+// a register-staged configuration
+#define V1_CONFIG(BM_, BN_, WM_, WN_, BK_)                                                                     \
+  {BM_, BN_, WM_ *WN_ * 64, BM_, BK_, 0, true,                                                                 \
+   {{PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 1), PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 2)},                  \
+    {PHPC_V1(BM_, BN_, WM_, WN_, BK_, true, 1), PHPC_V1(BM_, BN_, WM_, WN_, BK_, true, 2)}}, 0, 0}
+#define V1_CONFIG_SP(BM_, BN_, WM_, WN_, BK_)                                                                  \
+  {BM_, BN_, WM_ *WN_ * 64, BM_, BK_, 0, false,                                                                \
+   {{PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 1), PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 2)},                  \
+    {PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 1), PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 2)}}, 0, 0}
+
+constexpr int kSmall = 13, kMid = 5, kBig = 11, kBigPanels = 16;  // the planner's
 const ConfigEntry kConfigs[] = {
-    // 0: register-staged, 8 waves (wave tile 64x32), 16-deep slabs
-    {128, 128, 512, 16, {0, 0}, true,
-     {{PHPC_V1(128, 128, 2, 4, 16, false, 1), PHPC_V1(128, 128, 2, 4, 16, false, 2)},
-      {PHPC_V1(128, 128, 2, 4, 16, true, 1), PHPC_V1(128, 128, 2, 4, 16, true, 2)}}},
-    // 1: register-staged, 8 waves, 32-deep slabs
-    {128, 128, 512, 32, {0, 0}, true,
-     {{PHPC_V1(128, 128, 2, 4, 32, false, 1), PHPC_V1(128, 128, 2, 4, 32, false, 2)},
-      {PHPC_V1(128, 128, 2, 4, 32, true, 1), PHPC_V1(128, 128, 2, 4, 32, true, 2)}}},
-    // 2: register-staged, 4 waves (wave tile 32x32), 64x64 tiles for small problems
-    {64, 64, 256, 16, {0, 0}, true,
-     {{PHPC_V1(64, 64, 2, 2, 16, false, 1), PHPC_V1(64, 64, 2, 2, 16, false, 2)},
-      {PHPC_V1(64, 64, 2, 2, 16, true, 1), PHPC_V1(64, 64, 2, 2, 16, true, 2)}}},
-    // 3: direct-to-LDS, 8 waves (wave tile 64x32), 4-stage pipeline
-    {128, 128, 512, 16, {0, LDS_BYTES(128, 128, 4)}, true,
-     {{PHPC_V1(128, 128, 2, 4, 16, false, 1), PHPC_LDS(128, 128, 2, 4, 4, false)},
-      {PHPC_V1(128, 128, 2, 4, 16, true, 1), PHPC_LDS(128, 128, 2, 4, 4, true)}}},
-    // 4: direct-to-LDS, 4 waves (wave tile 64x64), 4-stage pipeline; single panel only
-    {128, 128, 256, 16, {0, LDS_BYTES(128, 128, 4)}, false,
-     {{PHPC_V1(128, 128, 2, 2, 16, false, 1), PHPC_LDS(128, 128, 2, 2, 4, false)},
-      {PHPC_V1(128, 128, 2, 2, 16, false, 1), PHPC_LDS(128, 128, 2, 2, 4, false)}}},
-    // 5: direct-to-LDS, 4 waves (wave tile 32x32), 64x64 tiles, 4-stage pipeline
-    {64, 64, 256, 16, {0, LDS_BYTES(64, 64, 4)}, true,
-     {{PHPC_V1(64, 64, 2, 2, 16, false, 1), PHPC_LDS(64, 64, 2, 2, 4, false)},
-      {PHPC_V1(64, 64, 2, 2, 16, true, 1), PHPC_LDS(64, 64, 2, 2, 4, true)}}},
-    // 6: register-staged, 8 waves (wave tile 64x64), 256x128 tiles; single panel only
-    {256, 128, 512, 16, {0, 0}, false,
-     {{PHPC_V1(256, 128, 4, 2, 16, false, 1), PHPC_V1(256, 128, 4, 2, 16, false, 2)},
-      {PHPC_V1(256, 128, 4, 2, 16, false, 1), PHPC_V1(256, 128, 4, 2, 16, false, 2)}}},
-    // 7: direct-to-LDS, 8 waves (wave tile 64x64), 256x128 tiles, 3 stages; single panel only
-    {256, 128, 512, 16, {0, LDS_BYTES(256, 128, 3)}, false,
-     {{PHPC_V1(256, 128, 4, 2, 16, false, 1), PHPC_LDS(256, 128, 4, 2, 3, false)},
-      {PHPC_V1(256, 128, 4, 2, 16, false, 1), PHPC_LDS(256, 128, 4, 2, 3, false)}}},
-    // 8: register-staged, 4 waves (wave tile 64x64), 128x128 tiles: 68 KiB of LDS, two
-    //    workgroups per CU so one's barrier stalls are covered by the other; single panel only
-    {128, 128, 256, 16, {0, 0}, false,
-     {{PHPC_V1(128, 128, 2, 2, 16, false, 1), PHPC_V1(128, 128, 2, 2, 16, false, 2)},
-      {PHPC_V1(128, 128, 2, 2, 16, false, 1), PHPC_V1(128, 128, 2, 2, 16, false, 2)}}},
-    // 9: direct-to-LDS, 4 waves (wave tile 64x64), 128x128 tiles, 2 stages (66 KiB, two
-    //    workgroups per CU); single panel only
-    {128, 128, 256, 16, {0, LDS_BYTES(128, 128, 2)}, false,
-     {{PHPC_V1(128, 128, 2, 2, 16, false, 1), PHPC_LDS(128, 128, 2, 2, 2, false)},
-      {PHPC_V1(128, 128, 2, 2, 16, false, 1), PHPC_LDS(128, 128, 2, 2, 2, false)}}},
-    // 10: transposed-A direct-to-LDS, 8 waves (wave tile 64x64), 256x128 tiles, 2 stages;
-    //     single panel only. The 8-byte slots are config 6's kernels: when B rules out
-    //     16-byte loads the launcher runs config 6 on the untransposed A instead.
-    {256, 128, 512, 16, {0, 2 * (size_t)F64At<256, 128, 4, 2>::STAGE_BYTES}, false,
-     {{PHPC_V1(256, 128, 4, 2, 16, false, 1), f64_at_256x128},
-      {PHPC_V1(256, 128, 4, 2, 16, false, 1), f64_at_256x128}},
-     true},
-    // 11: transposed-A direct-to-LDS, 4 waves (wave tile 64x64), 128x128 tiles, 2 stages
-    //     (68 KiB, two workgroups per CU); single panel only. 8-byte slots: config 8's kernel.
-    {128, 128, 256, 16, {0, 2 * (size_t)F64At<128, 128, 2, 2>::STAGE_BYTES}, false,
-     {{PHPC_V1(128, 128, 2, 2, 16, false, 1), f64_at_128x128},
-      {PHPC_V1(128, 128, 2, 2, 16, false, 1), f64_at_128x128}},
-     true},
-    // 12: transposed-A direct-to-LDS, 8 waves (wave tile 64x32), 128x128 tiles, 2 stages,
-    //     panel-grouped too (C carried in registers). 8-byte slots: config 0's kernels.
-    {128, 128, 512, 16, {0, 2 * (size_t)F64At<128, 128, 2, 4>::STAGE_BYTES}, true,
-     {{PHPC_V1(128, 128, 2, 4, 16, false, 1), f64_at_128x128_w8},
-      {PHPC_V1(128, 128, 2, 4, 16, true, 1), f64_at_128x128_w8_mp}},
-     true},
-    // 13: as 12 with three 16-deep stages (102 KiB)
-    {128, 128, 512, 16, {0, 3 * (size_t)F64At<128, 128, 2, 4, 3>::STAGE_BYTES}, true,
-     {{PHPC_V1(128, 128, 2, 4, 16, false, 1), f64_at_128x128_w8_s3},
-      {PHPC_V1(128, 128, 2, 4, 16, true, 1), f64_at_128x128_w8_mp_s3}},
-     true},
-    // 14: as 12 with four 16-deep stages (136 KiB)
-    {128, 128, 512, 16, {0, 4 * (size_t)F64At<128, 128, 2, 4, 4>::STAGE_BYTES}, true,
-     {{PHPC_V1(128, 128, 2, 4, 16, false, 1), f64_at_128x128_w8_s4},
-      {PHPC_V1(128, 128, 2, 4, 16, true, 1), f64_at_128x128_w8_mp_s4}},
-     true},
-    // 15: as 12 with two 32-deep stages (136 KiB)
-    {128, 128, 512, 32, {0, 2 * (size_t)F64At<128, 128, 2, 4, 2, 32>::STAGE_BYTES}, true,
-     {{PHPC_V1(128, 128, 2, 4, 16, false, 1), f64_at_128x128_w8_k32},
-      {PHPC_V1(128, 128, 2, 4, 16, true, 1), f64_at_128x128_w8_mp_k32}},
-     true},
-    // 16: as 15 with 16 waves (wave tile 32x32). There is no 1024-thread register-staged
-    //     kernel for the 8-byte slots; they are never launched (a transposed-A launch
-    //     needs 16-byte B rows, and phpc_f64_grouped switches to config 0 when A cannot be
-    //     staged), so they hold the same kernels, keeping every slot's shape 1024 threads.
-    {128, 128, 1024, 32, {2 * (size_t)F64At<128, 128, 4, 4, 2, 32>::STAGE_BYTES,
-                          2 * (size_t)F64At<128, 128, 4, 4, 2, 32>::STAGE_BYTES}, true,
-     {{f64_at_128x128_w16_k32, f64_at_128x128_w16_k32},
-      {f64_at_128x128_w16_mp_k32, f64_at_128x128_w16_mp_k32}},
-     true},
+    V1_CONFIG(128, 128, 2, 4, 16),             // 0: register-staged, 8 waves (wave tile 64x32)
+    V1_CONFIG(128, 128, 2, 4, 32),             // 1: register-staged, 8 waves, 32-deep slabs
+    V1_CONFIG(64, 64, 2, 2, 16),               // 2: register-staged, 4 waves (wave tile 32x32)
+    rm_config<T128W8, T128W8>(),               // 3
+    rm_config<T64W8, T64W8, true>(),           // 4: single panel only
+    rm_config<T64, T32K32>(),                  // 5: the planner's for middle sizes
+    V1_CONFIG_SP(256, 128, 4, 2, 16),          // 6: register-staged, 8 waves (wave tile 64x64); single panel only
+    rm_config<T256W8, T256W8, true>(),         // 7: single panel only
+    V1_CONFIG_SP(128, 128, 2, 2, 16),          // 8: register-staged, 4 waves (wave tile 64x64); single panel only
+    rm_config<T64x32, T64x32, true>(),         // 9: single panel only
+    rm_config<T64W16, T64W16, true>(),         // 10: single panel only
+    rm_config<T256, T64W16, true>(),           // 11: the planner's for large single-panel work; single panel only
+    rm_config<T128x64, T128x64>(),             // 12
+    rm_config<T32, T32>(),                     // 13: the planner's for small work
+    rm_config<T128, T128>(),                   // 14
+    rm_config<T128K32, T128K32>(),             // 15
+    rm_config<T128, T64W16>(),                 // 16: the planner's for large panel-grouped work
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 
@@ -1040,25 +890,16 @@ size_t g_pinned_cap = 0;
 std::mutex g_desc_mu;  // guards the descriptor buffers below (never held with g_mu)
 hipEvent_t g_desc_done = nullptr;  // recorded after the last launch that read g_desc_dev
 
-// Threads per workgroup of a configuration's kernels. Single-panel configurations fill
-// their panel-grouped slots with the single-panel kernels, which are never launched with
-// panels (phpc_f64_grouped_dev rejects that), so every slot has the configuration's shape.
-int kernel_threads(int cfg, int mp, int vec2) {
-  (void)mp;
-  (void)vec2;
-  return kConfigs[cfg].threads;
-}
-
 void init_kernels_locked() {
   if (g_occ_ready) return;
   for (int c = 0; c < kNumConfigs; ++c)
     for (int a = 0; a < 2; ++a)
       for (int b = 0; b < 2; ++b) {
         const void *fn = reinterpret_cast<const void *>(kConfigs[c].fn[a][b]);
-        const size_t lds = kConfigs[c].lds_bytes[b];
+        const size_t lds = kConfigs[c].lds_bytes;
         if (lds > 0) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, kernel_threads(c, a, b), lds) != hipSuccess || n < 1)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, kConfigs[c].threads, lds) != hipSuccess || n < 1)
           n = 1;
         g_occ[c][a][b] = n;
       }
@@ -1072,6 +913,17 @@ int occupancy(int cfg, int mp, int vec2) {
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+bool has_panels(const GemmDesc &d) { return d.panel > 0 && d.panel < d.k; }
+long tiles_of(const GemmDesc &d, int bm, int bn) { return (long)((d.m + bm - 1) / bm) * ((d.n + bn - 1) / bn); }
+
+// the planner's configurations, replaceable through phpc_set_tuning; -1: the planner's own
+// choice (config_for)
+int g_big_config = -1;       // large panel-grouped work on device-resident lists
+int g_big_single = -1;       // large single-panel work on device-resident lists
+int g_big_single_host = kBig;
+int g_big_config_host = kBigPanels;
+int g_group_m = 8;
+int g_xcd_remap = 1;
 
 }  // namespace
 
@@ -1088,258 +940,153 @@ F64Config phpc_f64_config(int id) {
   return c;
 }
 
-// Planner. Single-panel work on enough 256x128 tiles to cover the CUs takes the
-// 256x128 tile (16 independent MFMA chains per wave); panel-grouped work takes the
-// 128x128 tile, whose waves also carry C in registers; small problems take 64x64.
-int g_big_config = 0;       // large, panel-grouped
-int g_big_single = 6;       // large, one panel
-int g_group_m = 8;
-int g_xcd_remap = 1;
-
-int phpc_f64_pick_config(const GemmDesc *descs, int ndesc) {
-  long tiles128 = 0, tiles256 = 0;
-  bool mp = false;
-  for (int i = 0; i < ndesc; ++i) {
-    tiles128 += (long)((descs[i].m + 127) / 128) * ((descs[i].n + 127) / 128);
-    tiles256 += (long)((descs[i].m + 255) / 256) * ((descs[i].n + 127) / 128);
-    if (descs[i].panel > 0 && descs[i].panel < descs[i].k) mp = true;
-  }
-  const int cus = phpc_device().cus;
-  if (!mp && tiles256 >= (long)cus) return g_big_single;
-  if (tiles128 >= (long)cus) return g_big_config;
-  return 5;
-}
-
 namespace {
 
-// Configuration for large single-panel work reached through host descriptors
-// (phpc_f64_grouped), which can stage a transposed copy of A first.
-int g_big_single_host = 11;
-int g_big_config_host = 16;  // large panel-grouped work through host descriptors
-
-bool b_vec2_ok(const GemmDesc &d) { return aligned16(d.B) && (d.ldb % 2 == 0) && (d.n % 2 == 0); }
-// the transposed-A kernels load B in 16-byte column pairs; with an even ldb and an aligned
-// base, the pair holding an odd n's last column ends inside the row, and the extra column
-// only feeds an output column that is never stored
-bool b_at_ok(const GemmDesc &d) { return aligned16(d.B) && (d.ldb % 2 == 0); }
-
-int launch_grouped(const GemmDesc *descs_dev, const GemmDesc *descs_host, int ndesc, int grid, int config_id,
-                   hipStream_t stream, bool a_transposed) {
-  if (ndesc <= 0) return PHPC_OK;
-  if (config_id < 0 || config_id >= kNumConfigs)
-    return phpc_set_error(PHPC_ERR_ARG, "bad FP64 config id %d", config_id);
-  const ConfigEntry &ce = kConfigs[config_id];
-  if (ce.trans_a != a_transposed)
-    return phpc_set_error(PHPC_ERR_ARG, "FP64 config %d %s a transposed A", config_id,
-                          ce.trans_a ? "needs" : "does not take");
-  bool mp = false, vec2 = true;
-  int total = 0;
+// Planner: by how many tiles the work gives the CUs. Measured on MI355X in TFLOP/s, with the
+// neighbouring choices:
+//   fewer 64x64 tiles than CUs: 32x32 tiles (512^3: 8.6 us against 20.4 on 64x64, N = 256:
+//     6.2 against 12.7), whose workgroups share a CU five at a time;
+//   then 64x64 tiles with a 32x32 tail (2048^3: 68 TFLOP/s against 54 on 32x32 alone);
+//   from two 256x128 tiles per CU on, those (4096^3: 73.2 against 68; 16384^3: 74.8 against 65
+//     on 64x64), or, with panels, 128x128 tiles, whose waves have room for the carried C.
+int config_for(const GemmDesc *descs, int ndesc, bool device_list) {
+  long t64 = 0, t128 = 0, t256 = 0;
+  bool mp = false;
   for (int i = 0; i < ndesc; ++i) {
-    const GemmDesc &d = descs_host[i];
-    if (d.panel > 0 && d.panel < d.k) mp = true;
-    // 32-bit buffer offsets: one A tile (bm rows) and one B slab (bk rows) must span < 2 GiB
-    if ((long)ce.bm * d.lda * 8 >= 0x7fffffffL || (long)ce.bk * d.ldb * 8 >= 0x7fffffffL)
-      return phpc_set_error(PHPC_ERR_ARG, "leading dimension too large (lda=%ld, ldb=%ld)", d.lda, d.ldb);
-    // 16-byte loads need 16-byte aligned rows and even k / n boundaries (a transposed A
-    // is stored that way by construction)
-    const bool a_ok = a_transposed || (aligned16(d.A) && (d.lda % 2 == 0) && (d.k % 2 == 0) &&
-                                       (d.panel <= 0 || d.panel >= d.k || d.panel % 2 == 0));
-    if (!a_ok || !(a_transposed ? b_at_ok(d) : b_vec2_ok(d))) vec2 = false;
-    total = d.tile_start + ((d.m + ce.bm - 1) / ce.bm) * d.tiles_n;
+    t64 += tiles_of(descs[i], 64, 64);
+    t128 += tiles_of(descs[i], 128, 128);
+    t256 += tiles_of(descs[i], 256, 128);
+    mp |= has_panels(descs[i]);
   }
-  if (a_transposed && !vec2) return phpc_set_error(PHPC_ERR_ARG, "transposed-A kernels need 16-byte B rows");
-  if (mp && !ce.panels)
+  const long cus = phpc_device().cus;
+  if (mp && t128 >= 4 * cus) return device_list && g_big_config >= 0 ? g_big_config : g_big_config_host;
+  if (!mp && t256 >= 2 * cus) return device_list && g_big_single >= 0 ? g_big_single : g_big_single_host;
+  return t64 >= cus ? kMid : kSmall;
+}
+
+// Split `live` (tiles planned for head tiles of ce) so that the head fills whole rounds of the
+// CUs and the rest runs on the smaller tail tiles: a last round of head tiles that is nearly
+// empty costs as much as a full one (1777 x 1999 x 1235: 560 tiles of 64x64 on 256 CUs take
+// three rounds, 187 us; 500 of them and the rest as 32x32 take 2.25). Every output's
+// arithmetic is its own, so where the line runs does not change a result. The cut takes rows
+// or columns of tiles, whichever step is finer, off the last GEMMs.
+void split_tail(std::vector<GemmDesc> &live, const ConfigEntry &ce, std::vector<GemmDesc> &tail) {
+  const long cus = phpc_device().cus;
+  long total = 0;
+  for (const GemmDesc &d : live) total += tiles_of(d, ce.bm, ce.bn);
+  const long rounds = total / cus, rest = total % cus;
+  if (rounds == 0 || rest == 0 || 5 * rest > 4 * cus) return;
+  long excess = rest;
+  for (int i = (int)live.size() - 1; i >= 0 && excess > 0; --i) {
+    GemmDesc &d = live[i];
+    const long tm = (d.m + ce.bm - 1) / ce.bm, tn = (d.n + ce.bn - 1) / ce.bn;
+    GemmDesc t = d;
+    if (tn <= tm) {  // whole rows of tn tiles
+      const long cut = std::min(tm, (excess + tn - 1) / tn), keep = (tm - cut) * ce.bm;
+      t.A += keep * t.lda;
+      t.C += keep * t.ldc;
+      t.m -= (int)keep;
+      d.m = (int)keep;
+      excess -= cut * tn;
+    } else {
+      const long cut = std::min(tn, (excess + tm - 1) / tm), keep = (tn - cut) * ce.bn;
+      t.B += keep;
+      t.C += keep;
+      t.n -= (int)keep;
+      d.n = (int)keep;
+      excess -= cut * tm;
+    }
+    tail.insert(tail.begin(), t);
+    if (d.m == 0 || d.n == 0) live.erase(live.begin() + i);
+  }
+}
+
+}  // namespace
+
+int phpc_f64_prepare(const GemmDesc *descs, int ndesc, int config_id, bool device_list, F64Work *w) {
+  w->descs.clear();
+  w->total = w->tail_start = 0;
+  // drop empty GEMMs; k == 0 leaves C unchanged (C += 0 adds +0.0 only to tiles we skip)
+  for (int i = 0; i < ndesc; ++i) {
+    const GemmDesc &d = descs[i];
+    if (d.m < 0 || d.n < 0 || d.k < 0) return phpc_set_error(PHPC_ERR_ARG, "negative GEMM size");
+    if (d.m > 0 && d.n > 0 && d.k > 0) w->descs.push_back(d);
+  }
+  if (config_id < 0) config_id = config_for(w->descs.data(), (int)w->descs.size(), device_list);
+  if (config_id >= kNumConfigs) return phpc_set_error(PHPC_ERR_ARG, "bad FP64 config id %d", config_id);
+  const ConfigEntry &ce = kConfigs[config_id];
+  w->config = config_id;
+  w->mp = false;
+  w->vec2 = true;
+  for (const GemmDesc &d : w->descs) {
+    w->mp |= has_panels(d);
+    if ((long)ce.a_rows * d.lda * 8 >= 0x7fffffffL || (long)ce.b_rows * d.ldb * 8 >= 0x7fffffffL)
+      return phpc_set_error(PHPC_ERR_ARG, "leading dimension too large (lda=%ld, ldb=%ld)", d.lda, d.ldb);
+    // the register-staged kernels' 16-byte loads need 16-byte aligned rows and even k / n
+    // boundaries
+    const bool a_ok = aligned16(d.A) && d.lda % 2 == 0 && d.k % 2 == 0 && (!has_panels(d) || d.panel % 2 == 0);
+    if (!a_ok || !aligned16(d.B) || d.ldb % 2 || d.n % 2) w->vec2 = false;
+  }
+  if (w->mp && !ce.panels)
     return phpc_set_error(PHPC_ERR_ARG, "FP64 config %d does not support panel grouping", config_id);
-  if (total <= 0) return PHPC_OK;
+  std::vector<GemmDesc> tail;
+  if (ce.tail_bm) split_tail(w->descs, ce, tail);
+  long t = 0;
+  auto number = [&t](std::vector<GemmDesc> &v, int bm, int bn) {
+    for (GemmDesc &d : v) {
+      d.tiles_n = (d.n + bn - 1) / bn;
+      d.tile_start = (int)t;
+      t += tiles_of(d, bm, bn);
+    }
+  };
+  number(w->descs, ce.bm, ce.bn);
+  w->tail_start = (int)t;
+  number(tail, ce.tail_bm, ce.tail_bn);
+  if (t > 0x7fffffffL) return phpc_set_error(PHPC_ERR_ARG, "too many tiles");
+  w->total = (int)t;
+  w->descs.insert(w->descs.end(), tail.begin(), tail.end());
+  return PHPC_OK;
+}
+
+int phpc_f64_launch(const F64Work &w, const GemmDesc *descs_dev, int grid, hipStream_t stream) {
+  if (w.total <= 0) return PHPC_OK;
+  const ConfigEntry &ce = kConfigs[w.config];
   GemmBatch b{};
   b.descs = descs_dev;
-  b.ndesc = ndesc;
-  b.total_tiles = total;
+  b.ndesc = (int)w.descs.size();
+  b.total_tiles = w.total;
   b.group_m = g_group_m;
   b.xcd_remap = g_xcd_remap;
-  b.d0 = descs_host[0];
+  b.tail_start = w.tail_start;
+  b.d0 = w.descs[0];
+  if (b.ndesc == 2) b.d1 = w.descs[1];
   int G = grid;
   if (G <= 0) {
-    G = occupancy(config_id, mp, vec2) * phpc_device().cus;
-    if (G > total) G = total;
+    // the row-major kernels leave it to the dispatcher to hand out tiles, so that a CU whose
+    // tiles end early takes the next one; the register-staged ones walk a persistent grid
+    G = ce.lds_bytes ? w.total : occupancy(w.config, w.mp, w.vec2) * phpc_device().cus;
+    if (G > w.total) G = w.total;
   }
-  if (G < 1) G = 1;
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    init_kernels_locked();
+  }
   const int kt = phpc_ktime_begin(stream);
-  hipLaunchKernelGGL(ce.fn[mp][vec2], dim3(G), dim3(kernel_threads(config_id, mp, vec2)), ce.lds_bytes[vec2],
-                     stream, b);
+  hipLaunchKernelGGL(ce.fn[w.mp][w.vec2], dim3(G), dim3(ce.threads), ce.lds_bytes, stream, b);
   phpc_ktime_end(kt, stream);
   PHPC_HIP(hipGetLastError());
   return PHPC_OK;
 }
 
-// Transposed copies of A for the transposed-A configurations: one per distinct
-// (A, lda, m, k), in a process-wide workspace used in stream order.
-SharedWorkspace g_at_ws;
-
-int launch_live(std::vector<GemmDesc> &live, int grid, int config_id, hipStream_t stream, bool a_transposed);
-
-int launch_transposed(std::vector<GemmDesc> &live, int grid, int config_id, hipStream_t stream) {
-  F64Staging st;
-  st.plan(live.data(), (int)live.size());
-  std::lock_guard<std::mutex> lk(g_at_ws.mu);
-  g_at_ws.after_previous(stream);
-  double *ws = static_cast<double *>(g_at_ws.ws.get(st.total * sizeof(double), 0, stream));
-  if (!ws) return phpc_set_error(PHPC_ERR_MEM, "transposed-A workspace allocation failed (%zu bytes)", st.total * 8);
-  if (int rc = st.run(ws, stream)) return rc;
-  st.apply(ws, live.data(), (int)live.size());
-  const int rc = launch_live(live, grid, config_id, stream, true);
-  g_at_ws.mark_used(stream);
-  return rc;
-}
-
-}  // namespace
-
-int phpc_f64_grouped_dev(const GemmDesc *descs_dev, const GemmDesc *descs_host, int ndesc, int grid,
-                         int config_id, hipStream_t stream) {
-  return launch_grouped(descs_dev, descs_host, ndesc, grid, config_id, stream, false);
-}
-
-bool phpc_f64_config_trans_a(int id) { return id >= 0 && id < kNumConfigs && kConfigs[id].trans_a; }
-
-long phpc_f64_at_pitch(int m) { return ((long)m + 1) / 2 * 2; }
-
-bool phpc_f64_trans_a_ok(const GemmDesc *descs, int ndesc) {
-  for (int i = 0; i < ndesc; ++i) {
-    const GemmDesc &d = descs[i];
-    if (d.m <= 0 || d.n <= 0 || d.k <= 0) continue;
-    // grid limits of the staging kernels
-    if (phpc_f64_at_pitch(d.m) / 32 >= 65535 || (!b_at_ok(d) && d.k >= 65535)) return false;
-  }
-  return true;
-}
-
-void F64Staging::plan(const GemmDesc *descs, int ndesc) {
-  copies.clear();
-  a_copy.assign(ndesc, -1);
-  b_copy.assign(ndesc, -1);
-  total = 0;
-  auto find_or_add = [&](const double *src, long ld, int rows, int cols, bool tr) {
-    for (size_t j = 0; j < copies.size(); ++j) {
-      const Copy &c = copies[j];
-      if (c.src == src && c.ld == ld && c.rows == rows && c.cols == cols && c.transpose == tr) return (int)j;
-    }
-    const long pitch = phpc_f64_at_pitch(tr ? rows : cols);
-    const size_t n = (size_t)(tr ? cols : rows) * pitch;
-    copies.push_back({src, ld, rows, cols, pitch, total, tr});
-    total += (n + 31) / 32 * 32;  // 256-byte aligned copies
-    return (int)copies.size() - 1;
-  };
-  for (int i = 0; i < ndesc; ++i) {
-    const GemmDesc &d = descs[i];
-    if (d.m <= 0 || d.n <= 0 || d.k <= 0) continue;
-    a_copy[i] = find_or_add(d.A, d.lda, d.m, d.k, true);
-    if (!b_at_ok(d)) b_copy[i] = find_or_add(d.B, d.ldb, d.k, d.n, false);
-  }
-}
-
-int F64Staging::run(double *ws, hipStream_t stream) const {
-  for (const Copy &c : copies) {
-    if (c.transpose) {
-      if (int rc = phpc_f64_transpose(c.src, c.ld, c.rows, c.cols, ws + c.off, c.pitch, stream)) return rc;
-    } else {
-      const dim3 grid((unsigned)std::min<long>((c.pitch + 255) / 256, 64), (unsigned)c.rows);
-      hipLaunchKernelGGL(f64_copy_pad_kernel, grid, dim3(256), 0, stream, c.src, c.ld, c.rows, c.cols, ws + c.off,
-                         c.pitch);
-      PHPC_HIP(hipGetLastError());
-    }
-  }
-  return PHPC_OK;
-}
-
-void F64Staging::apply(double *ws, GemmDesc *descs, int ndesc) const {
-  for (int i = 0; i < ndesc; ++i) {
-    if (a_copy[i] >= 0) {
-      descs[i].A = ws + copies[a_copy[i]].off;
-      descs[i].lda = copies[a_copy[i]].pitch;
-    }
-    if (b_copy[i] >= 0) {
-      descs[i].B = ws + copies[b_copy[i]].off;
-      descs[i].ldb = copies[b_copy[i]].pitch;
-    }
-  }
-}
-
-int phpc_f64_reserve_staging(const GemmDesc *descs, int ndesc, hipStream_t stream) {
-  const int cfg = phpc_f64_pick_config_at(descs, ndesc);
-  if (!kConfigs[cfg].trans_a) return PHPC_OK;
-  F64Staging st;
-  st.plan(descs, ndesc);
-  std::lock_guard<std::mutex> lk(g_at_ws.mu);
-  g_at_ws.after_previous(stream);
-  if (!g_at_ws.ws.get(st.total * sizeof(double), 0, stream))
-    return phpc_set_error(PHPC_ERR_MEM, "transposed-A workspace allocation failed (%zu bytes)", st.total * 8);
-  g_at_ws.mark_used(stream);
-  return PHPC_OK;
-}
-
-int phpc_f64_transpose(const double *A, long lda, int m, int k, double *At, long ldat, hipStream_t stream) {
-  if (m <= 0 || k <= 0) return PHPC_OK;
-  const dim3 tg((unsigned)((k + 31) / 32), (unsigned)((ldat + 31) / 32));
-  hipLaunchKernelGGL(f64_transpose_kernel, tg, dim3(256), 0, stream, A, lda, m, k, At, ldat);
-  PHPC_HIP(hipGetLastError());
-  return PHPC_OK;
-}
-
-int phpc_f64_grouped_dev_at(const GemmDesc *descs_dev, const GemmDesc *descs_host, int ndesc, int grid,
-                            int config_id, hipStream_t stream) {
-  return launch_grouped(descs_dev, descs_host, ndesc, grid, config_id, stream, true);
-}
-
-int phpc_f64_pick_config_at(const GemmDesc *descs, int ndesc) {
-  const int cfg = phpc_f64_pick_config(descs, ndesc);
-  if (!phpc_f64_trans_a_ok(descs, ndesc)) return cfg;
-  if (cfg == g_big_single) return g_big_single_host;
-  if (cfg == g_big_config) return g_big_config_host;
-  return cfg;
-}
-
-int phpc_f64_grouped(const GemmDesc *descs_in, int ndesc, int grid, int config_id,
-                     hipStream_t stream) {
-  if (ndesc <= 0) return PHPC_OK;
-  for (int i = 0; i < ndesc; ++i) {
-    const GemmDesc &d = descs_in[i];
-    if (d.m < 0 || d.n < 0 || d.k < 0) return phpc_set_error(PHPC_ERR_ARG, "negative GEMM size");
-  }
-  std::vector<GemmDesc> descs(descs_in, descs_in + ndesc);
-  if (config_id < 0) config_id = phpc_f64_pick_config_at(descs.data(), ndesc);
-  if (config_id < 0 || config_id >= kNumConfigs)
-    return phpc_set_error(PHPC_ERR_ARG, "bad FP64 config id %d", config_id);
-  // the transposed copy needs 16-byte B rows and a grid-sized m; otherwise the same tile
-  // runs register-staged on A as it is
-  if (kConfigs[config_id].trans_a && !phpc_f64_trans_a_ok(descs.data(), ndesc))
-    config_id = kConfigs[config_id].bm == 256 ? 6 : kConfigs[config_id].panels ? 0 : 8;
-  const ConfigEntry &ce = kConfigs[config_id];
-  // drop empty GEMMs; k == 0 leaves C unchanged (C += 0 adds +0.0 only to tiles we skip)
-  std::vector<GemmDesc> live;
-  live.reserve(ndesc);
-  int start = 0;
-  for (auto d : descs) {
-    if (d.m == 0 || d.n == 0 || d.k == 0) continue;
-    d.tiles_n = (d.n + ce.bn - 1) / ce.bn;
-    d.tile_start = start;
-    start += ((d.m + ce.bm - 1) / ce.bm) * d.tiles_n;
-    live.push_back(d);
-  }
-  if (live.empty()) return PHPC_OK;
-  if (ce.trans_a) return launch_transposed(live, grid, config_id, stream);
-  return launch_live(live, grid, config_id, stream, false);
-}
-
-namespace {
-
-// One grouped launch of prepared descriptors (host copies in `live`).
-int launch_live(std::vector<GemmDesc> &live, int grid, int config_id, hipStream_t stream, bool a_transposed) {
-  if (live.size() == 1) return launch_grouped(nullptr, live.data(), 1, grid, config_id, stream, a_transposed);
-  // Several GEMMs: descriptors go through one process-wide device buffer. Callers on
-  // other streams may still have a launch queued that reads it, so the buffer is
-  // rewritten only after the previous user's launch has finished (g_desc_done).
+int phpc_f64_grouped(const GemmDesc *descs, int ndesc, int grid, int config_id, hipStream_t stream) {
+  F64Work w;
+  if (int rc = phpc_f64_prepare(descs, ndesc, config_id, false, &w)) return rc;
+  if (w.descs.size() <= 2) return phpc_f64_launch(w, nullptr, grid, stream);
+  // More GEMMs than travel with the launch: descriptors go through one process-wide device
+  // buffer. Callers on other streams may still have a launch queued that reads it, so the
+  // buffer is rewritten only after the previous user's launch has finished (g_desc_done).
   std::lock_guard<std::mutex> lk(g_desc_mu);
-  const size_t bytes = live.size() * sizeof(GemmDesc);
+  const size_t bytes = w.descs.size() * sizeof(GemmDesc);
   if (g_desc_done) PHPC_HIP(hipEventSynchronize(g_desc_done));
   if (bytes > g_desc_cap) {
     if (g_desc_dev) PHPC_HIP(hipFree(g_desc_dev));
@@ -1358,26 +1105,23 @@ int launch_live(std::vector<GemmDesc> &live, int grid, int config_id, hipStream_
     g_pinned_cap = cap;
   }
   if (!g_desc_done) PHPC_HIP(hipEventCreateWithFlags(&g_desc_done, hipEventDisableTiming));
-  memcpy(g_desc_pinned, live.data(), bytes);
+  memcpy(g_desc_pinned, w.descs.data(), bytes);
   PHPC_HIP(hipMemcpyAsync(g_desc_dev, g_desc_pinned, bytes, hipMemcpyHostToDevice, stream));
-  const int rc = launch_grouped(g_desc_dev, live.data(), (int)live.size(), grid, config_id, stream, a_transposed);
+  const int rc = phpc_f64_launch(w, g_desc_dev, grid, stream);
   PHPC_HIP(hipEventRecord(g_desc_done, stream));
   return rc;
 }
 
-}  // namespace
-
-// Tuning knobs for the autotuner: 0 = config for large panel-grouped problems, 1 =
-// tile-row swizzle width, 2 = XCD-contiguous tile order on/off, 3 = config for large
-// single-panel problems on device descriptors, 4 = the same through host descriptors
-// (may be a transposed-A configuration), 5 = large panel-grouped problems through host
-// descriptors.
+// Tuning knobs for the autotuner: 0 = config for large panel-grouped problems on device
+// descriptors, 1 = tile-row swizzle width, 2 = XCD-contiguous tile order on/off, 3 = config
+// for large single-panel problems on device descriptors, 4 = the same through host
+// descriptors, 5 = large panel-grouped problems through host descriptors.
 extern "C" int phpc_set_tuning(int key, int value) {
   switch (key) {
     case 0:
-      if (value < 0 || value >= kNumConfigs || kConfigs[value].trans_a)
-        return phpc_set_error(PHPC_ERR_ARG, "config %d out of range", value);
-      g_big_config = value;
+    case 3:
+      if (value < 0 || value >= 10) return phpc_set_error(PHPC_ERR_ARG, "config %d out of range", value);
+      (key == 0 ? g_big_config : g_big_single) = value;
       break;
     case 1:
       if (value < 1 || value > 64) return phpc_set_error(PHPC_ERR_ARG, "group width %d out of range", value);
@@ -1385,11 +1129,6 @@ extern "C" int phpc_set_tuning(int key, int value) {
       break;
     case 2:
       g_xcd_remap = value ? 1 : 0;
-      break;
-    case 3:
-      if (value < 0 || value >= kNumConfigs || kConfigs[value].trans_a)
-        return phpc_set_error(PHPC_ERR_ARG, "config %d out of range", value);
-      g_big_single = value;
       break;
     case 4:
       if (value < 0 || value >= kNumConfigs) return phpc_set_error(PHPC_ERR_ARG, "config %d out of range", value);
@@ -1412,18 +1151,6 @@ extern "C" int phpc_set_tuning(int key, int value) {
       return phpc_set_error(PHPC_ERR_ARG, "unknown tuning key %d", key);
   }
   return phpc_set_error(PHPC_OK, nullptr);
-}
-
-int phpc_f64_plan_tiles(GemmDesc *descs, int ndesc, int id) {
-  const ConfigEntry &ce = kConfigs[id];
-  int start = 0;
-  for (int i = 0; i < ndesc; ++i) {
-    GemmDesc &d = descs[i];
-    d.tiles_n = (d.n + ce.bn - 1) / ce.bn;
-    d.tile_start = start;
-    start += ((d.m + ce.bm - 1) / ce.bm) * d.tiles_n;
-  }
-  return start;
 }
 
 bool phpc_f64_config_panels(int id) { return id >= 0 && id < kNumConfigs && kConfigs[id].panels; }

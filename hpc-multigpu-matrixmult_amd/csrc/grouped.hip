@@ -21,11 +21,7 @@ struct phpc_plan {
   int total_tiles = 0;
   int grid = 0;
   double tuned_ms = 0.0;
-  // transposed-A configurations: the operand copies they read (plan-owned workspace) and
-  // the descriptors that point at them
-  F64Staging staging;
-  std::vector<GemmDesc> d64_at;
-  double *at_ws = nullptr;
+  F64Work w64;  // FP64: the items numbered for the configuration, as descs_dev holds them
   // the FP32 transposed-A configuration: staged copies, their list on the device, and the
   // descriptors that point at them
   F32Staging staging32;
@@ -59,21 +55,6 @@ std::string signature(int dtype, const phpc_gemm_item *it, int n) {
          std::to_string(it[i].panel) + "," + std::to_string(it[i].lda % 4) + std::to_string(it[i].ldb % 4) + ";";
   }
   return s;
-}
-
-// Transposed-A copies for a plan: allocated once (the plan keeps them), filled by every
-// launch before the GEMM kernel.
-int plan_prepare_at(phpc_plan *p) {
-  if (p->at_ws) return PHPC_OK;
-  p->staging.plan(p->d64.data(), p->count);
-  if (hipMalloc(&p->at_ws, p->staging.total * sizeof(double)) != hipSuccess) {
-    p->at_ws = nullptr;
-    return phpc_set_error(PHPC_ERR_MEM, "plan transposed-A workspace allocation failed (%zu bytes)",
-                          p->staging.total * 8);
-  }
-  p->d64_at = p->d64;
-  p->staging.apply(p->at_ws, p->d64_at.data(), p->count);
-  return PHPC_OK;
 }
 
 int plan_prepare_at32(phpc_plan *p) {
@@ -110,16 +91,12 @@ void plan_release_at32(phpc_plan *p) {
 int plan_upload(phpc_plan *p, int id, hipStream_t s) {
   size_t bytes;
   const void *src;
-  if (p->dtype == PHPC_F64 && phpc_f64_config_trans_a(id)) {
-    if (int rc = plan_prepare_at(p)) return rc;
-    p->total_tiles = phpc_f64_plan_tiles(p->d64_at.data(), p->count, id);
-    phpc_f64_plan_tiles(p->d64.data(), p->count, id);
-    bytes = sizeof(GemmDesc) * p->count;
-    src = p->d64_at.data();
-  } else if (p->dtype == PHPC_F64) {
-    p->total_tiles = phpc_f64_plan_tiles(p->d64.data(), p->count, id);
-    bytes = sizeof(GemmDesc) * p->count;
-    src = p->d64.data();
+  if (p->dtype == PHPC_F64) {
+    if (int rc = phpc_f64_prepare(p->d64.data(), p->count, id, true, &p->w64)) return rc;
+    p->total_tiles = p->w64.total;
+    bytes = sizeof(GemmDesc) * p->w64.descs.size();
+    src = p->w64.descs.data();
+    id = p->w64.config;
   } else if (p->dtype == PHPC_F32 && id == kF32AtConfig) {
     if (int rc = plan_prepare_at32(p)) return rc;
     p->total_tiles = phpc_f32_plan_tiles(p->d32_at.data(), p->count, id);
@@ -147,13 +124,7 @@ int plan_upload(phpc_plan *p, int id, hipStream_t s) {
 
 int launch(phpc_plan *p, hipStream_t s) {
   if (p->count == 0 || p->total_tiles == 0) return PHPC_OK;
-  if (p->dtype == PHPC_F64 && phpc_f64_config_trans_a(p->config)) {
-    if (int rc = p->staging.run(p->at_ws, s)) return rc;
-    return phpc_f64_grouped_dev_at((const GemmDesc *)p->descs_dev, p->d64_at.data(), p->count, p->grid, p->config,
-                                   s);
-  }
-  if (p->dtype == PHPC_F64)
-    return phpc_f64_grouped_dev((const GemmDesc *)p->descs_dev, p->d64.data(), p->count, p->grid, p->config, s);
+  if (p->dtype == PHPC_F64) return phpc_f64_launch(p->w64, (const GemmDesc *)p->descs_dev, p->grid, s);
   if (p->dtype == PHPC_F32 && p->config == kF32AtConfig) {
     if (int rc = p->staging32.run(p->copies_dev, s)) return rc;
     return phpc_f32_launch_at((const F32Desc *)p->descs_dev, p->d32_at.data(), p->count, p->total_tiles, p->grid, s);
@@ -231,15 +202,12 @@ extern "C" int phpc_plan_create(int dtype, const phpc_gemm_item *items, int coun
     *out = p;
     return phpc_set_error(PHPC_OK, nullptr);
   }
-  const size_t bytes = dtype == PHPC_F64 ? sizeof(GemmDesc) * p->count : sizeof(F32Desc) * p->count;  // F32, F32X3
+  const size_t bytes = dtype == PHPC_F64 ? 2 * sizeof(GemmDesc) * p->count : sizeof(F32Desc) * p->count;  // F32, F32X3
   if (hipMalloc(&p->descs_dev, bytes) != hipSuccess) {
     delete p;
     return phpc_set_error(PHPC_ERR_MEM, "descriptor allocation failed");
   }
-  // default choice: the planner's rule; large single-panel FP64 work takes the
-  // transposed-A kernel when B allows 16-byte loads (the plan then keeps a copy of A)
-  int cfg = dtype == PHPC_F64 ? phpc_f64_pick_config_at(p->d64.data(), p->count) : 0;
-  const bool at_ok = dtype == PHPC_F64 && phpc_f64_trans_a_ok(p->d64.data(), p->count);
+  int cfg = dtype == PHPC_F64 ? -1 : 0;  // the planner's rule
   const bool at32_ok = dtype == PHPC_F32 && phpc_f32_at_ok(p->d32.data(), p->count);
   if (dtype == PHPC_F32) cfg = phpc_f32_pick_plan_config(p->d32.data(), p->count);
   if (dtype == PHPC_F32X3) cfg = phpc_f32x3_pick_plan_config(p->d32.data(), p->count);
@@ -278,7 +246,6 @@ extern "C" int phpc_plan_create(int dtype, const phpc_gemm_item *items, int coun
       (void)hipEventCreate(&e1);
       for (int c = 0; c < ncfg; ++c) {
         if (dtype == PHPC_F64 && mp && !phpc_f64_config_panels(c)) continue;
-        if (dtype == PHPC_F64 && phpc_f64_config_trans_a(c) && !at_ok) continue;
         if (dtype == PHPC_F32X3 && c != 2 && c < kF32X3PlanesConfig) continue;
         if (dtype == PHPC_F32 && c == kF32AtConfig && !at32_ok) continue;
         if (plan_upload(p, c, s) != PHPC_OK) continue;
@@ -319,13 +286,6 @@ extern "C" int phpc_plan_create(int dtype, const phpc_gemm_item *items, int coun
   if (rc) {
     phpc_plan_destroy(p);
     return rc;
-  }
-  if (p->at_ws && !(dtype == PHPC_F64 && phpc_f64_config_trans_a(cfg))) {
-    // the autotuner tried a transposed-A configuration but kept another one
-    (void)hipStreamSynchronize(s);
-    (void)hipFree(p->at_ws);
-    p->at_ws = nullptr;
-    p->d64_at.clear();
   }
   if (p->at32_ws && cfg != kF32AtConfig) {
     (void)hipStreamSynchronize(s);
@@ -389,7 +349,6 @@ extern "C" void phpc_plan_destroy(phpc_plan_t p) {
     (void)hipEventDestroy(kv.second);
   }
   if (p->descs_dev) (void)hipFree(p->descs_dev);
-  if (p->at_ws) (void)hipFree(p->at_ws);
   plan_release_at32(p);
   p->planes.release();
   delete p;

@@ -186,8 +186,6 @@ int phpc_f32x3_launch(const F32Desc *descs_dev, const F32Desc *descs_host, int n
 int phpc_f32_launch(const F32Desc *descs_dev, const F32Desc *descs_host, int ndesc, int total_tiles, int id, bool vec4,
                     int grid, hipStream_t stream);
 
-// FP64: fill tiles_n / tile_start for config id; returns the total tile count.
-int phpc_f64_plan_tiles(GemmDesc *descs, int ndesc, int id);
 bool phpc_f64_config_panels(int id);
 
 // Kernel-level tile configuration chosen by the planner / autotuner.
@@ -215,54 +213,26 @@ struct DeviceInfo {
 };
 const DeviceInfo &phpc_device();
 
-// Grouped FP64 launch. `descs_host` are copied into a library-owned device buffer
-// (stream-ordered). `grid` <= 0 selects the autotuned persistent grid. Returns
-// PHPC_OK or an error code.
-int phpc_f64_grouped(const GemmDesc *descs_host, int ndesc, int grid, int config_id,
-                     hipStream_t stream);
-// Same, but with the descriptor array already resident on the device (graph-friendly).
-int phpc_f64_grouped_dev(const GemmDesc *descs_dev, const GemmDesc *descs_host, int ndesc,
-                         int grid, int config_id, hipStream_t stream);
+// Grouped FP64 launch. Descriptors that do not travel with the launch are copied into a
+// library-owned device buffer (stream-ordered). `grid` <= 0 selects the configuration's own
+// workgroup count, config_id < 0 the planner's. Returns PHPC_OK or an error code.
+int phpc_f64_grouped(const GemmDesc *descs_host, int ndesc, int grid, int config_id, hipStream_t stream);
+
+// A grouped FP64 launch prepared for one configuration: the GEMMs that hold work, numbered in
+// tiles, the ones cut off for the tail's smaller tiles (from tile tail_start on) last; at most
+// twice the GEMMs passed in. The caller of phpc_f64_launch holds `descs` on the device where
+// there are more than two. device_list: the work comes from a caller that keeps its
+// descriptors on the device (a plan, the serving loop), which two tuning knobs set apart.
+struct F64Work {
+  int config = 0;
+  bool mp = false, vec2 = false;
+  int total = 0, tail_start = 0;
+  std::vector<GemmDesc> descs;
+};
+int phpc_f64_prepare(const GemmDesc *descs, int ndesc, int config_id, bool device_list, F64Work *w);
+int phpc_f64_launch(const F64Work &w, const GemmDesc *descs_dev, int grid, hipStream_t stream);
 int phpc_f64_num_configs();
 F64Config phpc_f64_config(int id);
-int phpc_f64_pick_config(const GemmDesc *descs, int ndesc);
-// Configurations whose kernels read a transposed copy of A (descriptor A = At[k][m] with
-// lda = phpc_f64_at_pitch(m), pad column zero). phpc_f64_grouped stages the copy itself;
-// callers with device descriptors stage it with phpc_f64_transpose and launch through
-// phpc_f64_grouped_dev_at (phpc_f64_grouped_dev rejects these configurations).
-bool phpc_f64_config_trans_a(int id);
-bool phpc_f64_trans_a_ok(const GemmDesc *descs, int ndesc);
-long phpc_f64_at_pitch(int m);
-int phpc_f64_transpose(const double *A, long lda, int m, int k, double *At, long ldat, hipStream_t stream);
-
-// Operand copies that the transposed-A kernels read: At[k][m] for every distinct A block,
-// and, for a B block whose rows are not 16-byte aligned (base or odd ldb), a copy with an
-// even pitch. `plan` lists them and sizes the workspace; `run` fills a workspace; `apply`
-// points descriptors at the copies.
-struct F64Staging {
-  struct Copy {
-    const double *src;
-    long ld;
-    int rows, cols;  // of the source block
-    long pitch;      // of the copy
-    size_t off;      // doubles into the workspace
-    bool transpose;
-  };
-  std::vector<Copy> copies;
-  std::vector<int> a_copy, b_copy;  // per descriptor; b_copy -1: B is read in place
-  size_t total = 0;                 // doubles
-  void plan(const GemmDesc *descs, int ndesc);
-  int run(double *ws, hipStream_t stream) const;
-  void apply(double *ws, GemmDesc *descs, int ndesc) const;
-};
-int phpc_f64_grouped_dev_at(const GemmDesc *descs_dev, const GemmDesc *descs_host, int ndesc, int grid,
-                            int config_id, hipStream_t stream);
-// the planner's choice, with the transposed-A configuration for large single-panel work
-// whose B allows it
-int phpc_f64_pick_config_at(const GemmDesc *descs, int ndesc);
-// Size the process-wide staging workspace for these descriptors now, so that a pipeline
-// of host-pointer launches does not allocate between its copies.
-int phpc_f64_reserve_staging(const GemmDesc *descs, int ndesc, hipStream_t stream);
 
 // Strided block pack: dst[r*ldd + c] = src[r*lds + c] for r < rows, c < cols.
 // Host <-> device copies through pinned staging buffers (rows x width bytes, strided).

@@ -210,10 +210,9 @@ void phpc_server::process(Worker *w, std::vector<Req *> &batch) {
                                  &info);
     batch[0]->res.error_estimate = info.error_estimate;
   } else if (status == PHPC_OK && kind == kF64Plain) {
-    GemmDesc *gd = (GemmDesc *)w->desc_host;
+    std::vector<GemmDesc> gd(nb);
     for (int i = 0; i < nb; ++i) {
       const phpc_request &r = batch[i]->r;
-      gd[i] = GemmDesc{};
       gd[i].A = (const double *)ptr(batch[i], 0);
       gd[i].B = (const double *)ptr(batch[i], 1);
       gd[i].C = (double *)ptr(batch[i], 2);
@@ -225,11 +224,14 @@ void phpc_server::process(Worker *w, std::vector<Req *> &batch) {
       gd[i].k = r.k;
       gd[i].panel = 0;
     }
-    const int cfg = phpc_f64_pick_config(gd, nb);
-    phpc_f64_plan_tiles(gd, nb, cfg);
-    if (nb > 1 && hipMemcpyAsync(w->desc_dev, gd, sizeof(GemmDesc) * nb, hipMemcpyHostToDevice, s) != hipSuccess)
-      status = PHPC_ERR_HIP;
-    if (status == PHPC_OK) status = phpc_f64_grouped_dev((const GemmDesc *)w->desc_dev, gd, nb, 0, cfg, s);
+    F64Work work;
+    status = phpc_f64_prepare(gd.data(), nb, -1, true, &work);
+    const size_t bytes = sizeof(GemmDesc) * work.descs.size();
+    if (status == PHPC_OK && work.descs.size() > 2) {
+      memcpy(w->desc_host, work.descs.data(), bytes);
+      if (hipMemcpyAsync(w->desc_dev, w->desc_host, bytes, hipMemcpyHostToDevice, s) != hipSuccess) status = PHPC_ERR_HIP;
+    }
+    if (status == PHPC_OK) status = phpc_f64_launch(work, (const GemmDesc *)w->desc_dev, 0, s);
   } else if (status == PHPC_OK && !batch[0]->small && (long)batch[0]->r.m * batch[0]->r.n >= 2048L * 2048 &&
              batch[0]->r.k >= 256) {
     // a large FP32-class request: FP32-accurate 3 x BF16 slice planes, alone
@@ -347,7 +349,7 @@ extern "C" int phpc_server_create(size_t budget_bytes, int slots, int max_dim, i
   // per-slot split workspace for max_dim^3 at up to 20 moduli: two int8 operand copies,
   // 20 residue planes, metadata
   const size_t kp = (size_t)phpc_split_kp(max_dim);
-  const size_t desc_bytes = (size_t)batch_max * std::max(sizeof(GemmDesc), sizeof(F32Desc));
+  const size_t desc_bytes = (size_t)batch_max * std::max(2 * sizeof(GemmDesc), sizeof(F32Desc));
   int rc = PHPC_OK;
   for (int i = 0; i < slots && rc == PHPC_OK; ++i) {
     Worker *w = new Worker();

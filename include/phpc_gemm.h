@@ -88,9 +88,8 @@ int phpc_num_configs(void);
 /* Tuning knobs used by the autotuner: key 0 = FP64 config for large panel-grouped
  * problems on device-resident descriptor lists (plans fall back to it), key 1 = tile-row
  * swizzle width (1..64), key 2 = XCD-contiguous tile order (0/1), key 3 = FP64 config for
- * large single-panel problems on device-resident descriptor lists, key 4 / key 5 = FP64
- * config for large single-panel / panel-grouped problems through the entry points that
- * may stage a transposed copy of A (configs 10-12 read such a copy), key 6 = large
+ * large single-panel problems on device-resident descriptor lists (keys 0 and 3 take configs
+ * 0-9), key 4 / key 5 = FP64 config for large single-panel / panel-grouped problems, key 6 = large
  * single FP32 products through phpc_sgemm_device on the transposed-A FP32 kernel (1,
  * default) or on the register-staged one (0); 0 also keeps FP32 plans created without
  * autotuning off configuration 3; key 7 = FP32 configuration of plans created
