@@ -1,12 +1,16 @@
-// FP32 grouped GEMM on gfx950 matrix cores (v_mfma_f32_32x32x2f32): C += A*B for a list
-// of independent row-major FP32 GEMMs of any shapes, one persistent launch.
+// FP32 grouped GEMM on gfx950 matrix cores: C += A*B for a list of independent row-major FP32
+// GEMMs of any shapes, one launch. Two families: the direct kernels (gemm_rm.h,
+// v_mfma_f32_16x16x4f32), which every product takes whose leading dimensions fit their 32-bit
+// offsets, and the register-staged ones below (v_mfma_f32_32x32x2f32), for the others. Both sum
+// each output as one FMA chain in k order: the same bits.
 //
-// Same structure as the FP64 kernel: a BM x BN macro tile per workgroup, 4 waves in a
+// The register-staged kernels: a BM x BN macro tile per workgroup, 4 waves in a
 // 2 x 2 arrangement, operands staged HBM -> registers (raw buffer loads, out-of-range
 // lanes read zero) -> LDS (A transposed, At[k][m]; B as Bs[k][n]) in 16-deep slabs with
 // double buffering, and a persistent workgroup loop over the flat tile list of all GEMMs.
 // MFMA 32x32x2: lane l holds A[row l%32][k l/32] and B[k l/32][col l%32]; the 16
 // accumulators of lane l are rows 8(r/4) + 4(l/32) + r%4, column l%32.
+#include "gemm_rm.h"
 #include "phpc_internal.h"
 #include "phpc_split.h"
 
@@ -19,26 +23,9 @@ namespace {
 
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef float f4v __attribute__((ext_vector_type(4)));
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
 typedef float __attribute__((address_space(1))) gfloat;
 
-constexpr uint32_t kOOB = 0x80000000u;
 constexpr int BK = 16;
-
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ long uni(long v) {
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)(uint64_t)v);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)v >> 32));
-  return (long)(((uint64_t)hi << 32) | lo);
-}
-template <typename T>
-__device__ __forceinline__ T *uni(T *p) {
-  return reinterpret_cast<T *>(uni((long)reinterpret_cast<uintptr_t>(p)));
-}
-__device__ __forceinline__ rsrc_t make_rsrc(const void *base, long bytes) {
-  const uint32_t nb = bytes > 0x7fffffffL ? 0x7fffffffu : (uint32_t)(bytes < 0 ? 0 : bytes);
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)nb, 0x00020000);
-}
 
 struct F32Batch {
   const F32Desc *descs;
@@ -47,7 +34,7 @@ struct F32Batch {
   F32Desc d0;
 };
 
-__device__ __forceinline__ F32Desc uniform_desc(const F32Batch &b, int t) {
+__device__ __forceinline__ F32Desc f32_desc(const F32Batch &b, int t) {
   const F32Desc *d = &b.d0;
   if (b.ndesc > 1) {
     int lo = 0, hi = b.ndesc - 1;
@@ -96,7 +83,7 @@ __global__ __launch_bounds__(256) void f32_gemm_kernel(F32Batch batch) {
   for (int round = 0;; ++round) {
     const int t = round * G + slot;
     if (t >= batch.total_tiles) break;
-    const F32Desc d = uniform_desc(batch, uni(t));
+    const F32Desc d = f32_desc(batch, uni(t));
     const int lt = t - d.tile_start;
     const int row0 = uni((lt / d.tiles_n) * BM);
     const int col0 = uni((lt % d.tiles_n) * BN);
@@ -264,7 +251,7 @@ __global__ __launch_bounds__(256) void f32x3_gemm_kernel(F32Batch batch) {
   for (int round = 0;; ++round) {
     const int t = round * G + slot;
     if (t >= batch.total_tiles) break;
-    const F32Desc d = uniform_desc(batch, uni(t));
+    const F32Desc d = f32_desc(batch, uni(t));
     const int lt = t - d.tile_start;
     const int row0 = uni((lt / d.tiles_n) * BM);
     const int col0 = uni((lt % d.tiles_n) * BN);
@@ -387,241 +374,6 @@ __global__ __launch_bounds__(256) void f32x3_gemm_kernel(F32Batch batch) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// Transposed-A direct-to-LDS FP32 GEMM for large products: the caller stores A
-// transposed (At[k][m], row pitch = the descriptor's lda, a multiple of 4 floats, pad
-// columns zero) and B with 16-byte aligned rows, so both 16-row slabs are k-row-major and
-// reach LDS by 16-byte buffer loads with no staging registers and no LDS write
-// instructions. A 1 KiB load instruction fills two 128-float k rows; within a row the
-// 16-byte chunks of odd rows are XOR-permuted by 8, so the two half-waves of an MFMA
-// operand read (rows k and k+1) hit opposite halves of the banks. Two stages.
-// ---------------------------------------------------------------------------
-typedef __attribute__((address_space(3))) void lds_void;
-
-template <int N>
-__device__ __forceinline__ void f32_wait_vm() {
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 0xF) | (((N >> 4) & 3) << 14));
-}
-
-// B4: B rows need no alignment. Each B k row then arrives as two 4-byte-per-lane loads of 64
-// columns (lane i of half h at position 64 h + i holds column (64 h + i) ^ 32 on odd rows,
-// the same permutation as the 16-byte chunks' XOR by 8), exact to the last column of the
-// row; A still arrives in 1 KiB blocks.
-template <bool B4>
-__device__ __forceinline__ void f32_at_body(const F32Batch &batch) {
-  constexpr int BM = 128, BN = 128, WTM = 64, WTN = 64, TM = 2, TN = 2;
-  constexpr int ROW_BYTES = 512;                  // one 128-float k row
-  constexpr int A_BYTES = BK * ROW_BYTES;         // 16 rows
-  constexpr int STAGE_BYTES = 2 * A_BYTES;        // A then B
-  constexpr int A_BLOCKS = A_BYTES / 1024, BLOCKS = 2 * A_BLOCKS, PER = BLOCKS / 4;
-  constexpr int B4_PER = 2 * BK / 4;              // 4-byte B loads per wave and slab
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int tid = threadIdx.x;
-  const int wave = uni(tid >> 6);
-  const int lane = tid & 63;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int G = gridDim.x, bid = blockIdx.x;
-  const int slot = uni((G % 8) == 0 ? (bid % 8) * (G / 8) + bid / 8 : bid);
-  // this lane's place in any 1 KiB block: row pair offset (lane / 32) and chunk
-  const int lrow = lane >> 5;
-  const int lchunk = (lane & 31) ^ (lrow << 3);
-
-  for (int round = 0;; ++round) {
-    const int t = round * G + slot;
-    if (t >= batch.total_tiles) break;
-    const F32Desc d = uniform_desc(batch, uni(t));
-    const int lt = t - d.tile_start;
-    const int row0 = uni((lt / d.tiles_n) * BM);
-    const int col0 = uni((lt % d.tiles_n) * BN);
-    const int m_rem = d.m - row0, n_rem = d.n - col0;
-    const long ldat = d.lda, ldb = d.ldb, ldc = d.ldc;
-    const float *At_g = d.A + row0;
-    const float *Bg = d.B + col0;
-    gfloat *Cg = (gfloat *)(d.C + (long)row0 * ldc + col0);
-    const int Kdim = d.k;
-    const int nslab = (Kdim + BK - 1) / BK;
-
-    uint32_t goff[PER];
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int blk = wave + u * 4;
-      const bool isA = blk < A_BLOCKS;
-      const int r = 2 * (isA ? blk : blk - A_BLOCKS) + lrow;  // k row within the slab
-      const int c = lchunk * 4;                               // column of the chunk
-      const int rem = isA ? m_rem : n_rem;
-      goff[u] = c < rem ? (uint32_t)(((long)r * (isA ? ldat : ldb) + c) * 4) : kOOB;
-    }
-    uint32_t goff_b4[B4 ? B4_PER : 1];
-    if constexpr (B4) {
-#pragma unroll
-      for (int v = 0; v < B4_PER; ++v) {
-        const int j = wave + v * 4;  // row j / 2, half j % 2
-        const int r = j >> 1, h = j & 1;
-        const int c = (64 * h + lane) ^ ((r & 1) << 5);
-        goff_b4[v] = c < n_rem ? (uint32_t)(((long)r * ldb + c) * 4) : kOOB;
-      }
-    }
-    const int full_a = (int)(BK * ldat * 4), full_b = (int)(BK * ldb * 4);
-    auto issue = [&](int sidx) {
-      const int kb = sidx * BK;
-      const int krem = min(BK, Kdim - kb);
-      char *stage = smem + (sidx & 1) * STAGE_BYTES;
-      const int na = krem == BK ? full_a : krem * (int)ldat * 4;
-      const int nb = krem == BK ? full_b : krem * (int)ldb * 4;
-      const rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(At_g + (long)kb * ldat), (short)0, na,
-                                                          0x00020000);
-      const rsrc_t rB =
-          __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(Bg + (long)kb * ldb), (short)0, nb, 0x00020000);
-      if constexpr (B4) {
-#pragma unroll
-        for (int u = 0; u < A_BLOCKS / 4; ++u) {
-          const int blk = wave + u * 4;
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, (lds_void *)(stage + blk * 1024), 16, goff[u], 0, 0, 0);
-        }
-#pragma unroll
-        for (int v = 0; v < B4_PER; ++v) {
-          const int j = wave + v * 4;
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, (lds_void *)(stage + A_BYTES + (j >> 1) * ROW_BYTES + (j & 1) * 256),
-                                                    4, goff_b4[v], 0, 0, 0);
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < PER; ++u) {
-          const int blk = wave + u * 4;
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(blk < A_BLOCKS ? rA : rB, (lds_void *)(stage + blk * 1024), 16,
-                                                    goff[u], 0, 0, 0);
-        }
-      }
-    };
-
-    f16v acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = f16v{};
-
-    // LDS read offsets of this lane's operands for k step kk: row k = 2 kk + lane / 32
-    int a_off[TM], b_off[TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int col = wm * WTM + i * 32 + (lane & 31);
-      a_off[i] = lrow * ROW_BYTES + (((col >> 2) ^ (lrow << 3)) << 4) + (col & 3) * 4;
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int col = wn * WTN + j * 32 + (lane & 31);
-      b_off[j] = A_BYTES + lrow * ROW_BYTES + (((col >> 2) ^ (lrow << 3)) << 4) + (col & 3) * 4;
-    }
-
-    __syncthreads();
-    if (nslab > 0) issue(0);
-    for (int sidx = 0; sidx < nslab; ++sidx) {
-      f32_wait_vm<0>();
-      __syncthreads();
-      const char *stage = smem + (sidx & 1) * STAGE_BYTES;
-      auto kstep = [&](int kk) {
-        float a[TM], b[TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i) a[i] = *reinterpret_cast<const float *>(stage + a_off[i] + kk * 2 * ROW_BYTES);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) b[j] = *reinterpret_cast<const float *>(stage + b_off[j] + kk * 2 * ROW_BYTES);
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-      };
-      kstep(0);
-      if (sidx + 1 < nslab) issue(sidx + 1);
-#pragma unroll
-      for (int kk = 1; kk < BK / 2; ++kk) kstep(kk);
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int cc = wn * WTN + j * 32 + (lane & 31);
-        if (cc >= n_rem) continue;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int rr = wm * WTM + i * 32 + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4);
-          if (rr < m_rem) {
-            gfloat *pc = Cg + (long)rr * ldc + cc;
-            *pc = *pc + acc[i][j][r];
-          }
-        }
-      }
-  }
-}
-
-__global__ __launch_bounds__(256) void f32_at_128x128(F32Batch batch) { f32_at_body<false>(batch); }
-__global__ __launch_bounds__(256) void f32_at_128x128_b4(F32Batch batch) { f32_at_body<true>(batch); }
-
-// At[k][m] = A[m][k] for m < M, k < K; 0 for M <= m < ldat
-// 64 x 64 tiles, 16 entries per thread
-constexpr int kF32TransTile = 64;
-__global__ __launch_bounds__(256) void f32_transpose_kernel(const float *__restrict__ A, long lda, int M, int Kd,
-                                                            float *__restrict__ At, long ldat) {
-  constexpr int T = kF32TransTile;
-  __shared__ float tile[T][T + 1];
-  const int k0 = blockIdx.x * T, m0 = blockIdx.y * T;
-  const int tx = threadIdx.x % T, ty = threadIdx.x / T;
-  constexpr int RS = 256 / T;  // row step
-  float v[T / RS];
-#pragma unroll
-  for (int u = 0; u < T / RS; ++u) {
-    const int m = m0 + ty + u * RS, k = k0 + tx;
-    v[u] = load_or_zero(A, (long)m * lda + k, m < M && k < Kd);
-  }
-#pragma unroll
-  for (int u = 0; u < T / RS; ++u) tile[ty + u * RS][tx] = v[u];
-  __syncthreads();
-  // 16-byte stores: a thread writes 4 consecutive m of 4 rows k (ldat and m are multiples
-  // of 4, so a group lies wholly below or wholly past ldat)
-  static_assert(T == 64, "store groups assume 64 x 64 tiles");
-  const int q = threadIdx.x & 15;
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int r = (threadIdx.x >> 4) + 16 * u;
-    const int k = k0 + r, m = m0 + 4 * q;
-    if (k < Kd && m < ldat)
-      *reinterpret_cast<float4 *>(At + (long)k * ldat + m) =
-          make_float4(tile[4 * q][r], tile[4 * q + 1][r], tile[4 * q + 2][r], tile[4 * q + 3][r]);
-  }
-}
-
-// All transposed A copies of a grouped transposed-A launch in one kernel: one workgroup per
-// 64 x 64 tile of a copy's destination, its copy read from a per-tile table.
-__global__ __launch_bounds__(256) void f32_stage_kernel(const F32StageCopy *__restrict__ copies,
-                                                        const int *__restrict__ block_copy) {
-  __shared__ float tile[64][65];
-  const int b = blockIdx.x;
-  const F32StageCopy c = copies[block_copy[b]];
-  const int lb = b - c.block_start;
-  const int d0 = (lb / c.tiles_x) * 64;  // first destination row (k) of the tile
-  const int e0 = (lb % c.tiles_x) * 64;  // first destination column (m)
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  float v[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int sr = e0 + ty + 4 * i, sc = d0 + tx;
-    v[i] = load_or_zero(c.src, (long)sr * c.ld + sc, sr < c.rows && sc < c.cols);
-  }
-#pragma unroll
-  for (int i = 0; i < 16; ++i) tile[ty + 4 * i][tx] = v[i];
-  __syncthreads();
-  // 16-byte stores of 4 consecutive destination columns (pitch and dc are multiples of 4,
-  // copies 256-byte aligned)
-  const int q = threadIdx.x & 15;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = (threadIdx.x >> 4) + 16 * i;
-    const int dr = d0 + r, dc = e0 + 4 * q;
-    if (dr < c.cols && dc < c.pitch)
-      *reinterpret_cast<float4 *>(c.dst + (long)dr * c.pitch + dc) =
-          make_float4(tile[4 * q][r], tile[4 * q + 1][r], tile[4 * q + 2][r], tile[4 * q + 3][r]);
-  }
-}
-
 typedef void (*F32Fn)(F32Batch);
 struct F32Cfg {
   int bm, bn;
@@ -657,87 +409,54 @@ int occ(int c, int v) {
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-int g_f32_at = 1;  // large single FP32 products through the transposed-A kernel
+int g_f32_direct = 1;  // FP32 products through the direct kernels
 int g_f32_plan_cfg = -1;  // FP32 plans' configuration without autotuning (-1: by work)
-SharedWorkspace g_f32_at_ws;
-int g_f32_at_occ[2] = {0, 0};
 
-constexpr size_t kF32AtLds = 2 * 2 * 16 * 512;  // two stages of A and B slabs
-
-// b4: some B rows are not 16-byte aligned (or their pitch is not a multiple of 4 floats);
-// the kernel then loads B 4 bytes per lane
-int f32_at_run(const F32Batch &b, bool b4, int grid, hipStream_t stream) {
-  const void *fn = b4 ? reinterpret_cast<const void *>(f32_at_128x128_b4) : reinterpret_cast<const void *>(f32_at_128x128);
-  int &occ_v = g_f32_at_occ[b4 ? 1 : 0];
-  {
-    std::lock_guard<std::mutex> lk(g_mu);
-    if (!occ_v) {
-      (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kF32AtLds);
-      int n = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, 256, kF32AtLds) != hipSuccess || n < 1) n = 1;
-      occ_v = n;
-    }
-  }
-  int G = grid > 0 ? grid : occ_v * phpc_device().cus;
-  if (G > b.total_tiles) G = b.total_tiles;
-  if (G < 1) G = 1;
-  const int kt = phpc_ktime_begin(stream);
-  if (b4)
-    hipLaunchKernelGGL(f32_at_128x128_b4, dim3(G), dim3(256), kF32AtLds, stream, b);
-  else
-    hipLaunchKernelGGL(f32_at_128x128, dim3(G), dim3(256), kF32AtLds, stream, b);
-  phpc_ktime_end(kt, stream);
-  PHPC_HIP(hipGetLastError());
-  return PHPC_OK;
+// The direct kernels (gemm_rm.h) by tile shape: head T, tail U (the same type: no tail).
+struct F32RmConfig {
+  int bm, bn, threads;
+  int a_rows, b_rows;  // rows of A, rows of B under one 32-bit buffer offset
+  size_t lds_bytes;
+  void (*fn)(RmBatch<F32Desc>);
+  int tail_bm, tail_bn;  // 0: no tail
+};
+template <class T, class U>
+constexpr F32RmConfig f32_rm_config() {
+  constexpr bool same = std::is_same<T, U>::value;
+  return {T::BM, T::BN, T::THREADS, std::max(T::A_ROWS, U::A_ROWS), std::max(T::B_ROWS, U::B_ROWS),
+          (size_t)std::max(T::LDS, U::LDS), rm_kernel<T, U>, same ? 0 : U::BM, same ? 0 : U::BN};
 }
-
-bool b16_ok(const F32Desc &d) { return aligned16(d.B) && d.ldb % 4 == 0; }
-
-// One large FP32 GEMM: A staged transposed, then the transposed-A kernel over 128 x 128
-// tiles, B read in place (16-byte loads when its rows are 16-byte aligned with a pitch of 4
-// floats, else 4-byte loads). With 16-byte loads, the chunk holding a row's last column
-// starts on a 16-byte boundary and so lies in the same page as that column; its extra
-// columns only feed output columns that are never stored.
-int f32_launch_transposed(F32Desc d, hipStream_t stream) {
-  const long ldat = ((long)d.m + 3) / 4 * 4;
-  const size_t total = ((size_t)d.k * ldat + 63) / 64 * 64;
-  if (16L * ldat * 4 >= 0x7fffffffL || 16L * d.ldb * 4 >= 0x7fffffffL)
-    return phpc_set_error(PHPC_ERR_ARG, "leading dimension too large");
-  std::lock_guard<std::mutex> lk(g_f32_at_ws.mu);
-  g_f32_at_ws.after_previous(stream);
-  float *ws = static_cast<float *>(g_f32_at_ws.ws.get(total * sizeof(float), 0, stream));
-  if (!ws) return phpc_set_error(PHPC_ERR_MEM, "FP32 staging workspace allocation failed");
-  hipLaunchKernelGGL(f32_transpose_kernel,
-                     dim3((unsigned)((d.k + kF32TransTile - 1) / kF32TransTile),
-                          (unsigned)((ldat + kF32TransTile - 1) / kF32TransTile)),
-                     dim3(256), 0, stream, d.A, d.lda, d.m, d.k, ws, ldat);
-  PHPC_HIP(hipGetLastError());
-  d.A = ws;
-  d.lda = ldat;
-  d.tiles_n = (d.n + 127) / 128;
-  d.tile_start = 0;
-  const int total_tiles = ((d.m + 127) / 128) * d.tiles_n;
-  F32Batch b{};
-  b.ndesc = 1;
-  b.total_tiles = total_tiles;
-  b.d0 = d;
-  if (int rc = f32_at_run(b, !b16_ok(d), 0, stream)) return rc;
-  g_f32_at_ws.mark_used(stream);
-  return PHPC_OK;
-}
+using G32 = RmTile<float, 32, 32, 2, 2, 32, 4, false>;
+using G32K64 = RmTile<float, 32, 32, 2, 2, 64, 4, false>;
+using G64 = RmTile<float, 64, 64, 2, 2, 32, 4, false>;
+using G64W8 = RmTile<float, 64, 64, 4, 2, 32, 4, false>;
+using G128 = RmTile<float, 128, 64, 4, 2, 32, 3, false>;
+// The tile shapes of the planner's rule. Measured (device time): 256^3 5.4 us on 32x32 against
+// 9.5 on 64x64; 1500x1000x700 28.1 on 64x64 with the tail against 40 without it and 54.4 on the
+// register-staged 64x64 tiles before; 4096^3 949 us (145 TF/s) on 128x64 with two workgroups to
+// a CU, 966 on 64x64, 966 on 256x128 with one; 512 products log-uniform in [64, 4096] 9.25 ms
+// on 128x64, 9.45 on 64x64, 9.9 on 256x128, 11.6 before (128x128, operands staged).
+enum { kF32Small = 0, kF32Mid = 1, kF32Big = 2 };
+const F32RmConfig kF32Rm[] = {
+    f32_rm_config<G32, G32>(),
+    f32_rm_config<G64, G32K64>(),
+    f32_rm_config<G128, G64W8>(),
+};
+std::once_flag g_rm_once;
 
 }  // namespace
 
-static_assert(kF32AtConfig == kNumF32, "the transposed-A configuration follows the register-staged ones");
+static_assert(kF32DirectConfig == kNumF32, "the direct kernels follow the register-staged ones");
 
 int phpc_f32_num_configs() { return kNumF32 + 1; }
 
 void phpc_f32_config_tile(int id, int *bm, int *bn) {
-  *bm = id == kF32AtConfig ? 128 : kF32[id].bm;
-  *bn = id == kF32AtConfig ? 128 : kF32[id].bn;
+  *bm = kF32[id].bm;
+  *bn = kF32[id].bn;
 }
 
-// Fills tiles_n / tile_start of descs for config `id`; returns the total tile count.
+// Fills tiles_n / tile_start of descs for register-staged config `id`; returns the total tile
+// count.
 int phpc_f32_plan_tiles(F32Desc *descs, int ndesc, int id) {
   int bm, bn;
   phpc_f32_config_tile(id, &bm, &bn);
@@ -751,101 +470,70 @@ int phpc_f32_plan_tiles(F32Desc *descs, int ndesc, int id) {
   return start;
 }
 
-bool phpc_f32_at_ok(const F32Desc *descs, int ndesc) {
-  for (int i = 0; i < ndesc; ++i) {
-    const F32Desc &d = descs[i];
-    const long ldat = ((long)d.m + 3) / 4 * 4;
-    if (16L * ldat * 4 >= 0x7fffffffL || 16L * d.ldb * 4 >= 0x7fffffffL) return false;
-  }
+bool phpc_f32_direct_ok(const F32Desc *descs, int ndesc) {
+  for (int i = 0; i < ndesc; ++i)
+    for (const F32RmConfig &c : kF32Rm)
+      if ((long)c.a_rows * descs[i].lda * 4 >= 0x7fffffffL || (long)c.b_rows * descs[i].ldb * 4 >= 0x7fffffffL)
+        return false;
   return true;
 }
 
-void F32Staging::plan(const F32Desc *descs, int ndesc) {
-  copies.clear();
-  off.clear();
-  block_copy.clear();
-  a_copy.assign(ndesc, -1);
-  total = 0;
-  blocks = 0;
-  auto find_or_add = [&](const float *src, long ld, int rows, int cols) {
-    for (size_t j = 0; j < copies.size(); ++j) {
-      const F32StageCopy &c = copies[j];
-      if (c.src == src && c.ld == ld && c.rows == rows && c.cols == cols) return (int)j;
-    }
-    F32StageCopy c{};
-    c.src = src;
-    c.ld = ld;
-    c.rows = rows;
-    c.cols = cols;
-    c.pitch = ((long)rows + 3) / 4 * 4;
-    c.tiles_x = (int)((c.pitch + 63) / 64);
-    c.block_start = blocks;
-    const int nt = c.tiles_x * ((cols + 63) / 64);
-    blocks += nt;
-    block_copy.insert(block_copy.end(), nt, (int)copies.size());
-    copies.push_back(c);
-    off.push_back(total);
-    const size_t n = (size_t)cols * c.pitch;
-    total += (n + 63) / 64 * 64;  // 256-byte aligned copies
-    return (int)copies.size() - 1;
-  };
+int phpc_f32_prepare(const F32Desc *descs, int ndesc, F32Work *w) {
+  w->descs.clear();
+  w->total = w->tail_start = 0;
+  long t64 = 0, t128 = 0;
   for (int i = 0; i < ndesc; ++i) {
-    const F32Desc &d = descs[i];
-    if (d.m <= 0 || d.n <= 0 || d.k <= 0) continue;
-    a_copy[i] = find_or_add(d.A, d.lda, d.m, d.k);
+    if (descs[i].m <= 0 || descs[i].n <= 0 || descs[i].k <= 0) continue;
+    w->descs.push_back(descs[i]);
+    t64 += rm_tiles(descs[i], 64, 64);
+    t128 += rm_tiles(descs[i], 128, 64);
   }
-}
-
-void F32Staging::apply(float *ws, F32Desc *descs, int ndesc) {
-  for (size_t j = 0; j < copies.size(); ++j) copies[j].dst = ws + off[j];
-  for (int i = 0; i < ndesc; ++i) {
-    if (a_copy[i] >= 0) {
-      descs[i].A = copies[a_copy[i]].dst;
-      descs[i].lda = copies[a_copy[i]].pitch;
-    }
-  }
-}
-
-static size_t copies_bytes(size_t n) { return (n * sizeof(F32StageCopy) + 255) / 256 * 256; }
-
-size_t F32Staging::list_bytes() const { return copies_bytes(copies.size()) + block_copy.size() * sizeof(int); }
-
-int F32Staging::upload(void *list_dev) const {
-  if (copies.empty()) return PHPC_OK;
-  char *p = static_cast<char *>(list_dev);
-  PHPC_HIP(hipMemcpy(p, copies.data(), copies.size() * sizeof(F32StageCopy), hipMemcpyHostToDevice));
-  PHPC_HIP(hipMemcpy(p + copies_bytes(copies.size()), block_copy.data(), block_copy.size() * sizeof(int),
-                     hipMemcpyHostToDevice));
+  const long cus = phpc_device().cus;
+  // 128x64 tiles from four a CU on (two rounds of the two resident ones): 3000^3, 4.4 a CU, 404
+  // us against 416 on 64x64, but 2500^3, 3.1 a CU, 265 against 249. 32x32 tiles where 64x64 ones
+  // would leave CUs empty: 256^3 5.4 us against 9.5.
+  w->config = t128 >= 4 * cus ? kF32Big : t64 >= cus ? kF32Mid : kF32Small;
+  const F32RmConfig &c = kF32Rm[w->config];
+  if (!phpc_f32_direct_ok(w->descs.data(), (int)w->descs.size()))
+    return phpc_set_error(PHPC_ERR_ARG, "leading dimension too large");
+  std::vector<F32Desc> tail;
+  if (c.tail_bm) rm_split_tail(w->descs, c.bm, c.bn, cus, tail);
+  long t = 0;
+  bool fits = rm_number(w->descs, c.bm, c.bn, &t);
+  w->tail_start = (int)t;
+  fits = fits && rm_number(tail, c.tail_bm, c.tail_bn, &t);
+  if (!fits) return phpc_set_error(PHPC_ERR_ARG, "too many tiles");
+  w->total = (int)t;
+  w->descs.insert(w->descs.end(), tail.begin(), tail.end());
+  w->list.clear();
+  if (w->descs.size() > 2) w->list = rm_list(w->descs, w->total);
   return PHPC_OK;
 }
 
-int F32Staging::run(const void *list_dev, hipStream_t stream) const {
-  if (copies.empty() || blocks <= 0) return PHPC_OK;
-  const char *p = static_cast<const char *>(list_dev);
-  hipLaunchKernelGGL(f32_stage_kernel, dim3((unsigned)blocks), dim3(256), 0, stream,
-                     reinterpret_cast<const F32StageCopy *>(p), reinterpret_cast<const int *>(p + copies_bytes(copies.size())));
+int phpc_f32_launch_direct(const F32Work &w, const void *list_dev, int grid, hipStream_t stream) {
+  if (w.total <= 0) return PHPC_OK;
+  std::call_once(g_rm_once, [] {
+    for (const F32RmConfig &c : kF32Rm)
+      (void)hipFuncSetAttribute(reinterpret_cast<const void *>(c.fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)c.lds_bytes);
+  });
+  const F32RmConfig &c = kF32Rm[w.config];
+  RmBatch<F32Desc> b{};
+  b.descs = static_cast<const F32Desc *>(list_dev);
+  b.ndesc = (int)w.descs.size();
+  b.total_tiles = w.total;
+  b.group_m = 8;
+  b.xcd_remap = 1;
+  b.window = rm_window(!w.list.empty(), w.total, phpc_device().cus);
+  b.tail_start = w.tail_start;
+  b.d0 = w.descs[0];
+  if (b.ndesc == 2) b.d1 = w.descs[1];
+  const int G = grid > 0 ? std::min(grid, w.total) : w.total;
+  const int kt = phpc_ktime_begin(stream);
+  hipLaunchKernelGGL(c.fn, dim3(G), dim3(c.threads), c.lds_bytes, stream, b);
+  phpc_ktime_end(kt, stream);
   PHPC_HIP(hipGetLastError());
   return PHPC_OK;
-}
-
-int phpc_f32_launch_at(const F32Desc *descs_dev, const F32Desc *descs_host, int ndesc, int total_tiles, int grid,
-                       hipStream_t stream) {
-  if (ndesc <= 0 || total_tiles <= 0) return PHPC_OK;
-  bool b4 = false;
-  for (int i = 0; i < ndesc; ++i) {
-    const F32Desc &d = descs_host[i];
-    if (d.lda % 4 || !aligned16(d.A) || d.lda < ((long)d.m + 3) / 4 * 4)
-      return phpc_set_error(PHPC_ERR_ARG, "transposed-A FP32 launch needs a staged A");
-    if (16L * d.lda * 4 >= 0x7fffffffL || 16L * d.ldb * 4 >= 0x7fffffffL)
-      return phpc_set_error(PHPC_ERR_ARG, "leading dimension too large");
-    if (!b16_ok(d)) b4 = true;
-  }
-  F32Batch b{};
-  b.descs = descs_dev;
-  b.ndesc = ndesc;
-  b.total_tiles = total_tiles;
-  b.d0 = descs_host[0];
-  return f32_at_run(b, b4, grid, stream);
 }
 
 bool phpc_f32_vec4_ok(const F32Desc *descs, int ndesc) {
@@ -952,12 +640,13 @@ extern "C" int phpc_sgemm_device(const float *dA, long lda, const float *dB, lon
     const int tiles = phpc_f32_plan_tiles(&d, 1, 2);
     rc = phpc_f32x3_launch(nullptr, &d, 1, tiles, vec4, 0, (hipStream_t)stream);
   } else {
-    const long work = (long)((m + 127) / 128) * ((n + 127) / 128);
-    const int cfg = work >= 2L * phpc_device().cus ? 2 : 0;
-    // the transpose's grid.y is the staged pitch / 32
-    if (cfg == 2 && g_f32_at && (m + 3L) / 4 * 4 / 32 < 65535)
-      rc = f32_launch_transposed(d, (hipStream_t)stream);
-    else {
+    if (g_f32_direct && phpc_f32_direct_ok(&d, 1)) {
+      F32Work w;
+      rc = phpc_f32_prepare(&d, 1, &w);
+      if (!rc) rc = phpc_f32_launch_direct(w, nullptr, 0, (hipStream_t)stream);
+    } else {
+      const long work = (long)((m + 127) / 128) * ((n + 127) / 128);
+      const int cfg = work >= 2L * phpc_device().cus ? 2 : 0;
       const int tiles = phpc_f32_plan_tiles(&d, 1, cfg);
       rc = phpc_f32_launch(nullptr, &d, 1, tiles, cfg, vec4, 0, (hipStream_t)stream);
     }
@@ -965,18 +654,18 @@ extern "C" int phpc_sgemm_device(const float *dA, long lda, const float *dB, lon
   return rc ? rc : phpc_set_error(PHPC_OK, nullptr);
 }
 
-void phpc_f32_set_transposed_a(int on) { g_f32_at = on ? 1 : 0; }
+void phpc_f32_set_direct(int on) { g_f32_direct = on ? 1 : 0; }
 
 int phpc_f32_set_plan_config(int id) {
-  if (id < -1 || id > kF32AtConfig) return phpc_set_error(PHPC_ERR_ARG, "FP32 config %d out of range", id);
+  if (id < -1 || id > kF32DirectConfig) return phpc_set_error(PHPC_ERR_ARG, "FP32 config %d out of range", id);
   g_f32_plan_cfg = id;
   return phpc_set_error(PHPC_OK, nullptr);
 }
 
 int phpc_f32_pick_plan_config(const F32Desc *descs, int ndesc) {
-  if (g_f32_plan_cfg >= 0 && (g_f32_plan_cfg != kF32AtConfig || phpc_f32_at_ok(descs, ndesc))) return g_f32_plan_cfg;
+  if (g_f32_plan_cfg >= 0 && (g_f32_plan_cfg != kF32DirectConfig || phpc_f32_direct_ok(descs, ndesc))) return g_f32_plan_cfg;
+  if (g_f32_direct && phpc_f32_direct_ok(descs, ndesc)) return kF32DirectConfig;
   long work = 0;
   for (int i = 0; i < ndesc; ++i) work += (long)((descs[i].m + 127) / 128) * ((descs[i].n + 127) / 128);
-  if (work < 2L * phpc_device().cus) return 0;
-  return g_f32_at && phpc_f32_at_ok(descs, ndesc) ? kF32AtConfig : 2;
+  return work < 2L * phpc_device().cus ? 0 : 2;
 }

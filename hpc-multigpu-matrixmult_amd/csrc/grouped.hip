@@ -15,19 +15,15 @@ struct phpc_plan {
   int count = 0;
   std::vector<GemmDesc> d64;
   std::vector<F32Desc> d32;
-  void *descs_dev = nullptr;
+  void *descs_dev = nullptr;  // the list that the launch reads
+  size_t descs_cap = 0;
   int config = 0;
   bool vec = false;
   int total_tiles = 0;
   int grid = 0;
   double tuned_ms = 0.0;
   F64Work w64;  // FP64: the items numbered for the configuration, as descs_dev holds them
-  // the FP32 transposed-A configuration: staged copies, their list on the device, and the
-  // descriptors that point at them
-  F32Staging staging32;
-  std::vector<F32Desc> d32_at;
-  float *at32_ws = nullptr;
-  void *copies_dev = nullptr;  // the staging list (F32Staging::list_bytes)
+  F32Work w32;  // FP32 on the direct kernels: likewise
   // 3 x BF16 plans on slice planes (configurations kF32X3PlanesConfig + g): the planes,
   // the cut list and the level launch's items
   Bf3Planes planes;
@@ -57,36 +53,6 @@ std::string signature(int dtype, const phpc_gemm_item *it, int n) {
   return s;
 }
 
-int plan_prepare_at32(phpc_plan *p) {
-  if (p->at32_ws) return PHPC_OK;
-  p->staging32.plan(p->d32.data(), p->count);
-  const size_t ws_bytes = p->staging32.total * sizeof(float);
-  const size_t list_bytes = p->staging32.list_bytes();
-  if (hipMalloc(&p->at32_ws, ws_bytes) != hipSuccess) {
-    p->at32_ws = nullptr;
-    return phpc_set_error(PHPC_ERR_MEM, "plan FP32 staging workspace allocation failed (%zu bytes)", ws_bytes);
-  }
-  if (list_bytes && hipMalloc(&p->copies_dev, list_bytes) != hipSuccess) {
-    p->copies_dev = nullptr;
-    (void)hipFree(p->at32_ws);
-    p->at32_ws = nullptr;
-    return phpc_set_error(PHPC_ERR_MEM, "plan FP32 staging list allocation failed");
-  }
-  p->d32_at = p->d32;
-  p->staging32.apply(p->at32_ws, p->d32_at.data(), p->count);
-  if (list_bytes)
-    if (int rc = p->staging32.upload(p->copies_dev)) return rc;
-  return PHPC_OK;
-}
-
-void plan_release_at32(phpc_plan *p) {
-  if (p->copies_dev) (void)hipFree(p->copies_dev);
-  if (p->at32_ws) (void)hipFree(p->at32_ws);
-  p->copies_dev = nullptr;
-  p->at32_ws = nullptr;
-  p->d32_at.clear();
-}
-
 // (re)plan tiles for config id and upload the descriptors
 int plan_upload(phpc_plan *p, int id, hipStream_t s) {
   size_t bytes;
@@ -94,16 +60,14 @@ int plan_upload(phpc_plan *p, int id, hipStream_t s) {
   if (p->dtype == PHPC_F64) {
     if (int rc = phpc_f64_prepare(p->d64.data(), p->count, id, true, &p->w64)) return rc;
     p->total_tiles = p->w64.total;
-    bytes = sizeof(GemmDesc) * p->w64.descs.size();
-    src = p->w64.descs.data();
+    bytes = p->w64.list.size();
+    src = p->w64.list.data();
     id = p->w64.config;
-  } else if (p->dtype == PHPC_F32 && id == kF32AtConfig) {
-    if (int rc = plan_prepare_at32(p)) return rc;
-    p->total_tiles = phpc_f32_plan_tiles(p->d32_at.data(), p->count, id);
-    phpc_f32_plan_tiles(p->d32.data(), p->count, id);
-    p->vec = true;
-    bytes = sizeof(F32Desc) * p->count;
-    src = p->d32_at.data();
+  } else if (p->dtype == PHPC_F32 && id == kF32DirectConfig) {
+    if (int rc = phpc_f32_prepare(p->d32.data(), p->count, &p->w32)) return rc;
+    p->total_tiles = p->w32.total;
+    bytes = p->w32.list.size();
+    src = p->w32.list.data();
   } else if (p->dtype == PHPC_F32X3 && id >= kF32X3PlanesConfig) {
     if (int rc = p->planes.build(p->d32.data(), p->count, id - kF32X3PlanesConfig)) return rc;
     p->total_tiles = p->planes.total_tiles;
@@ -117,6 +81,19 @@ int plan_upload(phpc_plan *p, int id, hipStream_t s) {
     src = p->d32.data();
   }
   p->config = id;
+  if (bytes == 0) return PHPC_OK;
+  if (bytes > p->descs_cap) {
+    // the autotuner's launch of the configuration before may still read the old list
+    PHPC_HIP(hipStreamSynchronize(s));
+    if (p->descs_dev) PHPC_HIP(hipFree(p->descs_dev));
+    p->descs_dev = nullptr;
+    p->descs_cap = 0;
+    if (hipMalloc(&p->descs_dev, bytes) != hipSuccess) {
+      p->descs_dev = nullptr;
+      return phpc_set_error(PHPC_ERR_MEM, "descriptor allocation failed");
+    }
+    p->descs_cap = bytes;
+  }
   PHPC_HIP(hipMemcpyAsync(p->descs_dev, src, bytes, hipMemcpyHostToDevice, s));
   PHPC_HIP(hipStreamSynchronize(s));
   return PHPC_OK;
@@ -124,11 +101,9 @@ int plan_upload(phpc_plan *p, int id, hipStream_t s) {
 
 int launch(phpc_plan *p, hipStream_t s) {
   if (p->count == 0 || p->total_tiles == 0) return PHPC_OK;
-  if (p->dtype == PHPC_F64) return phpc_f64_launch(p->w64, (const GemmDesc *)p->descs_dev, p->grid, s);
-  if (p->dtype == PHPC_F32 && p->config == kF32AtConfig) {
-    if (int rc = p->staging32.run(p->copies_dev, s)) return rc;
-    return phpc_f32_launch_at((const F32Desc *)p->descs_dev, p->d32_at.data(), p->count, p->total_tiles, p->grid, s);
-  }
+  if (p->dtype == PHPC_F64) return phpc_f64_launch(p->w64, p->descs_dev, p->grid, s);
+  if (p->dtype == PHPC_F32 && p->config == kF32DirectConfig)
+    return phpc_f32_launch_direct(p->w32, p->descs_dev, p->grid, s);
   if (p->dtype == PHPC_F32X3 && p->config >= kF32X3PlanesConfig) return p->planes.run(s, p->grid);
   if (p->dtype == PHPC_F32X3)
     return phpc_f32x3_launch((const F32Desc *)p->descs_dev, p->d32.data(), p->count, p->total_tiles, p->vec, p->grid,
@@ -202,13 +177,8 @@ extern "C" int phpc_plan_create(int dtype, const phpc_gemm_item *items, int coun
     *out = p;
     return phpc_set_error(PHPC_OK, nullptr);
   }
-  const size_t bytes = dtype == PHPC_F64 ? 2 * sizeof(GemmDesc) * p->count : sizeof(F32Desc) * p->count;  // F32, F32X3
-  if (hipMalloc(&p->descs_dev, bytes) != hipSuccess) {
-    delete p;
-    return phpc_set_error(PHPC_ERR_MEM, "descriptor allocation failed");
-  }
   int cfg = dtype == PHPC_F64 ? -1 : 0;  // the planner's rule
-  const bool at32_ok = dtype == PHPC_F32 && phpc_f32_at_ok(p->d32.data(), p->count);
+  const bool direct_ok = dtype == PHPC_F32 && phpc_f32_direct_ok(p->d32.data(), p->count);
   if (dtype == PHPC_F32) cfg = phpc_f32_pick_plan_config(p->d32.data(), p->count);
   if (dtype == PHPC_F32X3) cfg = phpc_f32x3_pick_plan_config(p->d32.data(), p->count);
   if (flags & PHPC_PLAN_AUTOTUNE) {
@@ -247,7 +217,7 @@ extern "C" int phpc_plan_create(int dtype, const phpc_gemm_item *items, int coun
       for (int c = 0; c < ncfg; ++c) {
         if (dtype == PHPC_F64 && mp && !phpc_f64_config_panels(c)) continue;
         if (dtype == PHPC_F32X3 && c != 2 && c < kF32X3PlanesConfig) continue;
-        if (dtype == PHPC_F32 && c == kF32AtConfig && !at32_ok) continue;
+        if (dtype == PHPC_F32 && c == kF32DirectConfig && !direct_ok) continue;
         if (plan_upload(p, c, s) != PHPC_OK) continue;
         p->grid = 0;
         if (launch(p, s) != PHPC_OK) continue;
@@ -286,10 +256,6 @@ extern "C" int phpc_plan_create(int dtype, const phpc_gemm_item *items, int coun
   if (rc) {
     phpc_plan_destroy(p);
     return rc;
-  }
-  if (p->at32_ws && cfg != kF32AtConfig) {
-    (void)hipStreamSynchronize(s);
-    plan_release_at32(p);
   }
   if (p->planes.ws && cfg < kF32X3PlanesConfig) {
     (void)hipStreamSynchronize(s);
@@ -349,7 +315,6 @@ extern "C" void phpc_plan_destroy(phpc_plan_t p) {
     (void)hipEventDestroy(kv.second);
   }
   if (p->descs_dev) (void)hipFree(p->descs_dev);
-  plan_release_at32(p);
   p->planes.release();
   delete p;
 }

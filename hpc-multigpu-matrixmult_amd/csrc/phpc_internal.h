@@ -78,49 +78,26 @@ struct F32Desc {
 int phpc_f32_num_configs();
 void phpc_f32_config_tile(int id, int *bm, int *bn);
 int phpc_f32_plan_tiles(F32Desc *descs, int ndesc, int id);
-void phpc_f32_set_transposed_a(int on);
-// configuration of FP32 plans created without autotuning: -1 = by work (at least two
-// 128x128 tiles per CU: the transposed-A configuration 3, or 2 where its staged copies would
-// not fit its 32-bit offsets or tuning key 6 is off; else 0, 64x64); 0-3 = that
-// configuration (3 where it applies)
+void phpc_f32_set_direct(int on);
+// configuration of FP32 plans created without autotuning: -1 = the direct kernels
+// (configuration 3), or by work 0 (64x64) or 2 (128x128) where a leading dimension does not fit
+// their 32-bit offsets or tuning key 6 is off; 0-3 = that configuration (3 where it applies)
 int phpc_f32_set_plan_config(int id);
 int phpc_f32_pick_plan_config(const struct F32Desc *descs, int ndesc);
-// FP32 configuration ids: 0-2 register-staged (64x64, 128x64, 128x128); kF32AtConfig is the
-// transposed-A direct-to-LDS kernel (128x128), which reads staged operand copies.
-constexpr int kF32AtConfig = 3;
-// One transposed A copy of a grouped FP32 transposed-A launch, filled by one batched kernel:
-// dst[c][r] = src[r][c] for r < rows, c < cols, zero for rows <= r < pitch. 64 x 64 tiles of
-// dst, tiles_x across a dst row; block_start is the first tile's index in the batched grid.
-// B is read in place (the kernel loads unaligned B rows 4 bytes per lane).
-struct F32StageCopy {
-  const float *src;
-  long ld;
-  int rows, cols;
-  float *dst;
-  long pitch;
-  int tiles_x;
-  int block_start;
+// FP32 configuration ids: 0-2 register-staged (64x64, 128x64, 128x128); kF32DirectConfig the
+// direct kernels, whose tile shape follows from the work.
+constexpr int kF32DirectConfig = 3;
+// the descriptors fit the direct kernels' 32-bit buffer offsets
+bool phpc_f32_direct_ok(const F32Desc *descs, int ndesc);
+// A launch of the direct FP32 kernels: as F64Work
+struct F32Work {
+  int config = 0;
+  int total = 0, tail_start = 0;
+  std::vector<F32Desc> descs;
+  std::vector<char> list;
 };
-struct F32Staging {
-  std::vector<F32StageCopy> copies;  // dst set by apply
-  std::vector<size_t> off;           // floats into the workspace, per copy
-  std::vector<int> a_copy;           // per descriptor
-  std::vector<int> block_copy;       // the copy of each tile of the batched kernel
-  size_t total = 0;                  // floats
-  int blocks = 0;                    // tiles of the batched copy kernel
-  void plan(const F32Desc *descs, int ndesc);
-  void apply(float *ws, F32Desc *descs, int ndesc);
-  // the device list the kernel reads: the copies (dst set by apply), then block_copy
-  size_t list_bytes() const;
-  int upload(void *list_dev) const;
-  int run(const void *list_dev, hipStream_t stream) const;
-};
-// the descriptors fit the transposed-A kernel's 32-bit buffer offsets once staged
-bool phpc_f32_at_ok(const F32Desc *descs, int ndesc);
-// transposed-A kernel over descriptors already pointing at staged copies (tiles planned
-// with config kF32AtConfig); grid 0 = persistent default
-int phpc_f32_launch_at(const F32Desc *descs_dev, const F32Desc *descs_host, int ndesc, int total_tiles, int grid,
-                       hipStream_t stream);
+int phpc_f32_prepare(const F32Desc *descs, int ndesc, F32Work *w);
+int phpc_f32_launch_direct(const F32Work &w, const void *list_dev, int grid, hipStream_t stream);
 bool phpc_f32_vec4_ok(const F32Desc *descs, int ndesc);
 
 // FP32-accurate grouped plans on BF16 slice planes (3 x BF16). One batched kernel cuts
@@ -220,17 +197,19 @@ int phpc_f64_grouped(const GemmDesc *descs_host, int ndesc, int grid, int config
 
 // A grouped FP64 launch prepared for one configuration: the GEMMs that hold work, numbered in
 // tiles, the ones cut off for the tail's smaller tiles (from tile tail_start on) last; at most
-// twice the GEMMs passed in. The caller of phpc_f64_launch holds `descs` on the device where
-// there are more than two. device_list: the work comes from a caller that keeps its
-// descriptors on the device (a plan, the serving loop), which two tuning knobs set apart.
+// twice the GEMMs passed in. Where there are more than two, they do not travel with the launch:
+// the caller of phpc_f64_launch holds a copy of `list` on the device. device_list: the work
+// comes from a caller that keeps it there (a plan, the serving loop), which two tuning knobs
+// set apart.
 struct F64Work {
   int config = 0;
   bool mp = false, vec2 = false;
   int total = 0, tail_start = 0;
   std::vector<GemmDesc> descs;
+  std::vector<char> list;  // empty where the descriptors travel with the launch
 };
 int phpc_f64_prepare(const GemmDesc *descs, int ndesc, int config_id, bool device_list, F64Work *w);
-int phpc_f64_launch(const F64Work &w, const GemmDesc *descs_dev, int grid, hipStream_t stream);
+int phpc_f64_launch(const F64Work &w, const void *list_dev, int grid, hipStream_t stream);
 int phpc_f64_num_configs();
 F64Config phpc_f64_config(int id);
 

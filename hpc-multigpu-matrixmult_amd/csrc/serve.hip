@@ -200,6 +200,14 @@ void phpc_server::process(Worker *w, std::vector<Req *> &batch) {
     if (status) break;
   }
   (void)hipEventRecord(w->ev[1], s);
+  // a batch's list, where its descriptors do not travel with the launch
+  auto upload = [&](const std::vector<char> &list) {
+    if (list.empty()) return PHPC_OK;
+    if (list.size() > w->desc_cap) return PHPC_ERR_MEM;
+    memcpy(w->desc_host, list.data(), list.size());
+    return hipMemcpyAsync(w->desc_dev, w->desc_host, list.size(), hipMemcpyHostToDevice, s) == hipSuccess ? PHPC_OK
+                                                                                                    : PHPC_ERR_HIP;
+  };
   const Kind kind = batch[0]->kind;
   const int nb = (int)batch.size();
   if (status == PHPC_OK && kind == kF64Split) {
@@ -226,12 +234,8 @@ void phpc_server::process(Worker *w, std::vector<Req *> &batch) {
     }
     F64Work work;
     status = phpc_f64_prepare(gd.data(), nb, -1, true, &work);
-    const size_t bytes = sizeof(GemmDesc) * work.descs.size();
-    if (status == PHPC_OK && work.descs.size() > 2) {
-      memcpy(w->desc_host, work.descs.data(), bytes);
-      if (hipMemcpyAsync(w->desc_dev, w->desc_host, bytes, hipMemcpyHostToDevice, s) != hipSuccess) status = PHPC_ERR_HIP;
-    }
-    if (status == PHPC_OK) status = phpc_f64_launch(work, (const GemmDesc *)w->desc_dev, 0, s);
+    if (status == PHPC_OK) status = upload(work.list);
+    if (status == PHPC_OK) status = phpc_f64_launch(work, w->desc_dev, 0, s);
   } else if (status == PHPC_OK && !batch[0]->small && (long)batch[0]->r.m * batch[0]->r.n >= 2048L * 2048 &&
              batch[0]->r.k >= 256) {
     // a large FP32-class request: FP32-accurate 3 x BF16 slice planes, alone
@@ -239,11 +243,9 @@ void phpc_server::process(Worker *w, std::vector<Req *> &batch) {
     status = phpc_sgemm_bf16x3_planes((const float *)ptr(batch[0], 0), r.k, (const float *)ptr(batch[0], 1), r.n,
                                       (float *)ptr(batch[0], 2), r.n, r.m, r.k, r.n, s, &w->ws);
   } else if (status == PHPC_OK) {
-    F32Desc *fd = (F32Desc *)w->desc_host;
-    long work = 0;
+    std::vector<F32Desc> fd(nb);
     for (int i = 0; i < nb; ++i) {
       const phpc_request &r = batch[i]->r;
-      fd[i] = F32Desc{};
       fd[i].A = (const float *)ptr(batch[i], 0);
       fd[i].B = (const float *)ptr(batch[i], 1);
       fd[i].C = (float *)ptr(batch[i], 2);
@@ -253,14 +255,11 @@ void phpc_server::process(Worker *w, std::vector<Req *> &batch) {
       fd[i].m = r.m;
       fd[i].n = r.n;
       fd[i].k = r.k;
-      work += (long)((r.m + 127) / 128) * ((r.n + 127) / 128);
     }
-    const int cfg = work >= 2L * phpc_device().cus ? 2 : 0;
-    const int tiles = phpc_f32_plan_tiles(fd, nb, cfg);
-    if (nb > 1 && hipMemcpyAsync(w->desc_dev, fd, sizeof(F32Desc) * nb, hipMemcpyHostToDevice, s) != hipSuccess)
-      status = PHPC_ERR_HIP;
-    if (status == PHPC_OK)
-      status = phpc_f32_launch((const F32Desc *)w->desc_dev, fd, nb, tiles, cfg, phpc_f32_vec4_ok(fd, nb), 0, s);
+    F32Work work;
+    status = phpc_f32_prepare(fd.data(), nb, &work);
+    if (status == PHPC_OK) status = upload(work.list);
+    if (status == PHPC_OK) status = phpc_f32_launch_direct(work, w->desc_dev, 0, s);
   }
   (void)hipEventRecord(w->ev[2], s);
   for (int i = 0; i < nb && status == PHPC_OK; ++i) {
@@ -349,7 +348,9 @@ extern "C" int phpc_server_create(size_t budget_bytes, int slots, int max_dim, i
   // per-slot split workspace for max_dim^3 at up to 20 moduli: two int8 operand copies,
   // 20 residue planes, metadata
   const size_t kp = (size_t)phpc_split_kp(max_dim);
-  const size_t desc_bytes = (size_t)batch_max * std::max(2 * sizeof(GemmDesc), sizeof(F32Desc));
+  // per request: two descriptors and the list's index, an entry for every 64 of its tiles; a
+  // batched request has fewer than 256 tiles of 256x128, so at most 8192 of the smallest
+  const size_t desc_bytes = (size_t)batch_max * (2 * std::max(sizeof(GemmDesc), sizeof(F32Desc)) + 512) + 64;
   int rc = PHPC_OK;
   for (int i = 0; i < slots && rc == PHPC_OK; ++i) {
     Worker *w = new Worker();

@@ -89,13 +89,12 @@ int phpc_num_configs(void);
  * problems on device-resident descriptor lists (plans fall back to it), key 1 = tile-row
  * swizzle width (1..64), key 2 = XCD-contiguous tile order (0/1), key 3 = FP64 config for
  * large single-panel problems on device-resident descriptor lists (keys 0 and 3 take configs
- * 0-9), key 4 / key 5 = FP64 config for large single-panel / panel-grouped problems, key 6 = large
- * single FP32 products through phpc_sgemm_device on the transposed-A FP32 kernel (1,
- * default) or on the register-staged one (0); 0 also keeps FP32 plans created without
- * autotuning off configuration 3; key 7 = FP32 configuration of plans created
- * without autotuning (-1 = by work, default: 3 for at least two 128x128 tiles per CU, else
- * 0; 0-2 = register-staged 64x64, 128x64, 128x128; 3 = transposed-A 128x128, with the plan
- * keeping staged operand copies); key 8 = configuration of 3 x BF16 (PHPC_F32X3) plans
+ * 0-9), key 4 / key 5 = FP64 config for large single-panel / panel-grouped problems, key 6 =
+ * FP32 products through phpc_sgemm_device on the direct-to-LDS FP32 kernels (1, default) or
+ * on the register-staged ones (0); 0 also keeps FP32 plans created without autotuning off
+ * configuration 3; key 7 = FP32 configuration of plans created without autotuning (-1,
+ * default = 3; 0-2 = register-staged 64x64, 128x64, 128x128; 3 = the direct-to-LDS kernels
+ * on tiles picked by the work; all give the same bits); key 8 = configuration of 3 x BF16 (PHPC_F32X3) plans
  * created without autotuning (-1 = by work, default: 6 for at least one 256x256 tile per
  * CU, else 2; 2 = BF16 slices cut in registers, 128x128 tiles; 4, 5, 6 = BF16 slice planes
  * cut once per operand, then one grouped level launch on 128x128, 256x128 or 256x256 tiles,
