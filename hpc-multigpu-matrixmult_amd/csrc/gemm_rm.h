@@ -118,6 +118,127 @@ __device__ __forceinline__ void wait_vm_c() {
 // from moving memory operations across it.
 __device__ __forceinline__ void slab_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
+// C at a wave's tile: TM x TN MFMA blocks of MI x MI outputs, NR registers a lane each. Blocks
+// are read ahead and written, by buffer accesses whose lanes past the matrix edge are out
+// of range, so that nothing branches and several blocks' loads are in flight: element by
+// element (load, wait, add, store), 64 memory latencies in a row ended a 256x128 tile (FP64
+// 7187^3 in SUMMA steps 11.29 ms, 10.96 now).
+// Where a tile's rows span 2 GiB or more, lanes check and use full addresses.
+template <class E, class Acc, int TM, int TN, int MI, int NR>
+struct CTile {
+  typedef E __attribute__((address_space(1))) global_t;
+  static constexpr int SZ = sizeof(E);
+  static constexpr int kAhead = NR * SZ > 32 ? 2 : 128 / (NR * SZ);  // blocks in flight, 32 registers
+  rsrc_t rs;
+  global_t *C;
+  long ldc;
+  int m_rem, n_rem, lrow, lcol;
+  bool near;
+  uint32_t off[TN];
+  // C: the tile's first output; m_rem x n_rem outputs are the matrix's
+  __device__ __forceinline__ CTile(E *c, long ldc_, int m_rem_, int n_rem_, int lane)
+      : C((global_t *)c), ldc(ldc_), m_rem(m_rem_), n_rem(n_rem_) {
+    lrow = MI == 32 ? 4 * (lane >> 5) : SZ == 8 ? lane >> 4 : 4 * (lane >> 4);
+    lcol = lane % MI;
+    near = (long)TM * MI * ldc * SZ < 0x7fffffffL;
+    rs = make_rsrc(c, 0x7fffffffL);
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      off[j] = lcol + j * MI < n_rem ? (uint32_t)(((long)lrow * ldc + lcol + j * MI) * SZ) : kOOB;
+  }
+  // row of register r of block row i: a part of its own and the lane's
+  static __device__ __forceinline__ constexpr int row(int i, int r) {
+    return i * MI + (MI == 32 ? 8 * (r / 4) + r % 4 : SZ == 8 ? 4 * r : r);
+  }
+  __device__ __forceinline__ bool inside(int i, int j, int r, int lrow) const {
+    return row(i, r) + lrow < m_rem && lcol + j * MI < n_rem;
+  }
+  __device__ __forceinline__ global_t *at(int i, int j, int r, int lrow) const {
+    return C + (long)(row(i, r) + lrow) * ldc + lcol + j * MI;
+  }
+  template <bool NEAR>
+  __device__ __forceinline__ Acc load(int i, int j) const {
+    Acc c;
+    int lrow = this->lrow;
+    asm volatile("" : "+v"(lrow));  // its row tests are made again for the stores, not kept
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if constexpr (NEAR) {
+        const uint32_t o = row(i, r) + lrow < m_rem ? off[j] : kOOB;
+        const int so = (int)(row(i, r) * ldc * SZ);
+        if constexpr (SZ == 8)
+          c[r] = __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b64(rs, o, so, 0));
+        else
+          c[r] = __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b32(rs, o, so, 0));
+      } else {
+        c[r] = inside(i, j, r, lrow) ? *at(i, j, r, lrow) : E(0);
+      }
+    }
+    return c;
+  }
+  template <bool NEAR>
+  __device__ __forceinline__ void store(int i, int j, const Acc &v) const {
+    int lrow = this->lrow;
+    asm volatile("" : "+v"(lrow));
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if constexpr (NEAR) {
+        typedef uint32_t __attribute__((ext_vector_type(2))) u2v;
+        const uint32_t o = row(i, r) + lrow < m_rem ? off[j] : kOOB;
+        const int so = (int)(row(i, r) * ldc * SZ);
+        if constexpr (SZ == 8)
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2v, (E)v[r]), rs, o, so, 0);
+        else
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, (E)v[r]), rs, o, so, 0);
+      } else if (inside(i, j, r, lrow)) {
+        *at(i, j, r, lrow) = v[r];
+      }
+    }
+  }
+  __device__ __forceinline__ void load_all(Acc (&c)[TM][TN]) const {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) c[i][j] = near ? load<true>(i, j) : load<false>(i, j);
+  }
+  __device__ __forceinline__ void store_all(const Acc (&c)[TM][TN]) const {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        if (near)
+          store<true>(i, j, c[i][j]);
+        else
+          store<false>(i, j, c[i][j]);
+      }
+  }
+  // C = f(C, i, j, r)
+  template <class F>
+  __device__ __forceinline__ void update(const F &f) const {
+    if (near)
+      walk<true>(f);
+    else
+      walk<false>(f);
+  }
+  template <bool NEAR, class F>
+  __device__ __forceinline__ void walk(const F &f) const {
+    constexpr int N = TM * TN, D = N < kAhead ? N : kAhead;
+    Acc c[D];
+#pragma unroll
+    for (int q = 0; q < D; ++q) c[q] = load<NEAR>(q / TN, q % TN);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      Acc v;
+#pragma unroll
+      for (int r = 0; r < NR; ++r) v[r] = f(c[q % D][r], q / TN, q % TN, r);
+      if (q + D < N) c[q % D] = load<NEAR>((q + D) / TN, (q + D) % TN);
+      store<NEAR>(q / TN, q % TN, v);
+      __builtin_amdgcn_sched_barrier(0);  // no more of C in registers at once
+    }
+  }
+};
+
 // What differs between the element types. Both products keep a lane's operands at A[row l %
 // 16][k l / 16] and B[k l / 16][column l % 16] and add four k to each output as an FMA chain in
 // k order (checked on the device against 10^6 chains of each type, infinities, NaNs, signed
@@ -274,7 +395,6 @@ __device__ __forceinline__ void rm_tile(const Desc &d, int row0, int col0) {
     const long lda = uni(d.lda), ldb = uni(d.ldb), ldc = uni(d.ldc);
     const E *Ag = uni(d.A) + (long)row0 * lda;
     const E *Bg = uni(d.B) + col0;
-    global_t *Cg = (global_t *)(uni(d.C) + (long)row0 * ldc + col0);
     const int Kdim = uni(d.k);
     int w = Kdim;
     if constexpr (MP) {
@@ -433,15 +553,10 @@ __device__ __forceinline__ void rm_tile(const Desc &d, int row0, int col0) {
 #pragma unroll
       for (int j = 0; j < K::TN; ++j) {
         acc[i][j] = acc_t{};
-        if constexpr (CFIRST) {
-          const int cc = wn * K::WTN + j * 16 + li;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int rr = wm * K::WTM + i * 16 + X::row(r, g);
-            creg[i][j][r] = (rr < m_rem && cc < n_rem) ? Cg[(long)rr * ldc + cc] : E(0);
-          }
-        }
       }
+    const CTile<E, acc_t, K::TM, K::TN, 16, 4> ct(uni(d.C) + (long)(row0 + wm * K::WTM) * ldc + col0 + wn * K::WTN, ldc,
+                                                  m_rem - wm * K::WTM, n_rem - wn * K::WTN, lane);
+    if constexpr (CFIRST) ct.load_all(creg);
 
     auto read_ops = [&](int q, int kk, E(&x)[K::TM], E(&y)[K::TN]) {
 #pragma unroll
@@ -517,25 +632,16 @@ __device__ __forceinline__ void rm_tile(const Desc &d, int row0, int col0) {
         }
       }
     });
+    if constexpr (CFIRST) {
+      if constexpr (!MP)
 #pragma unroll
-    for (int i = 0; i < K::TM; ++i)
+        for (int i = 0; i < K::TM; ++i)
 #pragma unroll
-      for (int j = 0; j < K::TN; ++j) {
-        const int cc = wn * K::WTN + j * 16 + li;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int rr = wm * K::WTM + i * 16 + X::row(r, g);
-          if (rr < m_rem && cc < n_rem) {
-            global_t *pc = Cg + (long)rr * ldc + cc;
-            if constexpr (MP)
-              *pc = creg[i][j][r];
-            else if constexpr (CFIRST)
-              *pc = creg[i][j][r] + acc[i][j][r];
-            else
-              *pc = *pc + acc[i][j][r];
-          }
-        }
-      }
+          for (int j = 0; j < K::TN; ++j) creg[i][j] = creg[i][j] + acc[i][j];
+      ct.store_all(creg);
+    } else {
+      ct.update([&](E c, int i, int j, int r) { return c + acc[i][j][r]; });
+    }
   }
 }
 
