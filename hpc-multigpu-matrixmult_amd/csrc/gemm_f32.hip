@@ -225,15 +225,18 @@ __device__ __forceinline__ uint32_t bf16_rne(float x) {
 }
 __device__ __forceinline__ float bf16_val(uint32_t h) { return __uint_as_float(h << 16); }
 
+//
+// For products too small for the slice planes of gemm_bf3.hip. waves_per_eu(2) keeps the
+// accumulators where the MFMAs take them.
 template <int BM, int BN, int VEC>
-__global__ __launch_bounds__(256) void f32x3_gemm_kernel(F32Batch batch) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f32x3_gemm_kernel(F32Batch batch) {
   constexpr int BK = 32;
   constexpr int KP = BK + 8;  // bf16 per LDS row (80 bytes: 16-byte aligned, staggered banks)
   constexpr int WTM = BM / 2, WTN = BN / 2;
   constexpr int TM = WTM / 32, TN = WTN / 32;
   constexpr int AE = BM * BK / 256;  // A floats per thread
   constexpr int BE = BN * BK / 256;  // B floats per thread
-  static_assert(AE == 16 && BE == 16, "thread mapping assumes 128 x 128 tiles");
+  static_assert(BM == BN && AE % 8 == 0 && TM >= 1, "thread mapping");
   __shared__ __attribute__((aligned(16))) unsigned short lds[3 * BM * KP + 3 * BN * KP];
   unsigned short *Al = lds;
   unsigned short *Bl = lds + 3 * BM * KP;
@@ -244,9 +247,9 @@ __global__ __launch_bounds__(256) void f32x3_gemm_kernel(F32Batch batch) {
   const int wm = wave >> 1, wn = wave & 1;
   const int G = gridDim.x, bid = blockIdx.x;
   const int slot = uni((G % 8) == 0 ? (bid % 8) * (G / 8) + bid / 8 : bid);
-  // A: thread -> row tid / 2, k offset (tid % 2) * 16; B: column tid % 128, k half tid / 128
-  const int a_row = tid >> 1, a_k = (tid & 1) * 16;
-  const int b_col = tid & 127, b_k = (tid >> 7) * 16;
+  // AE consecutive k of one row of A, BE of one column of B per thread
+  const int a_row = tid / (BK / AE), a_k = tid % (BK / AE) * AE;
+  const int b_col = tid % BN, b_k = tid / BN * BE;
 
   for (int round = 0;; ++round) {
     const int t = round * G + slot;
@@ -268,12 +271,12 @@ __global__ __launch_bounds__(256) void f32x3_gemm_kernel(F32Batch batch) {
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] = f16v{};
 
-    float ra[16], rb[16];
+    float ra[AE], rb[BE];
     auto load = [&](int kb) {
       const int krem = d.k - kb;
       if constexpr (VEC == 4) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < AE / 4; ++q) {
           const int kc = a_k + 4 * q;
           const uint32_t off = (a_row < m_rem && kc < krem) ? (uint32_t)(((long)a_row * lda + kb + kc) * 4) : kOOB;
           const f4v v = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(rA, off, 0, 0));
@@ -282,7 +285,7 @@ __global__ __launch_bounds__(256) void f32x3_gemm_kernel(F32Batch batch) {
         }
       } else {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
+        for (int e = 0; e < AE; ++e) {
           const int kc = a_k + e;
           const uint32_t off = (a_row < m_rem && kc < krem) ? (uint32_t)(((long)a_row * lda + kb + kc) * 4) : kOOB;
           ra[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rA, off, 0, 0));
@@ -290,17 +293,17 @@ __global__ __launch_bounds__(256) void f32x3_gemm_kernel(F32Batch batch) {
       }
       const rsrc_t rB = make_rsrc(Bg + (long)kb * ldb, (long)krem * ldb * 4);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
+      for (int e = 0; e < BE; ++e) {
         const int kr = b_k + e;
         const uint32_t off = (kr < krem && b_col < n_rem) ? (uint32_t)(((long)kr * ldb + b_col) * 4) : kOOB;
         rb[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rB, off, 0, 0));
       }
     };
-    // split 16 consecutive-k values into three 16-element BF16 runs at dst + plane * pstride
+    // split AE consecutive-k values into three BF16 runs at dst + plane * pstride
     auto split_store = [&](const float *x, unsigned short *dst, int pstride) {
-      us8v h[2], m[2], l[2];
+      us8v h[AE / 8], m[AE / 8], l[AE / 8];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
+      for (int e = 0; e < AE; ++e) {
         const uint32_t hb = bf16_rne(x[e]);
         const float r1 = x[e] - bf16_val(hb);
         const uint32_t mb = bf16_rne(r1);
@@ -310,7 +313,7 @@ __global__ __launch_bounds__(256) void f32x3_gemm_kernel(F32Batch batch) {
         l[e >> 3][e & 7] = (unsigned short)bf16_rne(r2);
       }
 #pragma unroll
-      for (int hlf = 0; hlf < 2; ++hlf) {
+      for (int hlf = 0; hlf < AE / 8; ++hlf) {
         *(us8v *)(dst + 8 * hlf) = h[hlf];
         *(us8v *)(dst + pstride + 8 * hlf) = m[hlf];
         *(us8v *)(dst + 2 * pstride + 8 * hlf) = l[hlf];
@@ -544,27 +547,31 @@ bool phpc_f32_vec4_ok(const F32Desc *descs, int ndesc) {
   return true;
 }
 
-// FP32-accurate 3 x BF16 kernel: 128 x 128 tiles (plan with config 2's tile size).
-int phpc_f32x3_launch(const F32Desc *descs_dev, const F32Desc *descs_host, int ndesc, int total_tiles, bool vec4,
-                      int grid, hipStream_t stream) {
+// FP32-accurate 3 x BF16 kernel on the tiles of configuration 0 (64 x 64) or 2 (128 x 128).
+int phpc_f32x3_launch(const F32Desc *descs_dev, const F32Desc *descs_host, int ndesc, int total_tiles, int config,
+                      bool vec4, int grid, hipStream_t stream) {
   if (ndesc <= 0 || total_tiles <= 0) return PHPC_OK;
   for (int i = 0; i < ndesc; ++i) {
     const F32Desc &d = descs_host[i];
     if (128L * d.lda * 4 >= 0x7fffffffL || 32L * d.ldb * 4 >= 0x7fffffffL)
       return phpc_set_error(PHPC_ERR_ARG, "leading dimension too large");
   }
+  static void (*const kernels[2][2])(F32Batch) = {{f32x3_gemm_kernel<64, 64, 1>, f32x3_gemm_kernel<64, 64, 4>},
+                                                  {f32x3_gemm_kernel<128, 128, 1>, f32x3_gemm_kernel<128, 128, 4>}};
+  void (*fn)(F32Batch) = kernels[config == 2][vec4];
   int occ;
   {
-    static int occ_cache[2] = {0, 0};
+    static int occ_cache[2][2] = {};
     std::lock_guard<std::mutex> lk(g_mu);
-    const void *fn = vec4 ? reinterpret_cast<const void *>(f32x3_gemm_kernel<128, 128, 4>)
-                          : reinterpret_cast<const void *>(f32x3_gemm_kernel<128, 128, 1>);
-    if (occ_cache[vec4 ? 1 : 0] == 0) {
+    int &cached = occ_cache[config == 2][vec4];
+    if (cached == 0) {
       int n = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, 256, 0) != hipSuccess || n < 1) n = 1;
-      occ_cache[vec4 ? 1 : 0] = n;
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(fn), 256, 0) != hipSuccess ||
+          n < 1)
+        n = 1;
+      cached = n;
     }
-    occ = occ_cache[vec4 ? 1 : 0];
+    occ = cached;
   }
   F32Batch b{};
   b.descs = descs_dev;
@@ -574,10 +581,7 @@ int phpc_f32x3_launch(const F32Desc *descs_dev, const F32Desc *descs_host, int n
   int G = grid > 0 ? grid : occ * phpc_device().cus;
   if (G > total_tiles) G = total_tiles;
   if (G < 1) G = 1;
-  if (vec4)
-    hipLaunchKernelGGL((f32x3_gemm_kernel<128, 128, 4>), dim3(G), dim3(256), 0, stream, b);
-  else
-    hipLaunchKernelGGL((f32x3_gemm_kernel<128, 128, 1>), dim3(G), dim3(256), 0, stream, b);
+  hipLaunchKernelGGL(fn, dim3(G), dim3(256), 0, stream, b);
   PHPC_HIP(hipGetLastError());
   return PHPC_OK;
 }
@@ -627,19 +631,37 @@ extern "C" int phpc_sgemm_device(const float *dA, long lda, const float *dB, lon
   d.n = n;
   d.k = k;
   const bool vec4 = phpc_f32_vec4_ok(&d, 1);
-  int rc;
-  if (method == PHPC_SGEMM_BF16X3 && (long)m * n >= 2048L * 2048 && k >= 256) {
-    // large products: slice planes cut once, then the three slice levels on the
-    // direct-to-LDS pipeline
+  int rc = PHPC_OK;
+  bool planes = false;
+  const bool large = (long)m * n >= 2048L * 2048 && k >= 256;
+  if (method == PHPC_SGEMM_BF16X3) {
+    // Slice planes from one 64x64 tile per CU on: 1000^3 29 us against 40 on the in-register
+    // kernel, 1500^3 57 against 88; at 512^3, 18 against 21, the one launch that needs no shared
+    // workspace lets products on several streams run side by side. A stream being captured takes
+    // the workspace (which may grow, and waits for its last user) only where it always did.
+    planes = large;
+    if (!large && (long)((m + 63) / 64) * ((n + 63) / 64) >= phpc_device().cus && k >= 128 && phpc_bf3_fits(k)) {
+      hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+      const hipError_t e = hipStreamIsCapturing((hipStream_t)stream, &st);
+      if (e != hipSuccess) (void)hipGetLastError();
+      planes = e == hipSuccess && st == hipStreamCaptureStatusNone;
+    }
+  }
+  if (planes) {
+    // slice planes cut once, then multiplied on the direct-to-LDS pipeline
     static SharedWorkspace ws;
     std::lock_guard<std::mutex> lk(ws.mu);
     ws.after_previous((hipStream_t)stream);
     rc = phpc_sgemm_bf16x3_planes(dA, lda, dB, ldb, dC, ldc, m, k, n, (hipStream_t)stream, &ws.ws);
     ws.mark_used((hipStream_t)stream);
-  } else if (method == PHPC_SGEMM_BF16X3) {
-    const int tiles = phpc_f32_plan_tiles(&d, 1, 2);
-    rc = phpc_f32x3_launch(nullptr, &d, 1, tiles, vec4, 0, (hipStream_t)stream);
-  } else {
+    planes = large || rc != PHPC_ERR_MEM;
+    if (!planes) (void)hipGetLastError();  // the allocation's, before the launch below asks for its own
+  }
+  if (method == PHPC_SGEMM_BF16X3 && !planes) {
+    const int cfg = (long)((m + 127) / 128) * ((n + 127) / 128) >= phpc_device().cus ? 2 : 0;
+    const int tiles = phpc_f32_plan_tiles(&d, 1, cfg);
+    rc = phpc_f32x3_launch(nullptr, &d, 1, tiles, cfg, vec4, 0, (hipStream_t)stream);
+  } else if (method != PHPC_SGEMM_BF16X3) {
     if (g_f32_direct && phpc_f32_direct_ok(&d, 1)) {
       F32Work w;
       rc = phpc_f32_prepare(&d, 1, &w);

@@ -722,18 +722,24 @@ long rm_tiles(const Desc &d, int bm, int bn) {
   return (long)((d.m + bm - 1) / bm) * ((d.n + bn - 1) / bn);
 }
 
+// elements of B from one column to the next
+inline long rm_col_step(const GemmDesc &) { return 1; }
+inline long rm_col_step(const F32Desc &) { return 1; }
+inline long rm_col_step(const Bf3Desc &d) { return d.ldb; }
+
 // Split `live` so that its bm x bn head tiles fill whole rounds of the CUs and the rest, moved
 // to `tail`, runs on smaller tiles: a last round of head tiles that is nearly empty costs as
 // much as a full one (FP64 1777 x 1999 x 1235: 560 tiles of 64x64 on 256 CUs take three
 // rounds, 181 us; 500 of them and the rest as 32x32 take 2.25, 138 us). Every output's
 // arithmetic is its own, so where the line runs does not change a result. The cut takes rows
-// or columns of tiles, whichever step is finer, off the last GEMMs.
+// or columns of tiles, whichever step is finer, off the last GEMMs; a last round that is more
+// than `most` fifths full stays.
 template <class Desc>
-void rm_split_tail(std::vector<Desc> &live, int bm, int bn, long cus, std::vector<Desc> &tail) {
+void rm_split_tail(std::vector<Desc> &live, int bm, int bn, long cus, std::vector<Desc> &tail, int most = 4) {
   long total = 0;
   for (const Desc &d : live) total += rm_tiles(d, bm, bn);
   const long rounds = total / cus, rest = total % cus;
-  if (rounds == 0 || rest == 0 || 5 * rest > 4 * cus) return;
+  if (rounds == 0 || rest == 0 || 5 * rest > most * cus) return;
   long excess = rest;
   for (int i = (int)live.size() - 1; i >= 0 && excess > 0; --i) {
     Desc &d = live[i];
@@ -748,7 +754,7 @@ void rm_split_tail(std::vector<Desc> &live, int bm, int bn, long cus, std::vecto
       excess -= cut * tn;
     } else {
       const long cut = std::min(tn, (excess + tm - 1) / tm), keep = (tn - cut) * bn;
-      t.B += keep;
+      t.B += keep * rm_col_step(t);
       t.C += keep;
       t.n -= (int)keep;
       d.n = (int)keep;

@@ -19,6 +19,7 @@ struct phpc_plan {
   size_t descs_cap = 0;
   int config = 0;
   bool vec = false;
+  int x3_tile = 2;  // 3 x BF16 on the in-register kernel: its tiles (0: 64x64, 2: 128x128)
   int total_tiles = 0;
   int grid = 0;
   double tuned_ms = 0.0;
@@ -70,12 +71,18 @@ int plan_upload(phpc_plan *p, int id, hipStream_t s) {
     src = p->w32.list.data();
   } else if (p->dtype == PHPC_F32X3 && id >= kF32X3PlanesConfig) {
     if (int rc = p->planes.build(p->d32.data(), p->count, id - kF32X3PlanesConfig)) return rc;
-    p->total_tiles = p->planes.total_tiles;
+    p->total_tiles = p->planes.work.total;
     p->config = id;
     return PHPC_OK;
   } else {
-    // the in-register 3 x BF16 kernel has one tile shape, 128 x 128 (config 2's)
+    // the in-register 3 x BF16 kernel takes 128x128 tiles (config 2's) from one a CU on, else
+    // 64x64 (config 0's): 512^3 21 us against 47
     p->total_tiles = phpc_f32_plan_tiles(p->d32.data(), p->count, p->dtype == PHPC_F32X3 ? 2 : id);
+    p->x3_tile = 2;
+    if (p->dtype == PHPC_F32X3 && p->total_tiles < phpc_device().cus) {
+      p->x3_tile = 0;
+      p->total_tiles = phpc_f32_plan_tiles(p->d32.data(), p->count, 0);
+    }
     p->vec = phpc_f32_vec4_ok(p->d32.data(), p->count);
     bytes = sizeof(F32Desc) * p->count;
     src = p->d32.data();
@@ -106,7 +113,7 @@ int launch(phpc_plan *p, hipStream_t s) {
     return phpc_f32_launch_direct(p->w32, p->descs_dev, p->grid, s);
   if (p->dtype == PHPC_F32X3 && p->config >= kF32X3PlanesConfig) return p->planes.run(s, p->grid);
   if (p->dtype == PHPC_F32X3)
-    return phpc_f32x3_launch((const F32Desc *)p->descs_dev, p->d32.data(), p->count, p->total_tiles, p->vec, p->grid,
+    return phpc_f32x3_launch((const F32Desc *)p->descs_dev, p->d32.data(), p->count, p->total_tiles, p->x3_tile, p->vec, p->grid,
                              s);
   return phpc_f32_launch((const F32Desc *)p->descs_dev, p->d32.data(), p->count, p->total_tiles, p->config, p->vec,
                          p->grid, s);

@@ -34,7 +34,6 @@ typedef int i4v __attribute__((ext_vector_type(4)));
 typedef int i16v __attribute__((ext_vector_type(16)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef float f4v __attribute__((ext_vector_type(4)));
-typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 typedef int i8v __attribute__((ext_vector_type(8)));
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 typedef __attribute__((address_space(3))) void lds_void;
@@ -355,14 +354,6 @@ struct LevelArgs {
   int mod_m;  // 0: level mode (FP64 epilogue above)
   int8_t *res;
   long ldres;
-  // BF16 mode (operands are BF16 slices): C32[i,j] += the FP32 sum
-  float *C32;
-  long ldc32;
-  // BF16 mode: the k range may be up to three segments of one sum. Segment s starts at
-  // byte seg[s] of the kl range (seg[0] = 0; seg1 = 0: one segment) and reads A from
-  // row byte (k - seg[s]) and B from row byte (k - seg[s]) + segb[s].
-  int seg1, seg2;
-  int segb1, segb2;
 };
 
 // v mod m in the symmetric range for |v| < 2^31 and a wave-uniform m: m = 256 gives
@@ -415,24 +406,19 @@ __device__ __forceinline__ int i8_swz(int r) {
   return (r * CPR / SD) & (CPR - 1);
 }
 
-// BF = false: int8 operands, v_mfma_i32_32x32x32_i8, int32 sums (level or residue
-// epilogue). BF = true: BF16 operands (8 per 16-byte chunk), v_mfma_f32_32x32x16_bf16,
-// FP32 sums added to C32. F8 = true: FP8-E4M3 operands (16 per chunk); the chunks of two
-// k steps make one lane's 32 bytes of v_mfma_scale_f32_32x32x64_f8f6f4 at unit scales
-// (A and B take the same bytes, so the sum runs over the same 64 k), FP32 sums that stay
-// exact integers below 2^24, FP64 level epilogue. The byte layout and the pipeline are
-// the same.
+// F8 = false: int8 operands, int32 sums (level or residue epilogue). F8 = true: FP8-E4M3
+// operands (16 per chunk); the chunks of two k steps make one lane's 32 bytes of
+// v_mfma_scale_f32_32x32x64_f8f6f4 at unit scales (A and B take the same bytes, so the sum
+// runs over the same 64 k), FP32 sums that stay exact integers below 2^24, FP64 level epilogue.
+// The byte layout and the pipeline are the same.
 // The operands of one level product as the tile code reads them (wave-uniform values):
-// read once per product by the plain walk, once per tile by the grouped one.
+// read once per product.
 struct LevelOps {
   const int8_t *A8, *B8;  // at the product's k offset
   long lda8, ldb8;
   int m, n, nslab;
-  int sg1, sg2, sb1, sb2;  // BF16 segments
-  float *C32;              // BF16 epilogue
-  long ldc32;
 };
-template <int BK, bool BF>
+template <int BK>
 __device__ __forceinline__ LevelOps level_ops(const LevelArgs &args) {
   LevelOps o;
   o.m = uni(args.m);
@@ -442,21 +428,14 @@ __device__ __forceinline__ LevelOps level_ops(const LevelArgs &args) {
   o.ldb8 = uni(args.ldb8);
   o.A8 = uni(args.A8) + uni(args.a0);
   o.B8 = uni(args.B8) + uni(args.b0);
-  o.sg1 = BF ? uni(args.seg1) : 0;
-  o.sg2 = BF ? uni(args.seg2) : 0;
-  o.sb1 = BF ? uni(args.segb1) : 0;
-  o.sb2 = BF ? uni(args.segb2) : 0;
-  o.C32 = BF ? uni(args.C32) : nullptr;
-  o.ldc32 = BF ? uni(args.ldc32) : 0;
   return o;
 }
 
 // One BM x BN output tile at (row0, col0) of the product ops describes; args carries the
 // int8 and FP8 epilogues' fields (the tile walk is the caller's). MI: the MFMA block,
-// 32 x 32 (32 bytes of k per int8 product, 16 per BF16 one) or 16 x 16 (v_mfma_i32_16x16x64_i8
-// and v_mfma_f32_16x16x32_bf16: 64 bytes of k); a lane's 16-byte operand is row l % MI,
+// 32 x 32 (32 bytes of k per product) or 16 x 16 (v_mfma_i32_16x16x64_i8, 64); a lane's 16-byte operand is row l % MI,
 // chunk (64 / MI) kk + l / MI of the k step. Not for FP8 at 16.
-template <int BM, int BN, int WM, int WN, int BK_, int STAGES, int SD, bool BF, bool F8, int MI = 32>
+template <int BM, int BN, int WM, int WN, int BK_, int STAGES, int SD, bool F8, int MI = 32>
 __device__ __forceinline__ void level_tile(const LevelArgs &args, const LevelOps &ops, int row0, int col0) {
   using K = I8Cfg<BM, BN, WM, WN, BK_, STAGES>;
   static_assert(MI == 32 || (MI == 16 && !F8), "MFMA block");
@@ -474,8 +453,6 @@ __device__ __forceinline__ void level_tile(const LevelArgs &args, const LevelOps
   const int8_t *A8 = ops.A8;
   const int8_t *B8 = ops.B8;
   const int nslab = ops.nslab;
-  const int sg1 = ops.sg1, sg2 = ops.sg2;
-  const int sb1 = ops.sb1, sb2 = ops.sb2;
 
   // LDS operand offsets per k step: lane reads 16 bytes of row (l % 32), chunk
   // 2*kk + l/32, at its swizzled slot. The rows a lane reads are l % 32 plus multiples of
@@ -514,27 +491,8 @@ __device__ __forceinline__ void level_tile(const LevelArgs &args, const LevelOps
                    (((lane % K::CPR) ^ i8_swz<K::CPR, SD>(wave * K::ROWS_PER_BLOCK + lrow)) << 4));
     const uint32_t gstep_a = (uint32_t)(RSTEP * lda8), gstep_b = (uint32_t)(RSTEP * ldb8);
 
-    // k byte offsets of slab sidx in A's and B's rows
-    auto slab_k = [&](int sidx, int &ka, int &kbb) {
-      const int kb = sidx * K::BK;
-      ka = kb;
-      kbb = kb;
-      if constexpr (BF) {
-        // segments start on slab boundaries, so a slab lies in one segment
-        if (sg1 > 0 && kb >= sg1) {
-          if (sg2 > 0 && kb >= sg2) {
-            ka = kb - sg2;
-            kbb = ka + sb2;
-          } else {
-            ka = kb - sg1;
-            kbb = ka + sb1;
-          }
-        }
-      }
-    };
     auto issue = [&](int sidx) {
-      int ka, kbb;
-      slab_k(sidx, ka, kbb);
+      const int kb = sidx * K::BK;
       char *stage = smem + (sidx % STAGES) * K::STAGE_BYTES;
 #pragma unroll
       for (int u = 0; u < K::PER; ++u) {
@@ -544,13 +502,12 @@ __device__ __forceinline__ void level_tile(const LevelArgs &args, const LevelOps
         // rides in soffset
         const uint32_t go = isA ? ga0 + (uint32_t)u * gstep_a : gb0 + (uint32_t)(u - PA) * gstep_b;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(isA ? rA : rB, (lds_void *)(stage + blk * 1024), 16, go,
-                                                  isA ? ka : kbb, 0, 0);
+                                                  kb, 0, 0);
       }
     };
 
-    using acc32_t = typename std::conditional<BF || F8, f16v, i16v>::type;
-    using acc16_t = typename std::conditional<BF, f4v, i4v>::type;
-    using acc_t = typename std::conditional<MI == 32, acc32_t, acc16_t>::type;
+    using acc32_t = typename std::conditional<F8, f16v, i16v>::type;
+    using acc_t = typename std::conditional<MI == 32, acc32_t, i4v>::type;
     acc_t acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -615,13 +572,7 @@ __device__ __forceinline__ void level_tile(const LevelArgs &args, const LevelOps
           for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
-              if constexpr (BF && MI == 32)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8v, a[i]),
-                                                                   __builtin_bit_cast(bf8v, b[j]), acc[i][j], 0, 0, 0);
-              else if constexpr (BF)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8v, a[i]),
-                                                                   __builtin_bit_cast(bf8v, b[j]), acc[i][j], 0, 0, 0);
-              else if constexpr (MI == 32)
+              if constexpr (MI == 32)
                 acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[i], b[j], acc[i][j], 0, 0, 0);
               else
                 acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i], b[j], acc[i][j], 0, 0, 0);
@@ -635,25 +586,6 @@ __device__ __forceinline__ void level_tile(const LevelArgs &args, const LevelOps
     auto erow = [&](int i, int r) {
       return MI == 32 ? i * 32 + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4) : i * 16 + 4 * (lane >> 4) + r;
     };
-    if constexpr (BF) {
-      float __attribute__((address_space(1))) *Cg = (float __attribute__((address_space(1))) *)ops.C32;
-      const long ldc32 = ops.ldc32;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int col = col0 + wn * K::WTN + j * MI + (lane & (MI - 1));
-          if (col >= n) continue;
-#pragma unroll
-          for (int r = 0; r < NR; ++r) {
-            const int row = row0 + wm * K::WTM + erow(i, r);
-            if (row >= m) continue;
-            auto *pc = Cg + (long)row * ldc32 + col;
-            *pc = *pc + acc[i][j][r];
-          }
-        }
-      return;
-    }
     const int mod_m = uni(args.mod_m);
     if (mod_m > 0) {
       const int firstr = uni(args.first);
@@ -710,10 +642,9 @@ __device__ __forceinline__ void level_tile(const LevelArgs &args, const LevelOps
   }
 }
 
-template <int BM, int BN, int WM, int WN, int BK_, int STAGES, int SD = 16, bool BF = false, bool F8 = false,
-          int MI = 32>
+template <int BM, int BN, int WM, int WN, int BK_, int STAGES, int SD = 16, bool F8 = false, int MI = 32>
 __device__ __forceinline__ void i8_level_body(const LevelArgs &args) {
-  const LevelOps ops = level_ops<BK_, BF>(args);
+  const LevelOps ops = level_ops<BK_>(args);
   const int m = ops.m, n = ops.n;
   const int tiles_n = (n + BN - 1) / BN;
   const int tiles_m = (m + BM - 1) / BM;
@@ -732,7 +663,7 @@ __device__ __forceinline__ void i8_level_body(const LevelArgs &args) {
     const int in_grp = t - grp * gm * tiles_n;
     const int row0 = uni((first_m + in_grp % gsz) * BM);
     const int col0 = uni((in_grp / gsz) * BN);
-    level_tile<BM, BN, WM, WN, BK_, STAGES, SD, BF, F8, MI>(args, ops, row0, col0);
+    level_tile<BM, BN, WM, WN, BK_, STAGES, SD, F8, MI>(args, ops, row0, col0);
   }
 }
 
@@ -768,35 +699,21 @@ __global__ __launch_bounds__(1024) void i8_level_256x128_w16_k128_s3(LevelArgs a
 }
 // the default tile on 16 x 16 MFMA blocks (v_mfma_i32_16x16x64_i8)
 __global__ __launch_bounds__(1024) void i8_level_256x256_w16_k128_mi16(LevelArgs a) {
-  i8_level_body<256, 256, 4, 4, 128, 2, 16, false, false, 16>(a);
+  i8_level_body<256, 256, 4, 4, 128, 2, 16, false, 16>(a);
 }
 __global__ __launch_bounds__(512) void i8_level_256x256_w8_k128_mi16(LevelArgs a) {
-  i8_level_body<256, 256, 2, 4, 128, 2, 16, false, false, 16>(a);
+  i8_level_body<256, 256, 2, 4, 128, 2, 16, false, 16>(a);
 }
 __global__ __launch_bounds__(256) void i8_level_128x128_w4_mi16(LevelArgs a) {
-  i8_level_body<128, 128, 2, 2, 64, 4, 16, false, false, 16>(a);
+  i8_level_body<128, 128, 2, 2, 64, 4, 16, false, 16>(a);
 }
 // FP8-E4M3 digit slices on the same pipeline (FP64-accurate, scheme I with 4-bit digits)
 __global__ __launch_bounds__(1024) void f8_level_256x256_w16_k128(LevelArgs a) {
-  i8_level_body<256, 256, 4, 4, 128, 2, 16, false, true>(a);
+  i8_level_body<256, 256, 4, 4, 128, 2, 16, true>(a);
 }
 __global__ __launch_bounds__(256) void f8_level_128x128_w4(LevelArgs a) {
-  i8_level_body<128, 128, 2, 2, 64, 4, 16, false, true>(a);
+  i8_level_body<128, 128, 2, 2, 64, 4, 16, true>(a);
 }
-// BF16 slices on the same pipeline (FP32-accurate 3 x BF16 GEMM). Every BF16 level kernel,
-// single-product and grouped, uses the same MFMA block, so that they sum each output in the
-// same order.
-constexpr int kBfMI = 16;
-__global__ __launch_bounds__(512) void bf16_level_256x256_w8_k128(LevelArgs a) {
-  i8_level_body<256, 256, 2, 4, 128, 2, 16, true, false, kBfMI>(a);
-}
-__global__ __launch_bounds__(1024) void bf16_level_256x256_w16_k128(LevelArgs a) {
-  i8_level_body<256, 256, 4, 4, 128, 2, 16, true, false, kBfMI>(a);
-}
-__global__ __launch_bounds__(256) void bf16_level_128x128_w4(LevelArgs a) {
-  i8_level_body<128, 128, 2, 2, 64, 4, 16, true, false, kBfMI>(a);
-}
-
 typedef void (*LevelFn)(LevelArgs);
 struct I8Config {
   int bm, bn, bk, threads;
@@ -826,15 +743,6 @@ const I8Config kI8Configs[] = {
 constexpr int kNumI8 = sizeof(kI8Configs) / sizeof(kI8Configs[0]);
 int g_i8_big = 13;  // kI8Configs index for large problems
 
-// BF16-slice level kernels (FP32-accurate 3 x BF16 GEMM), kept apart from the int8
-// table so that phpc_split_set_config can only pick int8 kernels
-const I8Config kBfConfigs[] = {
-    I8CFG(256, 256, 4, 4, 128, 2, bf16_level_256x256_w16_k128),  // 0: large problems, 16 waves
-    I8CFG(128, 128, 2, 2, 64, 4, bf16_level_128x128_w4),         // 1: small problems
-    I8CFG(256, 256, 2, 4, 128, 2, bf16_level_256x256_w8_k128),   // 2: 8 waves
-};
-constexpr int kNumBf = sizeof(kBfConfigs) / sizeof(kBfConfigs[0]);
-
 // FP8-digit level kernels (scheme I with FP8-E4M3 slices)
 const I8Config kF8Configs[] = {
     I8CFG(256, 256, 4, 4, 128, 2, f8_level_256x256_w16_k128),  // 0: large problems, 16 waves
@@ -845,7 +753,6 @@ constexpr int kNumF8 = sizeof(kF8Configs) / sizeof(kF8Configs[0]);
 std::mutex g_mu;
 bool g_ready = false;
 int g_occ[kNumI8];
-int g_occ_bf[kNumBf];
 int g_occ_f8[kNumF8];
 
 int occupancy_of(const I8Config &c) {
@@ -859,7 +766,6 @@ int occupancy_of(const I8Config &c) {
 void init_locked() {
   if (g_ready) return;
   for (int c = 0; c < kNumI8; ++c) g_occ[c] = occupancy_of(kI8Configs[c]);
-  for (int c = 0; c < kNumBf; ++c) g_occ_bf[c] = occupancy_of(kBfConfigs[c]);
   for (int c = 0; c < kNumF8; ++c) g_occ_f8[c] = occupancy_of(kF8Configs[c]);
   g_ready = true;
 }
@@ -867,8 +773,7 @@ void init_locked() {
 int launch_with(const I8Config &c, int occ, const LevelArgs &a, hipStream_t s) {
   // the kernels walk k in whole slabs of c.bk bytes: a range that is not a whole number
   // of slabs, or starts inside one, would lose its tail
-  if (a.kl <= 0 || a.kl % c.bk != 0 || a.a0 % 16 != 0 || a.b0 % 16 != 0 ||
-      (a.seg1 | a.seg2 | a.segb1 | a.segb2) % c.bk != 0)
+  if (a.kl <= 0 || a.kl % c.bk != 0 || a.a0 % 16 != 0 || a.b0 % 16 != 0)
     return phpc_set_error(PHPC_ERR_ARG, "level range of %d bytes is not whole %d-byte slabs", a.kl, c.bk);
   // buffer offsets are 32-bit: a tile's rows of A and B must span less than 2 GiB
   if ((long)c.bm * a.lda8 >= 0x7fffffffL || (long)c.bn * a.ldb8 >= 0x7fffffffL)
@@ -903,272 +808,6 @@ int launch_f8_level(const LevelArgs &a, int cfg, hipStream_t s) {
     occ = g_occ_f8[cfg];
   }
   return launch_with(kF8Configs[cfg], occ, a, s);
-}
-
-int launch_bf_level(const LevelArgs &a, int cfg, hipStream_t s) {
-  int occ;
-  {
-    std::lock_guard<std::mutex> lk(g_mu);
-    init_locked();
-    occ = g_occ_bf[cfg];
-  }
-  return launch_with(kBfConfigs[cfg], occ, a, s);
-}
-
-// ---------------------------------------------------------------------------
-// FP32 -> three BF16 slice planes for the level kernels: x = hi + mid + lo exactly,
-// each rounded to nearest BF16 (the same cut as the FP32-accurate grouped kernel)
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t bf16_rne(float x) {
-  const uint32_t u = __float_as_uint(x);
-  return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
-}
-__device__ __forceinline__ void split3(float x, uint32_t &h, uint32_t &mi, uint32_t &lo) {
-  h = bf16_rne(x);
-  const float r1 = x - __uint_as_float(h << 16);
-  mi = bf16_rne(r1);
-  const float r2 = r1 - __uint_as_float(mi << 16);
-  lo = bf16_rne(r2);
-}
-typedef unsigned int u4v __attribute__((ext_vector_type(4)));
-
-// A3 row i = [hi | mid | lo], each plane kp BF16 wide (zero beyond k); 8 k per thread
-__global__ __launch_bounds__(256) void bf16x3_rows_kernel(const float *__restrict__ A, long lda, int m, int k,
-                                                          long kp, uint16_t *__restrict__ A3) {
-  const int i = blockIdx.y;
-  const float *row = A + (long)i * lda;
-  uint16_t *out = A3 + (long)i * 3 * kp;
-  for (long c = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 8; c < kp; c += (long)gridDim.x * blockDim.x * 8) {
-    uint32_t h[8], mi[8], lo[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) split3(load_or_zero(row, c + e, c + e < k), h[e], mi[e], lo[e]);
-    u4v vh, vm, vl;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      vh[q] = h[2 * q] | (h[2 * q + 1] << 16);
-      vm[q] = mi[2 * q] | (mi[2 * q + 1] << 16);
-      vl[q] = lo[2 * q] | (lo[2 * q + 1] << 16);
-    }
-    *reinterpret_cast<u4v *>(out + c) = vh;
-    *reinterpret_cast<u4v *>(out + kp + c) = vm;
-    *reinterpret_cast<u4v *>(out + 2 * kp + c) = vl;
-  }
-}
-
-// B3 row j (column j of B) = [lo | mid | hi], through a 64 x 64 LDS transpose
-__global__ __launch_bounds__(256) void bf16x3_cols_kernel(const float *__restrict__ B, long ldb, int k, int n,
-                                                          long kp, uint16_t *__restrict__ B3) {
-  __shared__ float tile[64][65];
-  const int k0 = blockIdx.x * 64, j0 = blockIdx.y * 64;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  float v[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int kk = k0 + ty + 4 * i, jj = j0 + tx;
-    v[i] = load_or_zero(B, (long)kk * ldb + jj, kk < k && jj < n);
-  }
-#pragma unroll
-  for (int i = 0; i < 16; ++i) tile[ty + 4 * i][tx] = v[i];
-  __syncthreads();
-#pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const int item = threadIdx.x + it * 256;  // 64 columns x 8 groups of 8 k
-    const int c = item >> 3, kq = (item & 7) * 8;
-    const int jj = j0 + c;
-    if (jj >= n) continue;
-    uint32_t h[8], mi[8], lo[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) split3(tile[kq + e][c], h[e], mi[e], lo[e]);
-    u4v vh, vm, vl;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      vh[q] = h[2 * q] | (h[2 * q + 1] << 16);
-      vm[q] = mi[2 * q] | (mi[2 * q + 1] << 16);
-      vl[q] = lo[2 * q] | (lo[2 * q + 1] << 16);
-    }
-    uint16_t *out = B3 + (long)jj * 3 * kp + k0 + kq;
-    *reinterpret_cast<u4v *>(out) = vl;
-    *reinterpret_cast<u4v *>(out + kp) = vm;
-    *reinterpret_cast<u4v *>(out + 2 * kp) = vh;
-  }
-}
-
-// Every cut of a grouped 3 x BF16 plan in one launch: one workgroup per 64 plane rows x 64
-// k of a cut, its cut read from a per-workgroup table. Each thread cuts 8 consecutive k of
-// one plane row (two per thread) and writes 16 bytes per plane. A's rows are its plane
-// rows, so a thread reads its 8 k straight from the row (16-byte loads where rows are
-// aligned); B's tile passes through LDS as tile[plane row][k], read along B's rows
-// (coalesced). Every load of a thread is issued before the first wait. The cut is split3,
-// as in bf16x3_rows_kernel / bf16x3_cols_kernel.
-__global__ __launch_bounds__(256) void bf16x3_cut_kernel(const Bf3Cut *__restrict__ cuts,
-                                                         const int *__restrict__ block_cut) {
-  __shared__ float tile[64][65];
-  const int b = blockIdx.x;
-  const Bf3Cut c = cuts[block_cut[b]];
-  const int lb = b - c.block_start;
-  const int r0 = (lb / c.tiles_k) * 64;  // first plane row
-  const int k0 = (lb % c.tiles_k) * 64;
-  const int nrows = c.is_b ? c.cols : c.rows;  // plane rows
-  const int kk = c.is_b ? c.rows : c.cols;     // k
-  float x2[2][8];
-  if (c.is_b) {
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    float v[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      // B row k0 + r, columns r0 + tx: plane row tx, k r
-      const int r = ty + 4 * i;
-      const int sk = k0 + r, sj = r0 + tx;
-      v[i] = load_or_zero(c.src, (long)sk * c.ld + sj, sk < kk && sj < nrows);
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) tile[tx][ty + 4 * i] = v[i];
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-      const int item = threadIdx.x + it * 256;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x2[it][e] = tile[item >> 3][(item & 7) * 8 + e];
-    }
-  } else {
-    // both items' loads go out before the first wait
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-      const int item = threadIdx.x + it * 256;
-      const int pr = min(item >> 3, nrows - 1 - r0), kq = (item & 7) * 8;  // rows past the edge: unused
-      const long base = (long)(r0 + pr) * c.ld + k0 + kq;
-      const int krem = kk - (k0 + kq);
-      if (c.vec && krem >= 8) {
-        const float4 v0 = *reinterpret_cast<const float4 *>(c.src + base);
-        const float4 v1 = *reinterpret_cast<const float4 *>(c.src + base + 4);
-        x2[it][0] = v0.x, x2[it][1] = v0.y, x2[it][2] = v0.z, x2[it][3] = v0.w;
-        x2[it][4] = v1.x, x2[it][5] = v1.y, x2[it][6] = v1.z, x2[it][7] = v1.w;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x2[it][e] = load_or_zero(c.src, base + e, e < krem);
-      }
-    }
-  }
-#pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const int item = threadIdx.x + it * 256;  // 64 plane rows x 8 groups of 8 k
-    const int pr = item >> 3, kq = (item & 7) * 8;
-    if (r0 + pr >= nrows) continue;
-    const float *x = x2[it];
-    uint32_t h[8], mi[8], lo[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) split3(x[e], h[e], mi[e], lo[e]);
-    u4v vh, vm, vl;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      vh[q] = h[2 * q] | (h[2 * q + 1] << 16);
-      vm[q] = mi[2 * q] | (mi[2 * q + 1] << 16);
-      vl[q] = lo[2 * q] | (lo[2 * q + 1] << 16);
-    }
-    uint16_t *out = c.dst + (long)(r0 + pr) * 3 * c.kp + k0 + kq;
-    *reinterpret_cast<u4v *>(out) = c.is_b ? vl : vh;
-    *reinterpret_cast<u4v *>(out + c.kp) = vm;
-    *reinterpret_cast<u4v *>(out + 2 * c.kp) = c.is_b ? vh : vl;
-  }
-}
-
-// One grouped launch of the BF16 level kernel over a 3 x BF16 plan's flat tile list
-// (items in the plan's order, each item's tiles in groups of 8 tile-rows): the persistent
-// workgroups take tiles from XCD-contiguous slots, find the tile's item by binary search
-// on tile_start, and run the level tile on its planes: the three k segments of
-// phpc_sgemm_bf16x3_planes, so the same sum per output.
-struct Bf3Group {
-  const Bf3Item *items;
-  int count;
-  int total_tiles;
-};
-template <int BM, int BN, int WM, int WN, int BK_, int STAGES>
-__device__ __forceinline__ void bf16_group_body(const Bf3Group &g) {
-  const int G = gridDim.x;
-  const int bid = blockIdx.x;
-  const int slot = uni((G % 8) == 0 ? (bid % 8) * (G / 8) + bid / 8 : bid);
-  const int total = uni(g.total_tiles);
-  const int count = uni(g.count);
-  const Bf3Item *items = uni(g.items);
-  const LevelArgs none{};  // the BF16 epilogue reads ops only
-  for (int round = 0;; ++round) {
-    const int t = round * G + slot;
-    if (t >= total) break;
-    int lo = 0, hi = count - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (uni(items[mid].tile_start) <= t)
-        lo = mid;
-      else
-        hi = mid - 1;
-    }
-    const Bf3Item *it = items + lo;
-    const int kp2 = uni(it->kp2);
-    LevelOps o;
-    o.A8 = (const int8_t *)uni(it->A3);
-    o.B8 = (const int8_t *)uni(it->B3);
-    o.lda8 = 3L * kp2;
-    o.ldb8 = 3L * kp2;
-    o.m = uni(it->m);
-    o.n = uni(it->n);
-    o.nslab = 6 * kp2 / BK_;
-    o.sg1 = 3 * kp2;
-    o.sg2 = 5 * kp2;
-    o.sb1 = kp2;
-    o.sb2 = 2 * kp2;
-    o.C32 = uni(it->C);
-    o.ldc32 = uni(it->ldc);
-    const int lt = t - uni(it->tile_start);
-    const int tiles_m = uni(it->tiles_m), tiles_n = uni(it->tiles_n);
-    const int gm = 8;
-    const int grp = lt / (gm * tiles_n);
-    const int first_m = grp * gm;
-    const int gsz = min(tiles_m - first_m, gm);
-    const int in_grp = lt - grp * gm * tiles_n;
-    const int row0 = uni((first_m + in_grp % gsz) * BM);
-    const int col0 = uni((in_grp / gsz) * BN);
-    level_tile<BM, BN, WM, WN, BK_, STAGES, 16, true, false, kBfMI>(none, o, row0, col0);
-  }
-}
-__global__ __launch_bounds__(256) void bf16_group_128x128_w4(Bf3Group g) { bf16_group_body<128, 128, 2, 2, 64, 4>(g); }
-__global__ __launch_bounds__(512) void bf16_group_256x128_w8_k128(Bf3Group g) {
-  bf16_group_body<256, 128, 4, 2, 128, 2>(g);
-}
-__global__ __launch_bounds__(1024) void bf16_group_256x256_w16_k128(Bf3Group g) {
-  bf16_group_body<256, 256, 4, 4, 128, 2>(g);
-}
-
-struct Bf3GroupConfig {
-  int bm, bn, bk, threads;
-  size_t lds;
-  void (*fn)(Bf3Group);
-};
-#define BF3CFG(BM_, BN_, WM_, WN_, BK_, ST_, FN_) \
-  Bf3GroupConfig { BM_, BN_, BK_, WM_ *WN_ * 64, (size_t)(ST_)*I8Cfg<BM_, BN_, WM_, WN_, BK_, ST_>::STAGE_BYTES, FN_ }
-const Bf3GroupConfig kBf3Group[] = {
-    BF3CFG(128, 128, 2, 2, 64, 4, bf16_group_128x128_w4),         // 0: 4 waves, 64x64 wave tiles
-    BF3CFG(256, 128, 4, 2, 128, 2, bf16_group_256x128_w8_k128),   // 1: 8 waves, 64x64 wave tiles
-    BF3CFG(256, 256, 4, 4, 128, 2, bf16_group_256x256_w16_k128),  // 2: 16 waves, 64x64 wave tiles
-};
-constexpr int kNumBf3Group = sizeof(kBf3Group) / sizeof(kBf3Group[0]);
-int g_occ_bf3[kNumBf3Group];
-bool g_bf3_ready = false;
-
-int bf3_occupancy(int g) {
-  std::lock_guard<std::mutex> lk(g_mu);
-  if (!g_bf3_ready) {
-    for (int c = 0; c < kNumBf3Group; ++c) {
-      const void *fn = reinterpret_cast<const void *>(kBf3Group[c].fn);
-      (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBf3Group[c].lds);
-      int n = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, kBf3Group[c].threads, kBf3Group[c].lds) != hipSuccess ||
-          n < 1)
-        n = 1;
-      g_occ_bf3[c] = n;
-    }
-    g_bf3_ready = true;
-  }
-  return g_occ_bf3[g];
 }
 
 // Error estimate used to pick the slice count: the truncated terms of one product are
@@ -1881,187 +1520,6 @@ int phpc_dgemm_split_ws(const double *dA, long lda, const double *dB, long ldb, 
     info->int_bits = bits * s_use;
   }
   return phpc_set_error(PHPC_OK, nullptr);
-}
-
-// FP32-accurate GEMM from BF16 slice planes: C += A*B (FP32, row-major, device pointers).
-// A3 rows hold [hi | mid | lo] and B3 rows (columns of B) [lo | mid | hi], so the six
-// products with slice-index sum <= 2 form three contiguous k ranges, summed smallest first
-// into one FP32 accumulator by one launch (three k segments): A3[:, 0:3kp] . B3[:, 0:3kp]
-// = hi.lo + mid.mid + lo.hi, then A3[:, 0:2kp] . B3[:, kp:3kp] = hi.mid + mid.hi, then
-// A3[:, 0:kp] . B3[:, 2kp:3kp] = hi.hi; the sum is added to C once.
-int phpc_sgemm_bf16x3_planes(const float *dA, long lda, const float *dB, long ldb, float *dC, long ldc, int m, int k,
-                             int n, hipStream_t s, Workspace *ws) {
-  const long kp = ((long)k + 63) / 64 * 64;
-  if (3 * kp * 2 >= 0x7fffffffL / 256) return phpc_set_error(PHPC_ERR_ARG, "k = %d too large for the slice planes", k);
-  uint16_t *A3 = (uint16_t *)ws->get((size_t)m * 3 * kp * 2, 0, s);
-  uint16_t *B3 = (uint16_t *)ws->get((size_t)n * 3 * kp * 2, 1, s);
-  if (!A3 || !B3) return phpc_set_error(PHPC_ERR_MEM, "slice plane allocation failed");
-  {
-    const long per_row = (kp / 8 + 255) / 256;
-    hipLaunchKernelGGL(bf16x3_rows_kernel, dim3((unsigned)std::min<long>(per_row, 64), (unsigned)m), dim3(256), 0, s,
-                       dA, lda, m, k, kp, A3);
-    PHPC_HIP(hipGetLastError());
-    hipLaunchKernelGGL(bf16x3_cols_kernel, dim3((unsigned)(kp / 64), (unsigned)((n + 63) / 64)), dim3(256), 0, s, dB,
-                       ldb, k, n, kp, B3);
-    PHPC_HIP(hipGetLastError());
-  }
-  const long tiles256 = (long)((m + 255) / 256) * ((n + 255) / 256);
-  const int cfg = tiles256 >= (long)phpc_device().cus / 2 ? 0 : 1;
-  const int kp2 = (int)(kp * 2);  // bytes of one plane row
-  LevelArgs a{};
-  a.A8 = (const int8_t *)A3;
-  a.B8 = (const int8_t *)B3;
-  a.lda8 = 3L * kp2;
-  a.ldb8 = 3L * kp2;
-  a.m = m;
-  a.n = n;
-  a.kl = 6 * kp2;
-  a.seg1 = 3 * kp2;
-  a.seg2 = 5 * kp2;
-  a.segb1 = kp2;
-  a.segb2 = 2 * kp2;
-  a.C32 = dC;
-  a.ldc32 = ldc;
-  return launch_bf_level(a, cfg, s);
-}
-
-// ---------------------------------------------------------------------------
-// Grouped 3 x BF16 plans on slice planes (declared in phpc_internal.h)
-// ---------------------------------------------------------------------------
-int phpc_bf3_num_configs() { return kNumBf3Group; }
-
-namespace {
-size_t bf3_align(size_t b) { return (b + 255) / 256 * 256; }
-int g_f32x3_plan_cfg = -1;
-}  // namespace
-
-int phpc_f32x3_set_plan_config(int id) {
-  if (id != -1 && id != 2 && (id < kF32X3PlanesConfig || id >= kF32X3PlanesConfig + kNumBf3Group))
-    return phpc_set_error(PHPC_ERR_ARG, "3 x BF16 plan config %d out of range", id);
-  g_f32x3_plan_cfg = id;
-  return phpc_set_error(PHPC_OK, nullptr);
-}
-
-int phpc_f32x3_pick_plan_config(const F32Desc *descs, int ndesc) {
-  if (g_f32x3_plan_cfg >= 0) return g_f32x3_plan_cfg;
-  // slice planes on 256 x 256 tiles (the fastest tile on the 512-GEMM mix) once the items
-  // give every CU at least one such tile
-  long work = 0;
-  for (int i = 0; i < ndesc; ++i) work += (long)((descs[i].m + 255) / 256) * ((descs[i].n + 255) / 256);
-  return work >= (long)phpc_device().cus ? kF32X3PlanesConfig + 2 : 2;
-}
-
-int Bf3Planes::build(const F32Desc *descs, int ndesc, int gcfg) {
-  release();
-  cuts.clear();
-  off.clear();
-  block_cut.clear();
-  items.clear();
-  if (gcfg < 0 || gcfg >= kNumBf3Group) return phpc_set_error(PHPC_ERR_ARG, "slice-plane tile %d out of range", gcfg);
-  g = gcfg;
-  const Bf3GroupConfig &cf = kBf3Group[g];
-  blocks = 0;
-  total_tiles = 0;
-  ws_bytes = 0;
-  // one cut per distinct operand (an A or B shared by several items is cut once)
-  auto find_or_add = [&](const float *src, long ld, int rows, int cols, int is_b, long kp) {
-    for (size_t j = 0; j < cuts.size(); ++j) {
-      const Bf3Cut &c = cuts[j];
-      if (c.src == src && c.ld == ld && c.rows == rows && c.cols == cols && c.is_b == is_b) return (int)j;
-    }
-    Bf3Cut c{};
-    c.src = src;
-    c.ld = ld;
-    c.rows = rows;
-    c.cols = cols;
-    c.kp = kp;
-    c.is_b = is_b;
-    c.vec = !is_b && (reinterpret_cast<uintptr_t>(src) & 15) == 0 && ld % 4 == 0;
-    c.tiles_k = (int)(kp / 64);
-    c.block_start = blocks;
-    const int prow = is_b ? cols : rows;
-    const int nt = c.tiles_k * ((prow + 63) / 64);
-    blocks += nt;
-    block_cut.insert(block_cut.end(), nt, (int)cuts.size());
-    cuts.push_back(c);
-    off.push_back(ws_bytes);
-    ws_bytes += bf3_align((size_t)prow * 3 * kp * 2);
-    return (int)cuts.size() - 1;
-  };
-  std::vector<int> ca, cb;
-  for (int i = 0; i < ndesc; ++i) {
-    const F32Desc &d = descs[i];
-    if (d.m <= 0 || d.n <= 0 || d.k <= 0) continue;
-    const long kp = ((long)d.k + 63) / 64 * 64;
-    // a tile's plane rows are read through 32-bit buffer offsets, and so is the k offset
-    if ((long)std::max(cf.bm, cf.bn) * 3 * kp * 2 >= 0x7fffffffL)
-      return phpc_set_error(PHPC_ERR_ARG, "k = %d too large for the slice planes", d.k);
-    ca.push_back(find_or_add(d.A, d.lda, d.m, d.k, 0, kp));
-    cb.push_back(find_or_add(d.B, d.ldb, d.k, d.n, 1, kp));
-    Bf3Item it{};
-    it.C = d.C;
-    it.ldc = d.ldc;
-    it.m = d.m;
-    it.n = d.n;
-    it.kp2 = (int)(kp * 2);
-    it.tiles_m = (d.m + cf.bm - 1) / cf.bm;
-    it.tiles_n = (d.n + cf.bn - 1) / cf.bn;
-    it.tile_start = total_tiles;
-    total_tiles += it.tiles_m * it.tiles_n;
-    items.push_back(it);
-  }
-  if (items.empty()) return PHPC_OK;
-  if (hipMalloc(&ws, ws_bytes) != hipSuccess) {
-    ws = nullptr;
-    return phpc_set_error(PHPC_ERR_MEM, "slice-plane workspace allocation failed (%zu bytes)", ws_bytes);
-  }
-  char *base = static_cast<char *>(ws);
-  for (size_t j = 0; j < cuts.size(); ++j) cuts[j].dst = reinterpret_cast<uint16_t *>(base + off[j]);
-  for (size_t i = 0; i < items.size(); ++i) {
-    items[i].A3 = cuts[ca[i]].dst;
-    items[i].B3 = cuts[cb[i]].dst;
-  }
-  const size_t cuts_b = bf3_align(cuts.size() * sizeof(Bf3Cut));
-  const size_t bc_b = bf3_align(block_cut.size() * sizeof(int));
-  const size_t it_b = items.size() * sizeof(Bf3Item);
-  if (hipMalloc(&list, cuts_b + bc_b + it_b) != hipSuccess) {
-    list = nullptr;
-    release();
-    return phpc_set_error(PHPC_ERR_MEM, "slice-plane list allocation failed");
-  }
-  char *l = static_cast<char *>(list);
-  PHPC_HIP(hipMemcpy(l, cuts.data(), cuts.size() * sizeof(Bf3Cut), hipMemcpyHostToDevice));
-  PHPC_HIP(hipMemcpy(l + cuts_b, block_cut.data(), block_cut.size() * sizeof(int), hipMemcpyHostToDevice));
-  PHPC_HIP(hipMemcpy(l + cuts_b + bc_b, items.data(), it_b, hipMemcpyHostToDevice));
-  return PHPC_OK;
-}
-
-int Bf3Planes::run(hipStream_t s, int grid) const {
-  if (items.empty() || total_tiles <= 0) return PHPC_OK;
-  const char *l = static_cast<const char *>(list);
-  const size_t cuts_b = bf3_align(cuts.size() * sizeof(Bf3Cut));
-  const size_t bc_b = bf3_align(block_cut.size() * sizeof(int));
-  hipLaunchKernelGGL(bf16x3_cut_kernel, dim3((unsigned)blocks), dim3(256), 0, s, reinterpret_cast<const Bf3Cut *>(l),
-                     reinterpret_cast<const int *>(l + cuts_b));
-  PHPC_HIP(hipGetLastError());
-  const Bf3GroupConfig &cf = kBf3Group[g];
-  const long G = std::min<long>(grid > 0 ? grid : (long)bf3_occupancy(g) * phpc_device().cus, total_tiles);
-  Bf3Group a{};
-  a.items = reinterpret_cast<const Bf3Item *>(l + cuts_b + bc_b);
-  a.count = (int)items.size();
-  a.total_tiles = total_tiles;
-  const int kt = phpc_ktime_begin(s);
-  hipLaunchKernelGGL(cf.fn, dim3((unsigned)G), dim3(cf.threads), cf.lds, s, a);
-  phpc_ktime_end(kt, s);
-  PHPC_HIP(hipGetLastError());
-  return PHPC_OK;
-}
-
-void Bf3Planes::release() {
-  if (list) (void)hipFree(list);
-  if (ws) (void)hipFree(ws);
-  list = nullptr;
-  ws = nullptr;
 }
 
 // ---------------------------------------------------------------------------
