@@ -274,6 +274,17 @@ inline long phpc_split_kp(long k) { return (k + 127) / 128 * 128; }
 // FP32-accurate 3 x BF16 GEMM through BF16 slice planes (workspace slots 0 and 1).
 int phpc_sgemm_bf16x3_planes(const float *dA, long lda, const float *dB, long ldb, float *dC, long ldc, int m, int k,
                              int n, hipStream_t s, Workspace *ws);
+// Residue operands of the CRT split GEMM, rows x kp bytes per modulus (kp a multiple of 64, rows
+// those of A or the columns of B): 16 rows at a time, and of these 64 k at a time, so that a load
+// of the product's is one contiguous KiB. The last rows lie as close together as there are of
+// them: no padding, modulus t's operand is rows * kp bytes.
+__host__ __device__ inline long crt_offset(int t, int rows, long kp, int r, long k) {
+  const int r0 = r / 16 * 16, held = rows - r0 < 16 ? rows - r0 : 16;
+  return ((long)t * rows + r0) * kp + k / 64 * (held * 64) + (r - r0) * 64 + k % 64;
+}
+// Residue products: res plane t (m x n bytes, row-major) = A_t B_t mod mods[t].
+int phpc_crt_level(const int8_t *A8, const int8_t *B8, long kp, int m, int n, int L, const int *mods, int8_t *res,
+                   hipStream_t s);
 int phpc_dgemm_split_ws(const double *dA, long lda, const double *dB, long ldb, double *dC, long ldc, int m, int k,
                         int n, int slices, double target_err, int method, hipStream_t stream, Workspace *ws,
                         phpc_split_info *info);

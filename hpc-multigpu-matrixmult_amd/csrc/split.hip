@@ -45,9 +45,6 @@ constexpr int kMaxSlicesF8 = 16;  // FP8-E4M3 slices carry 4 bits each
 // 74565 products: 225 * 74565 < 2^24
 constexpr long kMaxExactTermsF8 = 74565;
 constexpr long kMaxExactTerms = 131072;  // products per int32 accumulation (127^2 * 2^17 < 2^31)
-// residues reach -128: 128^2 * 130944 < 2^31 (130944 = 2^17 - 128, a whole number of
-// 128-byte slabs)
-constexpr long kMaxExactTermsCrt = 130944;
 // Widest integer operand of the CRT scheme: residues_of cuts |x| < 2^72 into nine bytes,
 // and the scaled operands satisfy |x| <= 2^p.
 constexpr int kMaxIntBits = 71;
@@ -350,29 +347,7 @@ struct LevelArgs {
   const int *eA;
   const int *eB;
   int first, last;
-  // residue mode (CRT scheme): res[i,j] = smod(S + (first ? 0 : res[i,j]), mod_m)
-  int mod_m;  // 0: level mode (FP64 epilogue above)
-  int8_t *res;
-  long ldres;
 };
-
-// v mod m in the symmetric range for |v| < 2^31 and a wave-uniform m: m = 256 gives
-// [-128, 127] (v's low byte), an odd m <= 255 gives |r| <= (m-1)/2, in int32 and FP32
-// arithmetic with rmf = 1/m rounded to FP32, on a = |v| (the residue of -a is minus that
-// of a for odd m). First round: float(a) is within 64 of a and the rounded product within
-// about 2 of a/m (< 2^24), so q1 = rint(a * rmf) leaves an exact remainder a - q1 m (a
-// 24-bit unsigned multiply) with |r| < 3m < 2^11. Second round: r is exact in FP32, r * rmf
-// is within 2^-20 of r/m, which for odd m lies at least 1/(2m) from a half-integer, so
-// q2 = rint(r * rmf) is the nearest quotient and r - q2 m the symmetric residue.
-__device__ __forceinline__ int smod_i32(int v, int m, float rmf) {
-  if (m == 256) return (int)(int8_t)(v & 0xff);
-  const uint32_t a = (uint32_t)(v < 0 ? -v : v);
-  const uint32_t q1 = (uint32_t)rintf((float)a * rmf);
-  const int r = (int)(a - __umul24(q1, (uint32_t)m));
-  const int q2 = (int)rintf((float)r * rmf);
-  const int s = r - __mul24(q2, m);
-  return v < 0 ? -s : s;
-}
 
 // LDS layout per stage: A then B, BM (BN) rows of BK k-bytes each, in 16-byte chunks.
 // Chunk c of row r sits at slot c ^ sw(r), sw(r) = (r * CPR / 16) mod CPR (CPR chunks per
@@ -586,32 +561,6 @@ __device__ __forceinline__ void level_tile(const LevelArgs &args, const LevelOps
     auto erow = [&](int i, int r) {
       return MI == 32 ? i * 32 + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4) : i * 16 + 4 * (lane >> 4) + r;
     };
-    const int mod_m = uni(args.mod_m);
-    if (mod_m > 0) {
-      const int firstr = uni(args.first);
-      const float rmf = 1.0f / (float)mod_m;
-      int8_t *resg = uni(args.res);
-      const long ldres = uni(args.ldres);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int col = col0 + wn * K::WTN + j * MI + (lane & (MI - 1));
-          if (col >= n) continue;
-#pragma unroll
-          for (int r = 0; r < NR; ++r) {
-            const int row = row0 + wm * K::WTM + erow(i, r);
-            if (row >= m) continue;
-            int8_t *pr = resg + (long)row * ldres + col;
-            // |sum| <= 128^2 x 130944 < 2^31 - 128 (kMaxExactTermsCrt), so adding the
-            // previous piece's residue stays in int32
-            int v = (int)acc[i][j][r];
-            if (!firstr) v += *pr;
-            *pr = (int8_t)smod_i32(v, mod_m, rmf);
-          }
-        }
-      return;
-    }
     const int sc = uni(args.scale_exp);
     const int first = uni(args.first), last = uni(args.last);
     gdouble *accg = (gdouble *)uni(args.acc);
@@ -946,27 +895,31 @@ __device__ __forceinline__ uint32_t pack4(int a, int b, int c, int d) {
 
 // residue_cols tile: k rows (a multiple of 4 dividing 128, the plane padding) by columns
 constexpr int kResColsTK = 128, kResColsTJ = 16;
-static_assert(128 % kResColsTK == 0 && kResColsTK == 4 * 32 && 256 % kResColsTJ == 0, "residue_cols tile");
+static_assert(128 % kResColsTK == 0 && kResColsTK % 64 == 0 && kResColsTJ == 16, "residue_cols tile");
 
-// A8 row i: residue plane t at bytes [t*kp, t*kp + k), zero to kp. Each thread handles
-// four consecutive k and stores one 32-bit word per plane; the next four k are loaded
-// before these are cut.
+// Residues of A's rows (crt_offset), zero from k to kp. A workgroup takes 16 rows and kResK k:
+// each thread four consecutive k of one row, so that 16 lanes read 512 bytes of a row and a wave
+// stores 256 contiguous bytes per modulus; the next four k are loaded before these are cut.
+constexpr int kResK = 1024;
 template <int L, bool NARROW>
-__global__ __launch_bounds__(256) void residue_rows_kernel(const double *__restrict__ A, long lda, int k, int p,
+__global__ __launch_bounds__(256) void residue_rows_kernel(const double *__restrict__ A, long lda, int m, int k, int p,
                                                            long kp, const int *__restrict__ eA, CrtConsts cc,
-                                                           int8_t *__restrict__ A8, long ld8) {
-  const int i = blockIdx.x;
+                                                           int8_t *__restrict__ A8) {
+  const int i = blockIdx.x * 16 + threadIdx.x / 16;
+  if (i >= m) return;
   const double *row = A + (long)i * lda;
   const int sh = p - eA[i];
-  int8_t *out = A8 + (long)i * ld8;
+  long l0 = (long)blockIdx.y * kResK + threadIdx.x % 16 * 4;
+  const long l1 = min(kp, (long)(blockIdx.y + 1) * kResK);
+  const long plane = (long)m * kp, step = crt_offset(0, m, kp, i, 64) - crt_offset(0, m, kp, i, 0);
+  int8_t *out = A8 + crt_offset(0, m, kp, i, l0);
   double xs[4];
-  long l0 = (long)threadIdx.x * 4;
 #pragma unroll
   for (int q = 0; q < 4; ++q) xs[q] = load_or_zero(row, l0 + q, l0 + q < k);
-  for (; l0 < kp; l0 += 1024) {
+  for (; l0 < l1; l0 += 64, out += step) {
     double nx[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) nx[q] = load_or_zero(row, l0 + 1024 + q, l0 + 1024 + q < k);
+    for (int q = 0; q < 4; ++q) nx[q] = load_or_zero(row, l0 + 64 + q, l0 + 64 + q < k);
     int r[4][L];
 #pragma unroll
     for (int q = 0; q < 4; ++q) residues_any<L, NARROW>(rint(ldexp(xs[q], sh)), cc, r[q]);  // 0 beyond k
@@ -974,18 +927,17 @@ __global__ __launch_bounds__(256) void residue_rows_kernel(const double *__restr
     for (int q = 0; q < 4; ++q) xs[q] = nx[q];
 #pragma unroll
     for (int t = 0; t < L; ++t)
-      *reinterpret_cast<uint32_t *>(out + (long)t * kp + l0) = pack4(r[0][t], r[1][t], r[2][t], r[3][t]);
+      *reinterpret_cast<uint32_t *>(out + t * plane) = pack4(r[0][t], r[1][t], r[2][t], r[3][t]);
   }
 }
 
-// B8 row j (column j of B): residue plane t at bytes [t*kp, t*kp + k). 128 (k) x 16 (j)
-// tiles pass through LDS (17 KiB: registers, not LDS, bound the occupancy); each thread
-// then takes four consecutive k of two columns, so 32 lanes write one column's 128 bytes
-// of a plane.
+// Residues of B's columns (crt_offset). 128 (k) x 16 (j) tiles pass through LDS (17 KiB:
+// registers, not LDS, bound the occupancy); each thread then takes four consecutive k of one
+// column, twice, so that the workgroup stores one contiguous KiB per modulus.
 template <int L, bool NARROW>
 __global__ __launch_bounds__(256) void residue_cols_kernel(const double *__restrict__ B, long ldb, int k, int n, int p,
                                                            long kp, const int *__restrict__ eB, CrtConsts cc,
-                                                           int8_t *__restrict__ B8, long ld8) {
+                                                           int8_t *__restrict__ B8) {
   constexpr int TK = kResColsTK, TJ = kResColsTJ;
   __shared__ double tile[TK][TJ + 1];
   const int k0 = blockIdx.x * TK;
@@ -1001,18 +953,19 @@ __global__ __launch_bounds__(256) void residue_cols_kernel(const double *__restr
 #pragma unroll
   for (int u = 0; u < NL; ++u) tile[ty + u * RS][tx] = v[u];
   __syncthreads();
-  const int kq = (threadIdx.x & 31) * 4;  // four consecutive k
-  for (int c = threadIdx.x >> 5; c < TJ; c += 8) {
-    const int jj = j0 + c;
-    if (jj >= n) continue;
-    const int sh = p - eB[jj];
+  const int c = threadIdx.x / 16, jj = j0 + c;
+  if (jj >= n) return;
+  const int sh = p - eB[jj];
+  const long plane = (long)n * kp;
+#pragma unroll 1
+  for (int kq = threadIdx.x % 16 * 4; kq < TK; kq += 64) {
     int r[4][L];
 #pragma unroll
     for (int q = 0; q < 4; ++q) residues_any<L, NARROW>(rint(ldexp(tile[kq + q][c], sh)), cc, r[q]);
-    int8_t *out = B8 + (long)jj * ld8 + k0 + kq;
+    int8_t *out = B8 + crt_offset(0, n, kp, jj, k0 + kq);
 #pragma unroll
     for (int t = 0; t < L; ++t)
-      *reinterpret_cast<uint32_t *>(out + (long)t * kp) = pack4(r[0][t], r[1][t], r[2][t], r[3][t]);
+      *reinterpret_cast<uint32_t *>(out + t * plane) = pack4(r[0][t], r[1][t], r[2][t], r[3][t]);
   }
 }
 
@@ -1126,19 +1079,19 @@ __global__ __launch_bounds__(256) void crt_reconstruct1_kernel(const int8_t *__r
 struct CrtLaunch {
   template <int L>
   static int run(hipStream_t s, const double *dA, long lda, const double *dB, long ldb, int m, int k, int n, int p,
-                 long kp, const int *eA, const int *eB, const CrtConsts &cc, int8_t *A8, int8_t *B8, long ld8,
-                 int stage, const int8_t *R8, double *dC, long ldc) {
+                 long kp, const int *eA, const int *eB, const CrtConsts &cc, int8_t *A8, int8_t *B8, int stage, const int8_t *R8, double *dC, long ldc) {
     if (stage == 0) {
       // |A'|, |B'| <= 2^p: the narrow residue form takes p <= kNarrowBits
       const bool narrow = p <= kNarrowBits;
       auto rows_fn = narrow ? residue_rows_kernel<L, true> : residue_rows_kernel<L, false>;
       auto cols_fn = narrow ? residue_cols_kernel<L, true> : residue_cols_kernel<L, false>;
-      hipLaunchKernelGGL(rows_fn, dim3(m), dim3(256), 0, s, dA, lda, k, p, kp, eA, cc, A8, ld8);
+      hipLaunchKernelGGL(rows_fn, dim3((unsigned)((m + 15) / 16), (unsigned)((kp + kResK - 1) / kResK)), dim3(256), 0, s,
+                         dA, lda, m, k, p, kp, eA, cc, A8);
       PHPC_HIP(hipGetLastError());
       hipLaunchKernelGGL(cols_fn,
                          dim3((unsigned)((kp + kResColsTK - 1) / kResColsTK),
                               (unsigned)((n + kResColsTJ - 1) / kResColsTJ)),
-                         dim3(256), 0, s, dB, ldb, k, n, p, kp, eB, cc, B8, ld8);
+                         dim3(256), 0, s, dB, ldb, k, n, p, kp, eB, cc, B8);
       PHPC_HIP(hipGetLastError());
     } else {
       const long total = (long)m * n;
@@ -1159,11 +1112,10 @@ struct CrtLaunch {
 
 template <int L>
 int crt_dispatch_t(int Lrt, hipStream_t s, const double *dA, long lda, const double *dB, long ldb, int m, int k, int n,
-                   int p, long kp, const int *eA, const int *eB, const CrtConsts &cc, int8_t *A8, int8_t *B8, long ld8,
-                   int stage, const int8_t *R8, double *dC, long ldc) {
-  if (Lrt == L) return CrtLaunch::run<L>(s, dA, lda, dB, ldb, m, k, n, p, kp, eA, eB, cc, A8, B8, ld8, stage, R8, dC, ldc);
+                   int p, long kp, const int *eA, const int *eB, const CrtConsts &cc, int8_t *A8, int8_t *B8, int stage, const int8_t *R8, double *dC, long ldc) {
+  if (Lrt == L) return CrtLaunch::run<L>(s, dA, lda, dB, ldb, m, k, n, p, kp, eA, eB, cc, A8, B8, stage, R8, dC, ldc);
   if constexpr (L < 20) {
-    return crt_dispatch_t<L + 1>(Lrt, s, dA, lda, dB, ldb, m, k, n, p, kp, eA, eB, cc, A8, B8, ld8, stage, R8, dC, ldc);
+    return crt_dispatch_t<L + 1>(Lrt, s, dA, lda, dB, ldb, m, k, n, p, kp, eA, eB, cc, A8, B8, stage, R8, dC, ldc);
   } else {
     return phpc_set_error(PHPC_ERR_ARG, "modulus count %d out of range", Lrt);
   }
@@ -1389,43 +1341,19 @@ int phpc_dgemm_split_ws(const double *dA, long lda, const double *dB, long ldb, 
     int8_t *R8 = (int8_t *)ws->get((size_t)L * m * n, 4, s);
     if (!A8 || !B8 || !R8) return phpc_set_error(PHPC_ERR_MEM, "CRT scratch allocation failed");
     {
-      int rc = crt_dispatch_t<2>(L, s, dA, lda, dB, ldb, m, k, n, pbits, kp, eA, eB, cc, A8, B8, ld8, 0, nullptr,
+      int rc = crt_dispatch_t<2>(L, s, dA, lda, dB, ldb, m, k, n, pbits, kp, eA, eB, cc, A8, B8, 0, nullptr,
                                  nullptr, 0);
       if (rc) return rc;
     }
-    long tiles256 = (long)((m + 255) / 256) * ((n + 255) / 256);
-    const int cfg = tiles256 >= (long)phpc_device().cus / 2 ? g_i8_big : 1;
-    const long piece = std::min<long>(kp, kMaxExactTermsCrt);
-    int launches = 0;
-    for (int t = 0; t < L; ++t) {
-      for (long off = 0; off < kp; off += piece) {
-        LevelArgs a{};
-        a.A8 = A8;
-        a.B8 = B8;
-        a.lda8 = ld8;
-        a.ldb8 = ld8;
-        a.a0 = (long)t * kp + off;
-        a.b0 = (long)t * kp + off;
-        a.m = m;
-        a.n = n;
-        a.kl = (int)std::min(piece, kp - off);
-        a.first = off == 0 ? 1 : 0;
-        a.mod_m = cc.m[t];
-        a.res = R8 + (size_t)t * m * n;
-        a.ldres = n;
-        int rc = launch_level(a, cfg, s);
-        if (rc) return rc;
-        ++launches;
-      }
-    }
+    if (int rc = phpc_crt_level(A8, B8, kp, m, n, L, cc.m, R8, s)) return rc;
     {
-      int rc = crt_dispatch_t<2>(L, s, dA, lda, dB, ldb, m, k, n, pbits, kp, eA, eB, cc, A8, B8, ld8, 1, R8, dC, ldc);
+      int rc = crt_dispatch_t<2>(L, s, dA, lda, dB, ldb, m, k, n, pbits, kp, eA, eB, cc, A8, B8, 1, R8, dC, ldc);
       if (rc) return rc;
     }
     if (info) {
       info->slices = L;
       info->products = L;
-      info->launches = launches + 7;
+      info->launches = 8;
       // exact scaling leaves the two roundings of C += 2^(e_i + f_j - 2p) C'
       info->error_estimate = exact_scaling ? std::ldexp(1.0, -52) : crt_error_estimate(pbits, mra, mrb, k);
       info->method = 1;
