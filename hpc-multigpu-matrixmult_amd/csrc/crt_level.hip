@@ -2,13 +2,14 @@
 // int8 operands, all moduli in one launch.
 //
 // What bounds it: the matrix cores, at the rate that the card sustains on dense int8 operands
-// (16384^3 with 13 moduli 44.8 ms, 2550 TOP/s; a plain library int8 product makes 2230), then the
-// reduction of each tile's sums. In 64x64 wave tiles, 16-byte LDS reads took as long as the
+// (16384^3 with 13 moduli 44.8 ms, 2550 TOP/s at the 1.83 GHz that its power leaves; a plain
+// library int8 product makes 2230), then the reduction of each tile's sums. In 64x64 wave
+// tiles, 16-byte LDS reads took as long as the
 // MFMAs; a wave of 8 now has 128x64 outputs (three quarters), reads a slab's operands behind the
 // MFMAs of the slab before, and does no vector arithmetic in the loop over slabs. One launch for
 // all moduli fills the last round once, not once per modulus: 1105x3061x7548 (150 tiles of
 // 256x256 a modulus) 715 -> 366 us, 2000^3 306 -> 116, 4096^3 960 -> 786, 8192^3 5.97 -> 5.7 ms,
-// 16384^3 45.0 -> 44.8 (the rate that the card holds).
+// 16384^3 46.1 -> 44.8 (the rate that the card holds).
 // Runs of tiles per XCD extend over two rounds, so that all eight work on a modulus or two and
 // operands come from memory about once (a run of whole moduli per XCD: 16384^3 47.6 ms;
 // 1105x3061x7548 is 366 us with two rounds, 425 with one).
@@ -53,6 +54,12 @@ __device__ __forceinline__ int smod_i32(int v, int m, float rmf) {
   return v < 0 ? -s : s;
 }
 
+// LDS slots of a 64-byte row. A 16-byte read serves lanes 0-3, 12-15 and 20-27 together, then
+// 4-11, 16-19 and 28-31 (the upper lanes likewise): with lane l on row l % 16, chunk l / 16, the
+// rows 8-15 two slots on, these cover all 64 banks once. (r / 4 % 4 covers them once for 16
+// neighbouring lanes, and cost a conflict on every read: 16384^3 47.1 ms, 44.8 now.)
+__device__ __forceinline__ int swizzle(int r) { return (r >> 3 & 1) << 1; }
+
 template <int BM, int BN, int WM, int WN, int STAGES>
 struct CrtShape {
   static constexpr int NW = WM * WN;
@@ -79,9 +86,9 @@ __device__ __forceinline__ void crt_tile(const CrtLevelArgs &g, int mod, int row
 
   // crt_offset() keeps 16 rows' 64 bytes together, so a load takes one KiB (rows of one modulus
   // 64 bytes at a time: 16384^3 59.7 ms against 50.2 on the same tiles).
-  // A stage holds rows of 64 bytes, 16-byte chunk c of row r at slot c ^ (r / 4 % 4), so the
-  // operand reads of 32 neighbouring rows cover the banks evenly. A wave's load fills 16 rows;
-  // rows past the matrix edge read the last one, whose outputs are not written.
+  // A stage holds rows of 64 bytes, 16-byte chunk c of row r at slot c ^ swizzle(r). A wave's
+  // load fills 16 rows; rows past the matrix edge read the last one, whose outputs are not
+  // written.
   rsrc_t src[K::PER];
   uint32_t off[K::PER];
   int step[K::PER];  // bytes from one slab to the next
@@ -93,7 +100,7 @@ __device__ __forceinline__ void crt_tile(const CrtLevelArgs &g, int mod, int row
                        (rows - 1) / 16 * 16);
     const int held = min(16, rows - r0);
     src[u] = make_rsrc((is_a ? g.A8 : g.B8) + ((long)mod * rows + r0) * g.kp, 0x7fffffffL);
-    off[u] = (uint32_t)(min(r, held - 1) * kBK + (((lane & 3) ^ ((r >> 2) & 3)) << 4));
+    off[u] = (uint32_t)(min(r, held - 1) * kBK + (((lane & 3) ^ swizzle(r)) << 4));
     step[u] = held * kBK;
   }
   auto issue = [&](int stage, int slab) {
@@ -166,7 +173,7 @@ __device__ __forceinline__ void crt_tile(const CrtLevelArgs &g, int mod, int row
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = i4v{};
   i4v a[2][TM], b[2][TN];
-  const int slot = ((lane >> 4) ^ ((lane >> 2) & 3)) << 4;
+  const int slot = ((lane >> 4) ^ swizzle(lane % 16)) << 4;
   const int a0 = (wm * K::WTM + lane % 16) * kBK + slot, b0 = K::B_BASE + (wn * K::WTN + lane % 16) * kBK + slot;
   auto read = [&](auto stage, auto set) {
     constexpr int q = decltype(stage)::value, x = decltype(set)::value;
