@@ -103,6 +103,10 @@ __device__ __forceinline__ int low_bit_code(double x) {
   return 1075 - q;
 }
 
+// The statistics are bound by memory, one read of each operand; 16 loads in flight per thread
+// (with four, rows and columns of 4096^2 took 60 us each, 45 and 32 now; a copy's rate is 28).
+constexpr int kStatLoads = 16;
+
 // One workgroup per row of A: exponent e_i, 2^e_i / mean|a_i.|, non-finite flag, and the
 // largest exact width over the rows (low_bit_code) into *width.
 __global__ __launch_bounds__(256) void row_stats_kernel(const double *__restrict__ A, long lda, int k,
@@ -116,15 +120,15 @@ __global__ __launch_bounds__(256) void row_stats_kernel(const double *__restrict
   double mx = 0.0, sm = 0.0;
   int code = 0;
   bool nonfinite = false;
-  // four loads in flight per thread; the zeros past k change neither the maximum, the
+  // kStatLoads loads in flight per thread; the zeros past k change neither the maximum, the
   // sum (+0.0 added to a sum of magnitudes) nor the code, so the order of the additions,
   // and the bits, are those of one element at a time
-  for (int l = threadIdx.x; l < k; l += 1024) {
-    double xs[4];
+  for (int l = threadIdx.x; l < k; l += 256 * kStatLoads) {
+    double xs[kStatLoads];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) xs[q] = load_or_zero(row, l + 256 * q, l + 256 * q < k);
+    for (int q = 0; q < kStatLoads; ++q) xs[q] = load_or_zero(row, l + 256 * q, l + 256 * q < k);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < kStatLoads; ++q) {
       const double x = xs[q];
       const double v = fabs(x);
       nonfinite |= !(v <= 1.79769313486231570815e308);  // inf or nan
@@ -138,19 +142,26 @@ __global__ __launch_bounds__(256) void row_stats_kernel(const double *__restrict
   red_sum[threadIdx.x] = sm;
   red_code[threadIdx.x] = code;
   __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if (threadIdx.x < off) {
-      red_max[threadIdx.x] = fmax(red_max[threadIdx.x], red_max[threadIdx.x + off]);
-      red_sum[threadIdx.x] += red_sum[threadIdx.x + off];
-      red_code[threadIdx.x] = max(red_code[threadIdx.x], red_code[threadIdx.x + off]);
-    }
-    __syncthreads();
+  // halves are added to halves, the last 64 of them within one wave
+  if (threadIdx.x >= 64) return;
+  mx = fmax(fmax(red_max[threadIdx.x], red_max[threadIdx.x + 128]),
+            fmax(red_max[threadIdx.x + 64], red_max[threadIdx.x + 192]));
+  sm = (red_sum[threadIdx.x] + red_sum[threadIdx.x + 128]) + (red_sum[threadIdx.x + 64] + red_sum[threadIdx.x + 192]);
+  code = max(max(red_code[threadIdx.x], red_code[threadIdx.x + 128]),
+             max(red_code[threadIdx.x + 64], red_code[threadIdx.x + 192]));
+  for (int off = 32; off > 0; off >>= 1) {
+    mx = fmax(mx, __shfl_down(mx, off));
+    sm += __shfl_down(sm, off);
+    code = max(code, __shfl_down(code, off));
   }
   if (threadIdx.x == 0) {
-    const int e = exp_of_max(red_max[0]);
+    const int e = exp_of_max(mx);
     eA[i] = e;
-    ratioA[i] = red_sum[0] > 0.0 ? ldexp((double)k, e) / red_sum[0] : 0.0;
-    if (red_code[0] > 0) atomicMax(width, e + red_code[0] - 1075);
+    ratioA[i] = sm > 0.0 ? ldexp((double)k, e) / sm : 0.0;
+    // one word for all rows: asked first, since most rows do not raise it (4096 atomics on it
+    // took 30 us)
+    const int w = e + code - 1075;
+    if (code > 0 && w > __hip_atomic_load(width, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(width, w);
   }
 }
 
@@ -208,38 +219,47 @@ struct RatioSummary {
   int pad;
 };
 
-__global__ __launch_bounds__(256) void ratio_summary_kernel(const double *__restrict__ ra, int m,
-                                                            const double *__restrict__ rb, int n,
-                                                            const int *__restrict__ bad,
-                                                            RatioSummary *__restrict__ out) {
-  __shared__ double red[4][256];
+__global__ __launch_bounds__(1024) void ratio_summary_kernel(const double *__restrict__ ra, int m,
+                                                             const double *__restrict__ rb, int n,
+                                                             const int *__restrict__ bad,
+                                                             RatioSummary *__restrict__ out) {
+  __shared__ double red[4][16];
   double v[4] = {0.0, 0.0, INFINITY, INFINITY};
-  for (int i = threadIdx.x; i < m; i += 256) {
-    const double x = ra[i];
-    if (x > v[0]) v[0] = x;
-    if (x > 0.0 && x < v[2]) v[2] = x;
-  }
-  for (int j = threadIdx.x; j < n; j += 256) {
-    const double x = rb[j];
-    if (x > v[1]) v[1] = x;
-    if (x > 0.0 && x < v[3]) v[3] = x;
-  }
-  for (int q = 0; q < 4; ++q) red[q][threadIdx.x] = v[q];
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) {
-      red[0][threadIdx.x] = fmax(red[0][threadIdx.x], red[0][threadIdx.x + h]);
-      red[1][threadIdx.x] = fmax(red[1][threadIdx.x], red[1][threadIdx.x + h]);
-      red[2][threadIdx.x] = fmin(red[2][threadIdx.x], red[2][threadIdx.x + h]);
-      red[3][threadIdx.x] = fmin(red[3][threadIdx.x], red[3][threadIdx.x + h]);
+  // eight loads in flight per thread: the zeros past the end are never positive
+  auto over = [&](const double *x, int count, double &mx, double &mn) {
+    for (int i = threadIdx.x; i < count; i += 8192) {
+      double xs[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) xs[q] = load_or_zero(x, i + 1024 * q, i + 1024 * q < count);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        if (xs[q] > mx) mx = xs[q];
+        if (xs[q] > 0.0 && xs[q] < mn) mn = xs[q];
+      }
     }
-    __syncthreads();
-  }
+  };
+  over(ra, m, v[0], v[2]);
+  over(rb, n, v[1], v[3]);
+  auto fold = [&](int width) {
+    for (int off = width / 2; off > 0; off >>= 1)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const double o = __shfl_down(v[q], off);
+        v[q] = q < 2 ? fmax(v[q], o) : fmin(v[q], o);
+      }
+  };
+  fold(64);
+  if ((threadIdx.x & 63) == 0)
+    for (int q = 0; q < 4; ++q) red[q][threadIdx.x >> 6] = v[q];
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  for (int q = 0; q < 4; ++q) v[q] = red[q][threadIdx.x & 15];
+  fold(16);
   if (threadIdx.x == 0) {
-    out->max_a = red[0][0];
-    out->max_b = red[1][0];
-    out->minpos_a = red[2][0];
-    out->minpos_b = red[3][0];
+    out->max_a = v[0];
+    out->max_b = v[1];
+    out->minpos_a = v[2];
+    out->minpos_b = v[3];
     out->bad = bad[0];
     out->width_a = bad[1];
     out->width_b = bad[2];
@@ -259,13 +279,13 @@ __global__ __launch_bounds__(256) void col_stats_kernel(const double *__restrict
   double mx = 0.0, sm = 0.0;
   int code = 0;
   bool nonfinite = false;
-  // four loads in flight per thread, the zeros past r1 neutral (as in row_stats_kernel)
-  for (int r = r0; r < r1; r += 4) {
-    double xs[4];
+  // the zeros past r1 are neutral (as in row_stats_kernel)
+  for (int r = r0; r < r1; r += kStatLoads) {
+    double xs[kStatLoads];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) xs[q] = load_or_zero(B, (long)(r + q) * ldb + j, r + q < r1);
+    for (int q = 0; q < kStatLoads; ++q) xs[q] = load_or_zero(B, (long)(r + q) * ldb + j, r + q < r1);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < kStatLoads; ++q) {
       const double x = xs[q];
       const double v = fabs(x);
       // per entry: fmax drops a NaN, so the maximum alone would not show one
@@ -1287,7 +1307,11 @@ int phpc_dgemm_split_ws(const double *dA, long lda, const double *dB, long ldb, 
   }
   hipLaunchKernelGGL(row_stats_kernel, dim3(m), dim3(256), 0, s, dA, lda, k, eA, ratioA, bad, bad + 1);
   PHPC_HIP(hipGetLastError());
-  const int rows_per_block = 256;
+  // enough workgroups to fill the GPU, and few enough atomics
+  const long col_blocks = (n + 255) / 256;
+  int rows_per_block = 256;
+  while (rows_per_block > 32 && col_blocks * ((k + rows_per_block - 1) / rows_per_block) < 4L * phpc_device().cus)
+    rows_per_block /= 2;
   hipLaunchKernelGGL(col_stats_kernel, dim3((n + 255) / 256, (k + rows_per_block - 1) / rows_per_block), dim3(256), 0,
                      s, dB, ldb, k, n, rows_per_block, cmax, csum, ccode, bad);
   PHPC_HIP(hipGetLastError());
@@ -1298,7 +1322,7 @@ int phpc_dgemm_split_ws(const double *dA, long lda, const double *dB, long ldb, 
   if (use_crt) {
     // CRT scheme: choose the integer width p, then the modulus count
     RatioSummary hs{};
-    hipLaunchKernelGGL(ratio_summary_kernel, dim3(1), dim3(256), 0, s, ratioA, m, ratioB, n, bad, summary);
+    hipLaunchKernelGGL(ratio_summary_kernel, dim3(1), dim3(1024), 0, s, ratioA, m, ratioB, n, bad, summary);
     PHPC_HIP(hipGetLastError());
     PHPC_HIP(hipMemcpyAsync(&hs, summary, sizeof(hs), hipMemcpyDeviceToHost, s));
     PHPC_HIP(hipStreamSynchronize(s));
@@ -1367,7 +1391,7 @@ int phpc_dgemm_split_ws(const double *dA, long lda, const double *dB, long ldb, 
   {
     // exponents and ratios decide the slice count (and reveal non-finite input)
     RatioSummary hs{};
-    hipLaunchKernelGGL(ratio_summary_kernel, dim3(1), dim3(256), 0, s, ratioA, m, ratioB, n, bad, summary);
+    hipLaunchKernelGGL(ratio_summary_kernel, dim3(1), dim3(1024), 0, s, ratioA, m, ratioB, n, bad, summary);
     PHPC_HIP(hipGetLastError());
     PHPC_HIP(hipMemcpyAsync(&hs, summary, sizeof(hs), hipMemcpyDeviceToHost, s));
     PHPC_HIP(hipStreamSynchronize(s));
