@@ -213,10 +213,25 @@ F64Config phpc_f64_config(int id);
 // Host <-> device copies through pinned staging buffers (rows x width bytes, strided).
 // h2d returns once the source may be reused (transfers complete in stream order); d2h
 // returns once the destination holds the data.
-int phpc_stage_h2d(void *dst, size_t dpitch, const void *src, size_t spitch, size_t width, size_t rows,
-                   hipStream_t stream);
-int phpc_stage_d2h(void *dst, size_t dpitch, const void *src, size_t spitch, size_t width, size_t rows,
-                   hipStream_t stream);
+struct StageCopy {
+  void *dst;
+  size_t dpitch;
+  const void *src;
+  size_t spitch;
+  size_t width, rows;  // bytes per row, rows
+};
+int phpc_stage_h2d(const StageCopy *copies, int count, hipStream_t stream);
+int phpc_stage_d2h(const StageCopy *copies, int count, hipStream_t stream);
+inline int phpc_stage_h2d(void *dst, size_t dpitch, const void *src, size_t spitch, size_t width, size_t rows,
+                          hipStream_t stream) {
+  const StageCopy c{dst, dpitch, src, spitch, width, rows};
+  return phpc_stage_h2d(&c, 1, stream);
+}
+inline int phpc_stage_d2h(void *dst, size_t dpitch, const void *src, size_t spitch, size_t width, size_t rows,
+                          hipStream_t stream) {
+  const StageCopy c{dst, dpitch, src, spitch, width, rows};
+  return phpc_stage_d2h(&c, 1, stream);
+}
 // Process-wide copy and compute streams of the host-pointer entry points.
 int phpc_host_streams(hipStream_t *copy, hipStream_t *compute);
 int phpc_pack_launch(const double *src, long lds, double *dst, long ldd, int rows, int cols,

@@ -326,11 +326,10 @@ static int gemm_cuda_impl(const double *a, int lda, const double *b, int ldb, do
   if (!dA || !dB || !dC) return phpc_set_error(PHPC_ERR_MEM, "device allocation failed");
   hipStream_t s, sc_unused;
   if (int rc = phpc_host_streams(&s, &sc_unused)) return rc;
-  if (k > 0) {
-    if (int rc = phpc_stage_h2d(dA, (size_t)k * 8, a, (size_t)lda * 8, (size_t)k * 8, m, s)) return rc;
-    if (int rc = phpc_stage_h2d(dB, (size_t)n * 8, b, (size_t)ldb * 8, (size_t)n * 8, k, s)) return rc;
-  }
-  if (int rc = phpc_stage_h2d(dC, (size_t)n * 8, c, (size_t)ldc * 8, (size_t)n * 8, m, s)) return rc;
+  const StageCopy in[3] = {{dC, (size_t)n * 8, c, (size_t)ldc * 8, (size_t)n * 8, (size_t)m},
+                           {dA, (size_t)k * 8, a, (size_t)lda * 8, (size_t)k * 8, (size_t)m},
+                           {dB, (size_t)n * 8, b, (size_t)ldb * 8, (size_t)n * 8, (size_t)k}};
+  if (int rc = phpc_stage_h2d(in, k > 0 ? 3 : 1, s)) return rc;
   ScopedEvent e0, e1;
   if (!e0.e || !e1.e) return phpc_set_error(PHPC_ERR_HIP, "event creation failed");
   PHPC_HIP(hipEventRecord(e0.e, s));
