@@ -228,13 +228,12 @@ def grouped_bench(phpc, seed=21):
             worst = max(worst, float(np.max(np.abs(got - ref) / np.maximum(scale, 1e-300))))
         info = plan.info()
         if dtype == phpc.F32X3:
-            launch = ("one batched kernel cutting every A and B into BF16 slice planes + one persistent "
-                      "BF16 level launch (three k segments per item) for all 512 GEMMs"
-                      if info["config"] >= 4 else "one persistent 3 x BF16 kernel for all 512 GEMMs")
+            launch = ("one batched kernel cutting every A and B into BF16 slice planes + one launch of all "
+                      "six products for all 512 GEMMs" if info["config"] >= 4 else
+                      "one persistent 3 x BF16 kernel for all 512 GEMMs")
         else:
-            launch = ("one batched kernel transposing every A + one persistent transposed-A kernel for all "
-                      "512 GEMMs (B read in place)" if info["config"] == 3 else
-                      "one persistent kernel for all 512 GEMMs")
+            launch = ("one direct-to-LDS launch for all 512 GEMMs (operands read in place)" if info["config"] == 3
+                      else "one persistent kernel for all 512 GEMMs")
         out[key] = {"tflops": round(flops / (ms * 1e-3) / 1e12, 3), "ms": round(ms, 3), "flops": flops,
                     "config": info["config"], "tiles": info["tiles"], "tuned_ms": round(info["tuned_ms"], 3),
                     "err_cw_max_sampled": worst, "fp32_mfma_util": round(flops / (ms * 1e-3) / 157.3e12, 4),
@@ -693,7 +692,7 @@ def main():
                       "moduli": i.slices, "int_bits": i.int_bits, "error_estimate": i.error_estimate,
                       "err_cw_max_sampled": cw, "err_nw_sampled": nw,
                       "int8_kernel_ms_avg": round(lvl_avg, 4), "int8_launches": lvl_n,
-                      "int8_kernel_tops": round(2.0 * N * N * kp / (lvl_avg * 1e-3) / 1e12, 2),
+                      "int8_kernel_tops": round(2.0 * N * N * kp * i.slices / (lvl_avg * 1e-3) / 1e12, 2),
                       "int8_share_of_time": round(lvl_ms / reps / t_ms, 4)}
         if tag == "uniform" and not args.no_clock:
             split[tag]["clock"] = clock_during(run_split)
@@ -752,9 +751,8 @@ def main():
             "N": N,
             "grid": f"{p}x{q}",
             "panel": panel,
-            "path": "plain FP64 MFMA, SUMMA CHAINED schedule: A row blocks transposed once per pass, "
-                    "then one persistent launch, 128x128 tiles fed HBM->LDS directly, one FMA chain per "
-                    "output over the 64 panels",
+            "path": "plain FP64 MFMA, SUMMA CHAINED schedule: one launch, 256x128 tiles fed HBM->LDS directly "
+                    "from where the operands lie, one FMA chain per output over the 64 panels",
             "flops_per_step": flops,
         },
         "roofline": {
@@ -766,12 +764,12 @@ def main():
             "traffic": traffic_from_profiles(workload),
             "traffic_source": "profiles/traffic.json (rocprofv3 FETCH_SIZE + WRITE_SIZE of this kernel, "
                               "scaled by a 1 GiB copy), not measured in this run",
-            "kernel": "f64_at_128x128 (transposed-A, direct-to-LDS, 2 workgroups per CU)",
+            "kernel": "rm_kernel 256x128 (direct-to-LDS, operands in place, 16 waves, 64x64 tail tiles)",
             "kernel_ms_avg": round(kernel_ms, 3),
             "kernel_launches_timed": k_launches,
             "pass_ms_avg": round(ms_per_step, 3),
             "timed_unit": "achieved = 2N^3 / kernel_ms_avg (HIP events around the GEMM launch alone, on its "
-                          "stream); a step (pass) adds the 4 A row-block transposes",
+                          "stream)",
             "clock_mhz": (plain_clock or {}).get("mhz_median"),
         },
         "accuracy": {"err_cw_max_sampled": err_cw, "err_nw_sampled": err_nw, "samples": 4096,
@@ -784,13 +782,13 @@ def main():
         "split_moduli": {"uniform": uni["moduli"], "wide_exponent": wide["moduli"]},
         "split_roofline": {
             "bound": "mfma",
-            "kernel": "i8_level_256x256_w16_k128_mi16 (one int8 residue GEMM per modulus, 16x16x64 MFMAs)",
+            "kernel": "crt_level_kernel 256x256 (the int8 residue GEMMs of all moduli in one launch, 16x16x64 MFMAs)",
             "achieved": uni["int8_kernel_tops"],
             "peak": 5000.0,
             "unit": "TOP/s",
             "frac": round(uni["int8_kernel_tops"] / 5000.0, 4),
             "kernel_ms_avg": uni["int8_kernel_ms_avg"],
-            "ops_per_launch": 2.0 * N * N * ((N + 127) // 128 * 128),
+            "ops_per_launch": 2.0 * N * N * ((N + 127) // 128 * 128) * uni["moduli"],
             "share_of_split_time": uni["int8_share_of_time"],
             # the nominal peak assumes 2.4 GHz; under this load the chip holds a lower clock
             "clock_mhz": (uni.get("clock") or {}).get("mhz_median"),
@@ -803,8 +801,8 @@ def main():
             "tflops": round(exact_tf, 3),
             "roofline": {"bound": "mfma", "achieved": round(exact_kernel_tf, 3), "peak": FP64_PEAK_TFLOPS,
                          "unit": "TFLOP/s", "frac": round(exact_kernel_tf / FP64_PEAK_TFLOPS, 4),
-                         "kernel": "f64_at_128x128_w16_mp_k32 (16 waves, 32-deep slabs; per-panel sums added "
-                                   "to the C carried in registers)",
+                         "kernel": "rm_kernel 128x128 with panels (16 waves, 64x64 tail tiles; per-panel sums "
+                                   "added to the C carried in registers)",
                          "kernel_ms_avg": round(exact_kernel_ms, 3), "pass_ms_avg": round(exact_ms, 3)},
             "arithmetic": "bit-exact to the reference's per-panel grouping (src/phpc_summa.c:63-95)",
         },
