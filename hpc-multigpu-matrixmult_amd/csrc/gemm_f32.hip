@@ -1,7 +1,7 @@
 // FP32 grouped GEMM on gfx950 matrix cores: C += A*B for a list of independent row-major FP32
 // GEMMs of any shapes, one launch. Two families: the direct kernels (gemm_rm.h,
-// v_mfma_f32_16x16x4f32), which every product takes whose leading dimensions fit their 32-bit
-// offsets, and the register-staged ones below (v_mfma_f32_32x32x2f32), for the others. Both sum
+// v_mfma_f32_16x16x4f32), and the register-staged ones below (v_mfma_f32_32x32x2f32), for tuning
+// and for leading dimensions of B that do not fit the direct kernels' 32-bit offsets. Both sum
 // each output as one FMA chain in k order: the same bits.
 //
 // The register-staged kernels: a BM x BN macro tile per workgroup, 4 waves in a
@@ -476,8 +476,7 @@ int phpc_f32_plan_tiles(F32Desc *descs, int ndesc, int id) {
 bool phpc_f32_direct_ok(const F32Desc *descs, int ndesc) {
   for (int i = 0; i < ndesc; ++i)
     for (const F32RmConfig &c : kF32Rm)
-      if ((long)c.a_rows * descs[i].lda * 4 >= 0x7fffffffL || (long)c.b_rows * descs[i].ldb * 4 >= 0x7fffffffL)
-        return false;
+      if ((long)c.b_rows * descs[i].ldb * 4 >= 0x7fffffffL) return false;
   return true;
 }
 
@@ -499,6 +498,7 @@ int phpc_f32_prepare(const F32Desc *descs, int ndesc, F32Work *w) {
   const F32RmConfig &c = kF32Rm[w->config];
   if (!phpc_f32_direct_ok(w->descs.data(), (int)w->descs.size()))
     return phpc_set_error(PHPC_ERR_ARG, "leading dimension too large");
+  rm_split_rows(w->descs, c.a_rows);
   std::vector<F32Desc> tail;
   if (c.tail_bm) rm_split_tail(w->descs, c.bm, c.bn, cus, tail);
   long t = 0;
@@ -665,7 +665,20 @@ extern "C" int phpc_sgemm_device(const float *dA, long lda, const float *dB, lon
     if (g_f32_direct && phpc_f32_direct_ok(&d, 1)) {
       F32Work w;
       rc = phpc_f32_prepare(&d, 1, &w);
-      if (!rc) rc = phpc_f32_launch_direct(w, nullptr, 0, (hipStream_t)stream);
+      if (!rc && w.list.empty()) {
+        rc = phpc_f32_launch_direct(w, nullptr, 0, (hipStream_t)stream);
+      } else if (!rc) {
+        // rows too far apart for one launch's offsets (rm_split_rows): one by one, without a list
+        for (int r = 0; r < m && !rc; ++r) {
+          F32Desc row = d;
+          row.A += (long)r * lda;
+          row.C += (long)r * ldc;
+          row.m = 1;
+          row.lda = k;
+          rc = phpc_f32_prepare(&row, 1, &w);
+          if (!rc) rc = phpc_f32_launch_direct(w, nullptr, 0, (hipStream_t)stream);
+        }
+      }
     } else {
       const long work = (long)((m + 127) / 128) * ((n + 127) / 128);
       const int cfg = work >= 2L * phpc_device().cus ? 2 : 0;

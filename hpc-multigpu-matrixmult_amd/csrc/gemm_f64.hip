@@ -453,6 +453,7 @@ int phpc_f64_prepare(const GemmDesc *descs, int ndesc, int config_id, bool devic
   w->config = config_id;
   w->mp = false;
   w->vec2 = true;
+  if (ce.lds_bytes) rm_split_rows(w->descs, ce.a_rows);
   for (const GemmDesc &d : w->descs) {
     w->mp |= has_panels(d);
     if ((long)ce.a_rows * d.lda * 8 >= 0x7fffffffL || (long)ce.b_rows * d.ldb * 8 >= 0x7fffffffL)

@@ -722,6 +722,30 @@ long rm_tiles(const Desc &d, int bm, int bn) {
   return (long)((d.m + bm - 1) / bm) * ((d.n + bn - 1) / bn);
 }
 
+// GEMMs whose rows of A lie so far apart that `rows` of them span 2 GiB or more, a load's 32-bit
+// offset, become GEMMs of one row each
+template <class Desc>
+void rm_split_rows(std::vector<Desc> &v, long rows) {
+  auto far = [&](const Desc &d) { return rows * d.lda * (long)sizeof(*d.C) >= 0x7fffffffL; };
+  if (std::none_of(v.begin(), v.end(), far)) return;
+  std::vector<Desc> split;
+  for (const Desc &d : v) {
+    if (!far(d)) {
+      split.push_back(d);
+      continue;
+    }
+    for (int r = 0; r < d.m; ++r) {
+      Desc t = d;
+      t.A += (long)r * d.lda;
+      t.C += (long)r * d.ldc;
+      t.m = 1;
+      t.lda = d.k;
+      split.push_back(t);
+    }
+  }
+  v.swap(split);
+}
+
 // elements of B from one column to the next
 inline long rm_col_step(const GemmDesc &) { return 1; }
 inline long rm_col_step(const F32Desc &) { return 1; }

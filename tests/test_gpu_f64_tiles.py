@@ -95,3 +95,27 @@ def test_tail_of_several_gemms_as_one_plan():
     for (_, _, dC), w in zip(items, want):
         assert np.array_equal(bits(dC.cpu().numpy()), bits(w))
     plan.close()
+
+
+# rows of A so far apart that a load's rows span 2 GiB: products of one row each
+@pytest.mark.parametrize("dtype,lda", [("f64", 34_000_000), ("f32", 68_000_000)])
+def test_rows_of_a_far_apart(dtype, lda):
+    import torch
+    f64 = dtype == "f64"
+    tdt = torch.float64 if f64 else torch.float32
+    m, k, n = 3, 37, 130
+    g = torch.Generator(device="cuda").manual_seed(3)
+    far = torch.empty((m - 1) * lda + k, dtype=tdt, device="cuda").as_strided((m, k), (lda, 1))
+    A, B, C0 = (torch.randint(-8, 9, s, generator=g, device="cuda").to(tdt) for s in ((m, k), (k, n), (m, n)))
+    far.copy_(A)
+    want = C0 + (A.double() @ B.double()).to(tdt)  # integers: exact in any order
+    C, D, E = C0.clone(), C0.clone(), C0.clone()
+    if f64:
+        phpc.dgemm_device(far, B, C)
+    else:
+        phpc.sgemm_device(far, B, C, method=phpc.SGEMM_FP32)
+    plan = phpc.Plan(phpc.F64 if f64 else phpc.F32, [(far, B, D), (A, B, E)])
+    plan.launch()
+    torch.cuda.synchronize()
+    plan.close()
+    assert torch.equal(C, want) and torch.equal(D, want) and torch.equal(E, want)
