@@ -432,6 +432,7 @@ constexpr F32RmConfig f32_rm_config() {
 using G32 = RmTile<float, 32, 32, 2, 2, 32, 4, false>;
 using G32K64 = RmTile<float, 32, 32, 2, 2, 64, 4, false>;
 using G64 = RmTile<float, 64, 64, 2, 2, 32, 4, false>;
+using G64K64 = RmTile<float, 64, 64, 4, 2, 64, 4, false>;
 using G64W8 = RmTile<float, 64, 64, 4, 2, 32, 4, false>;
 using G128 = RmTile<float, 128, 64, 4, 2, 32, 3, false>;
 // The tile shapes of the planner's rule. Measured (device time): 256^3 5.4 us on 32x32 against
@@ -439,11 +440,12 @@ using G128 = RmTile<float, 128, 64, 4, 2, 32, 3, false>;
 // register-staged 64x64 tiles before; 4096^3 949 us (145 TF/s) on 128x64 with two workgroups to
 // a CU, 966 on 64x64, 966 on 256x128 with one; 512 products log-uniform in [64, 4096] 9.25 ms
 // on 128x64, 9.45 on 64x64, 9.9 on 256x128, 11.6 before (128x128, operands staged).
-enum { kF32Small = 0, kF32Mid = 1, kF32Big = 2 };
+enum { kF32Small = 0, kF32Mid = 1, kF32Big = 2, kF32One = 3 };
 const F32RmConfig kF32Rm[] = {
     f32_rm_config<G32, G32>(),
     f32_rm_config<G64, G32K64>(),
     f32_rm_config<G128, G64W8>(),
+    f32_rm_config<G64K64, G64K64>(),
 };
 std::once_flag g_rm_once;
 
@@ -493,8 +495,13 @@ int phpc_f32_prepare(const F32Desc *descs, int ndesc, F32Work *w) {
   const long cus = phpc_device().cus;
   // 128x64 tiles from four a CU on (two rounds of the two resident ones): 3000^3, 4.4 a CU, 404
   // us against 416 on 64x64, but 2500^3, 3.1 a CU, 265 against 249. 32x32 tiles where 64x64 ones
-  // would leave CUs empty: 256^3 5.4 us against 9.5.
-  w->config = t128 >= 4 * cus ? kF32Big : t64 >= cus ? kF32Mid : kF32Small;
+  // would leave CUs empty: 256^3 5.4 us against 9.5. From three quarters of them to one 64x64
+  // tile per CU, those in 8 waves on 64-deep slabs: 1000^3 21.9 us against 24.1 in 4 waves and
+  // 22.6 on 32x32, 1024 x 4096 x 1024 66 against 70 and 75; 800^3, 0.66 a CU, 17.6 against 15.2.
+  w->config = t128 >= 4 * cus                    ? kF32Big
+              : 4 * t64 > 3 * cus && t64 <= cus ? kF32One
+              : t64 >= cus                      ? kF32Mid
+                                                : kF32Small;
   const F32RmConfig &c = kF32Rm[w->config];
   if (!phpc_f32_direct_ok(w->descs.data(), (int)w->descs.size()))
     return phpc_set_error(PHPC_ERR_ARG, "leading dimension too large");

@@ -328,7 +328,7 @@ template <bool MP> using T256 = RmTile<double, 256, 128, 4, 4, 16, 3, MP>;      
    {{PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 1), PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 2)},                  \
     {PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 1), PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 2)}}, 0, 0}
 
-constexpr int kSmall = 13, kMid = 5, kBig = 11, kBigPanels = 16, kListPanels = 3;  // the planner's
+constexpr int kSmall = 13, kMid = 5, kBig = 11, kBigPanels = 16, kListPanels = 3, kOne = 10;  // the planner's
 const ConfigEntry kConfigs[] = {
     V1_CONFIG(128, 128, 2, 4, 16),             // 0: register-staged, 8 waves (wave tile 64x32)
     V1_CONFIG(128, 128, 2, 4, 32),             // 1: register-staged, 8 waves, 32-deep slabs
@@ -340,7 +340,7 @@ const ConfigEntry kConfigs[] = {
     rm_config<T256W8, T256W8, true>(),         // 7: single panel only
     V1_CONFIG_SP(128, 128, 2, 2, 16),          // 8: register-staged, 4 waves (wave tile 64x64); single panel only
     rm_config<T64x32, T64x32, true>(),         // 9: single panel only
-    rm_config<T64W16, T64W16, true>(),         // 10: single panel only
+    rm_config<T64W16, T64W16, true>(),         // 10: the planner's for about one 64x64 tile per CU; single panel only
     rm_config<T256, T64W16, true>(),           // 11: the planner's for large single-panel work; single panel only
     rm_config<T128x64, T128x64>(),             // 12
     rm_config<T32, T32>(),                     // 13: the planner's for small work
@@ -415,7 +415,11 @@ namespace {
 // choices:
 //   fewer 64x64 tiles than CUs: 32x32 tiles (512^3: 8.6 us against 20.4 on 64x64, N = 256:
 //     6.2 against 12.7), whose workgroups share a CU five at a time;
-//   then 64x64 tiles with a 32x32 tail (2048^3: 68 TFLOP/s against 54 on 32x32 alone);
+//   from three quarters of them to one 64x64 tile per CU, those in 16 waves on 32-deep slabs,
+//     which hide each other's barriers where no second workgroup does (1024 x 4096 x 1024: 123
+//     us against 138 in 4 waves and 139 on 32x32; 1024^3 37.5 against 39.7 and 37.3;
+//     600 x 3000 x 900, 0.6 a CU, 92 against 79 on 32x32);
+//   then 64x64 tiles in 4 waves with a 32x32 tail (2048^3: 68 TFLOP/s against 54 on 32x32 alone);
 //   from two 256x128 tiles per CU on, those (4096^3: 73.2 against 68; 16384^3: 74.8 against 65
 //     on 64x64), or, with panels, 128x128 tiles, whose waves have room for the carried C. Large
 //     panel-grouped lists (plans) take 8 waves and no tail: where launches of several streams
@@ -433,6 +437,7 @@ int config_for(const GemmDesc *descs, int ndesc, bool device_list) {
   const long cus = phpc_device().cus;
   if (mp && t128 >= 4 * cus) return device_list && g_big_config >= 0 ? g_big_config : g_big_config_host;
   if (!mp && t256 >= 2 * cus) return device_list && g_big_single >= 0 ? g_big_single : g_big_single_host;
+  if (!mp && 4 * t64 > 3 * cus && t64 <= cus) return kOne;
   return t64 >= cus ? kMid : kSmall;
 }
 

@@ -42,7 +42,7 @@ def staged(A, B, C0):
 # with a 64x64 tail, on 256 CUs
 @pytest.mark.parametrize("m,k,n", [(1, 1, 1), (31, 31, 33), (65, 33, 63), (129, 64, 127), (255, 65, 257),
                                    (33, 97, 31), (64, 160, 129), (40, 401, 31), (1, 300, 700), (700, 300, 1),
-                                   (1100, 35, 1001), (500, 40, 2301), (1100, 161, 1001), (4100, 20, 2201),
+                                   (1100, 35, 1001), (500, 40, 2301), (1100, 161, 1001), (4100, 20, 2201), (1023, 63, 1000), (961, 257, 1024),
                                    (2200, 67, 4301), (4096, 129, 2049)])
 def test_tile_slab_and_tail_edges(m, k, n):
     import torch

@@ -74,7 +74,7 @@ def test_panel_edges(cfg, m, k, n, panel):
 
 # work that the planner cuts into head tiles and a tail of smaller ones: by rows, by columns,
 # on 64x64, 256x128 and (with panels) 128x128 heads, on 256 CUs
-@pytest.mark.parametrize("m,k,n,panel", [(1100, 35, 1001, 0), (500, 40, 2301, 0), (1100, 35, 1001, 16),
+@pytest.mark.parametrize("m,k,n,panel", [(1023, 33, 1000, 0), (961, 130, 1024, 0), (1023, 33, 1000, 9), (1100, 35, 1001, 0), (500, 40, 2301, 0), (1100, 35, 1001, 16),
                                          (4100, 20, 4201, 0), (4200, 20, 4101, 7)])
 def test_head_and_tail(m, k, n, panel):
     run(m, k, n, -1, panel)
