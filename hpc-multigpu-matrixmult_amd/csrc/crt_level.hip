@@ -8,7 +8,7 @@
 // MFMAs; a wave of 8 now has 128x64 outputs (three quarters), reads a slab's operands behind the
 // MFMAs of the slab before, and does no vector arithmetic in the loop over slabs. One launch for
 // all moduli fills the last round once, not once per modulus: 1105x3061x7548 (150 tiles of
-// 256x256 a modulus) 715 -> 366 us, 2000^3 306 -> 116, 4096^3 960 -> 786, 8192^3 5.97 -> 5.7 ms,
+// 256x256 a modulus) 715 -> 366 us, 2000^3 306 -> 116, 4096^3 960 -> 795, 8192^3 5.97 -> 5.7 ms,
 // 16384^3 46.1 -> 44.8 (the rate that the card holds).
 // Runs of tiles per XCD extend over two rounds, so that all eight work on a modulus or two and
 // operands come from memory about once (a run of whole moduli per XCD: 16384^3 47.6 ms;
@@ -34,24 +34,18 @@ struct CrtLevelArgs {
   int kp, m, n, L;
   int tiles_m, tiles_n, window;
   int mods[20];
+  int c19[20];  // 2^19 mod m, symmetric
 };
 
-// v mod m in the symmetric range for |v| < 2^31 and a wave-uniform m: m = 256 gives
-// [-128, 127] (v's low byte), an odd m <= 255 gives |r| <= (m-1)/2, in int32 and FP32
-// arithmetic with rmf = 1/m rounded to FP32, on a = |v| (the residue of -a is minus that
-// of a for odd m). First round: float(a) is within 64 of a and the rounded product within
-// about 2 of a/m (< 2^24), so q1 = rint(a * rmf) leaves an exact remainder a - q1 m (a
-// 24-bit unsigned multiply) with |r| < 3m < 2^11. Second round: r is exact in FP32, r * rmf
-// is within 2^-20 of r/m, which for odd m lies at least 1/(2m) from a half-integer, so
-// q2 = rint(r * rmf) is the nearest quotient and r - q2 m the symmetric residue.
-__device__ __forceinline__ int smod_i32(int v, int m, float rmf) {
-  if (m == 256) return (int)(int8_t)(v & 0xff);
-  const uint32_t a = (uint32_t)(v < 0 ? -v : v);
-  const uint32_t q1 = (uint32_t)rintf((float)a * rmf);
-  const int r = (int)(a - __umul24(q1, (uint32_t)m));
-  const int q2 = (int)rintf((float)r * rmf);
-  const int s = r - __mul24(q2, m);
-  return v < 0 ? -s : s;
+// v mod an odd m <= 255 in the symmetric range (|r| <= (m - 1) / 2), m wave-uniform: v = h 2^19 + l
+// with -4096 <= h < 4096, so h c + l with c = 2^19 mod m (|c| <= 127) is v mod m and below 2^20,
+// exact in FP32. Over m it is below 6100, where rounding 1 / m and the product moves it by less
+// than 0.001, while it lies at least 1 / (2 m) from a half-integer: the nearest integer is the
+// exact quotient. (Two rounds on |v|, with twice the instructions: 4096^3 with 13 moduli 840 us,
+// 795 now.)
+__device__ __forceinline__ int smod_odd(int v, int c, float m, float rm) {
+  const float f = (float)(__mul24(v >> 19, c) + (v & 0x7ffff));
+  return (int)fmaf(-rintf(f * rm), m, f);
 }
 
 // LDS slots of a 64-byte row. A 16-byte read serves lanes 0-3, 12-15 and 20-27 together, then
@@ -204,14 +198,17 @@ __device__ __forceinline__ void crt_tile(const CrtLevelArgs &g, int mod, int row
     }
   };
   const int mod_m = g.mods[mod];
-  const float rmf = 1.0f / (float)mod_m;
+  const int c19 = g.c19[mod];
+  const float mf = (float)mod_m, rmf = 1.0f / mf;
+  // m = 256 takes the low byte
+  auto smod = [&](int v) { return mod_m == 256 ? (int)(int8_t)v : smod_odd(v, c19, mf, rmf); };
   auto reduce = [&]() {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[i][j][r] = smod_i32(acc[i][j][r], mod_m, rmf);
+        for (int r = 0; r < 4; ++r) acc[i][j][r] = smod(acc[i][j][r]);
   };
   walk(0, min(kPiece, nslab), read, mul);
 #pragma unroll 1
@@ -227,9 +224,12 @@ __device__ __forceinline__ void crt_tile(const CrtLevelArgs &g, int mod, int row
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const int row = i * 16 + lane % 16, col = j * 16 + 4 * (lane >> 4);
-      uint32_t w = 0;
+      uint32_t b[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) w |= (uint32_t)(smod_i32(acc[i][j][r], mod_m, rmf) & 0xff) << (8 * r);
+      for (int r = 0; r < 4; ++r) b[r] = mod_m == 256 ? acc[i][j][r] : smod_odd(acc[i][j][r], c19, mf, rmf);
+      // their low bytes in order
+      const uint32_t w = __builtin_amdgcn_perm(__builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400),
+                                               __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400), 0x05040100);
       int8_t *o = out + (long)row * n + col;
       if (row < m_rem) {
         if (col + 3 < n_rem) {
@@ -269,7 +269,7 @@ const CrtConfig kCrt[] = {
     crt_config<64, 64, 2, 2, 3>(),
 };
 // By how many tiles all moduli give the CUs (13 moduli, device time): 256x256 from six a CU on
-// (4096^3, 13 a CU: 786 us against 854 on 128x128; 2000^3, 3.3 a CU: 143 against 116); 64x64 for
+// (4096^3, 13 a CU: 795 us against 854 on 128x128; 2000^3, 3.3 a CU: 143 against 116); 64x64 for
 // fewer than two 128x128 tiles a CU (100x130x70: 7.6 us against 12.5).
 int pick(long m, long n, int L) {
   const long cus = phpc_device().cus;
@@ -301,7 +301,11 @@ int phpc_crt_level(const int8_t *A8, const int8_t *B8, long kp, int m, int n, in
   g.L = L;
   g.tiles_m = (m + c.bm - 1) / c.bm;
   g.tiles_n = (n + c.bn - 1) / c.bn;
-  for (int t = 0; t < L; ++t) g.mods[t] = mods[t];
+  for (int t = 0; t < L; ++t) {
+    g.mods[t] = mods[t];
+    const int c = (1 << 19) % mods[t];
+    g.c19[t] = 2 * c > mods[t] ? c - mods[t] : c;
+  }
   const long total = (long)g.tiles_m * g.tiles_n * L;
   if (total > 0x7fffffffL) return phpc_set_error(PHPC_ERR_ARG, "too many tiles");
   g.window = 2 * phpc_device().cus;
