@@ -19,7 +19,6 @@ namespace {
 
 typedef int i4v __attribute__((ext_vector_type(4)));
 typedef float f16v __attribute__((ext_vector_type(16)));
-typedef float f4v __attribute__((ext_vector_type(4)));
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef unsigned int u4v __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
@@ -28,7 +27,7 @@ typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 // columns of B) x kFK k of one slice, 1 KiB, lane l's 16 bytes (row l % kMI, the 8 k from 8 (l /
 // kMI)) at 16 l; [row block][k block][slice] in memory. A load to LDS then moves one contiguous
 // KiB, and an operand read of LDS is linear in the lane: no swizzle, no bank conflicts.
-constexpr int kMI = 32, kFK = 512 / kMI;
+constexpr int kMI = 32, kFK = 16;
 constexpr int kBlock = 1024, kSlab = 3 * kBlock;
 
 __device__ __forceinline__ uint32_t bf16_rne(float x) {
@@ -147,8 +146,7 @@ struct Bf3Shape {
 template <int BM, int BN, int WM, int WN, int STAGES>
 __device__ __forceinline__ void bf3_tile(const Bf3Desc &d, int row0, int col0) {
   using K = Bf3Shape<BM, BN, WM, WN, STAGES>;
-  using acc_t = typename std::conditional<kMI == 32, f16v, f4v>::type;
-  constexpr int TM = K::TM, TN = K::TN, NR = kMI == 32 ? 16 : 4;
+  constexpr int TM = K::TM, TN = K::TN;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int wave = uni((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
@@ -236,11 +234,11 @@ __device__ __forceinline__ void bf3_tile(const Bf3Desc &d, int row0, int col0) {
     return;
   }
 
-  acc_t big[TM][TN], small[TM][TN];
+  f16v big[TM][TN], small[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) big[i][j] = small[i][j] = acc_t{};
+    for (int j = 0; j < TN; ++j) big[i][j] = small[i][j] = f16v{};
   i4v a[2][TM][3], b[2][TN][3];
   const int a0 = wm * TM * kSlab + lane * 16, b0 = K::B_BASE + wn * TN * kSlab + lane * 16;
   auto read = [&](auto stage, auto set) {
@@ -255,17 +253,13 @@ __device__ __forceinline__ void bf3_tile(const Bf3Desc &d, int row0, int col0) {
         b[x][j][p] = *reinterpret_cast<const i4v *>(smem + b0 + (q * K::B_BYTES + j * kSlab + p * kBlock));
     }
   };
-  auto product = [&](acc_t(&acc)[TM][TN], const i4v(&x)[TM][3], const i4v(&y)[TN][3], int p, int r) {
+  auto product = [&](f16v(&acc)[TM][TN], const i4v(&x)[TM][3], const i4v(&y)[TN][3], int p, int r) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
-        if constexpr (kMI == 32)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8v, x[i][p]),
-                                                              __builtin_bit_cast(bf8v, y[j][r]), acc[i][j], 0, 0, 0);
-        else
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8v, x[i][p]),
-                                                              __builtin_bit_cast(bf8v, y[j][r]), acc[i][j], 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8v, x[i][p]),
+                                                            __builtin_bit_cast(bf8v, y[j][r]), acc[i][j], 0, 0, 0);
   };
   auto mul = [&](auto set, auto steady) {
     constexpr int x = decltype(set)::value;
@@ -277,9 +271,8 @@ __device__ __forceinline__ void bf3_tile(const Bf3Desc &d, int row0, int col0) {
     product(small, a[x], b[x], 1, 0);
     if constexpr (decltype(steady)::value) {
       // the next slab's operand reads evenly between the MFMAs
-      constexpr int NRD = 3 * (TM + TN), NMF = 6 * TM * TN;
-      static_assert(NMF % NRD == 0 || NMF >= NRD || TM * TN == 1, "schedule");
-      constexpr int EACH = NMF / NRD > 0 ? NMF / NRD : 1;
+      constexpr int NRD = 3 * (TM + TN), NMF = 6 * TM * TN, EACH = NMF / NRD;
+      static_assert(EACH >= 1, "an MFMA for every read");
 #pragma unroll
       for (int r = 0; r < NRD; ++r) {
         __builtin_amdgcn_sched_group_barrier(0x008, EACH, 0);
@@ -290,7 +283,7 @@ __device__ __forceinline__ void bf3_tile(const Bf3Desc &d, int row0, int col0) {
   };
   walk(read, mul);
 
-  const CTile<float, acc_t, TM, TN, kMI, NR> ct(d.C + (long)wrow * d.ldc + wcol, d.ldc, d.m - wrow, d.n - wcol, lane);
+  const CTile<float, f16v, TM, TN, kMI, 16> ct(d.C + (long)wrow * d.ldc + wcol, d.ldc, d.m - wrow, d.n - wcol, lane);
   // in 64 bits, so that the two sums and C are rounded once
   ct.update([&](float c, int i, int j, int r) {
     return (float)((double)c + ((double)big[i][j][r] + (double)small[i][j][r]));

@@ -113,8 +113,8 @@ int launch(phpc_plan *p, hipStream_t s) {
     return phpc_f32_launch_direct(p->w32, p->descs_dev, p->grid, s);
   if (p->dtype == PHPC_F32X3 && p->config >= kF32X3PlanesConfig) return p->planes.run(s, p->grid);
   if (p->dtype == PHPC_F32X3)
-    return phpc_f32x3_launch((const F32Desc *)p->descs_dev, p->d32.data(), p->count, p->total_tiles, p->x3_tile, p->vec, p->grid,
-                             s);
+    return phpc_f32x3_launch((const F32Desc *)p->descs_dev, p->d32.data(), p->count, p->total_tiles, p->x3_tile, p->vec,
+                             p->grid, s);
   return phpc_f32_launch((const F32Desc *)p->descs_dev, p->d32.data(), p->count, p->total_tiles, p->config, p->vec,
                          p->grid, s);
 }
