@@ -801,7 +801,7 @@ def main():
             "tflops": round(exact_tf, 3),
             "roofline": {"bound": "mfma", "achieved": round(exact_kernel_tf, 3), "peak": FP64_PEAK_TFLOPS,
                          "unit": "TFLOP/s", "frac": round(exact_kernel_tf / FP64_PEAK_TFLOPS, 4),
-                         "kernel": "rm_kernel 128x128 with panels (16 waves, 64x64 tail tiles; per-panel sums "
+                         "kernel": "rm_kernel 192x128 with panels (8 waves, 64x64 tail tiles; per-panel sums "
                                    "added to the C carried in registers)",
                          "kernel_ms_avg": round(exact_kernel_ms, 3), "pass_ms_avg": round(exact_ms, 3)},
             "arithmetic": "bit-exact to the reference's per-panel grouping (src/phpc_summa.c:63-95)",

@@ -315,6 +315,7 @@ template <bool MP> using T128x64 = RmTile<double, 128, 64, 4, 2, 16, 3, MP>;    
 template <bool MP> using T128W8 = RmTile<double, 128, 128, 2, 4, 16, 4, MP>;    // 8 waves
 template <bool MP> using T128K32 = RmTile<double, 128, 128, 4, 4, 32, 2, MP>;   // 16 waves, two 32-deep stages
 template <bool MP> using T128 = RmTile<double, 128, 128, 4, 4, 16, 4, MP>;      // 16 waves
+template <bool MP> using T192 = RmTile<double, 192, 128, 4, 2, 16, 4, MP>;      // 8 waves, all of LDS
 template <bool MP> using T256W8 = RmTile<double, 256, 128, 4, 2, 16, 3, MP>;    // 8 waves
 template <bool MP> using T256 = RmTile<double, 256, 128, 4, 4, 16, 3, MP>;      // 16 waves
 
@@ -328,12 +329,12 @@ template <bool MP> using T256 = RmTile<double, 256, 128, 4, 4, 16, 3, MP>;      
    {{PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 1), PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 2)},                  \
     {PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 1), PHPC_V1(BM_, BN_, WM_, WN_, BK_, false, 2)}}, 0, 0}
 
-constexpr int kSmall = 13, kMid = 5, kBig = 11, kBigPanels = 16, kListPanels = 3, kOne = 10;  // the planner's
+constexpr int kSmall = 13, kMid = 5, kBig = 11, kBigPanels = 16, kOne = 10;  // the planner's
 const ConfigEntry kConfigs[] = {
     V1_CONFIG(128, 128, 2, 4, 16),             // 0: register-staged, 8 waves (wave tile 64x32)
     V1_CONFIG(128, 128, 2, 4, 32),             // 1: register-staged, 8 waves, 32-deep slabs
     V1_CONFIG(64, 64, 2, 2, 16),               // 2: register-staged, 4 waves (wave tile 32x32)
-    rm_config<T128W8, T128W8>(),               // 3: the planner's for large panel-grouped lists
+    rm_config<T128W8, T128W8>(),               // 3
     rm_config<T64W8, T64W8, true>(),           // 4: single panel only
     rm_config<T64, T32K32>(),                  // 5: the planner's for middle sizes
     V1_CONFIG_SP(256, 128, 4, 2, 16),          // 6: register-staged, 8 waves (wave tile 64x64); single panel only
@@ -346,7 +347,7 @@ const ConfigEntry kConfigs[] = {
     rm_config<T32, T32>(),                     // 13: the planner's for small work
     rm_config<T128, T128>(),                   // 14
     rm_config<T128K32, T128K32>(),             // 15
-    rm_config<T128, T64W16>(),                 // 16: the planner's for large panel-grouped work
+    rm_config<T192, T64W8>(),                  // 16: the planner's for large panel-grouped work
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 
@@ -387,8 +388,8 @@ bool has_panels(const GemmDesc &d) { return d.panel > 0 && d.panel < d.k; }
 
 // the planner's configurations, replaceable through phpc_set_tuning; -1: the planner's own
 // choice (config_for)
-int g_big_config = kListPanels;  // large panel-grouped work on device-resident lists
-int g_big_single = -1;           // large single-panel work on device-resident lists
+int g_big_config = kBigPanels;  // large panel-grouped work on device-resident lists
+int g_big_single = -1;          // large single-panel work on device-resident lists
 int g_big_single_host = kBig;
 int g_big_config_host = kBigPanels;
 int g_group_m = 8;
@@ -421,21 +422,26 @@ namespace {
 //     600 x 3000 x 900, 0.6 a CU, 92 against 79 on 32x32);
 //   then 64x64 tiles in 4 waves with a 32x32 tail (2048^3: 68 TFLOP/s against 54 on 32x32 alone);
 //   from two 256x128 tiles per CU on, those (4096^3: 73.2 against 68; 16384^3: 74.8 against 65
-//     on 64x64), or, with panels, 128x128 tiles, whose waves have room for the carried C. Large
-//     panel-grouped lists (plans) take 8 waves and no tail: where launches of several streams
-//     meet, 9602^3 on 4 x 2 ranks 26.4 ms against 27.9 on 16 waves with the tail, 10000^3 on 3 x 3
-//     31.4 against 31.7; alone on the GPU 26.7 against 26.0 and 31.1 against 30.0.
+//     on 64x64). With panels, from six 192x128 tiles per CU on (four of 128x128 in a list), those:
+//     the largest whose waves have room for accumulators and the carried C (16384^3 in panels of
+//     256 122.9 ms against 127.8 on 128x128 in 16 waves and 126.4 on 64x64; 6000^3, 5.9 a CU, 6.26
+//     against 6.47 and 6.28; 5000^3, 4.2 a CU, 3.81 against 3.83 and 3.69; 10000^3 on 3 x 3 ranks
+//     as a plan 29.4, 31.0 on 128x128 in 8 waves). They load less of L2 per output than any
+//     smaller tile, which counts where launches of several streams meet on the GPU: the plan
+//     29.7 against 31.4 there, and 35 on 64x64.
 int config_for(const GemmDesc *descs, int ndesc, bool device_list) {
-  long t64 = 0, t128 = 0, t256 = 0;
+  long t64 = 0, t128 = 0, t192 = 0, t256 = 0;
   bool mp = false;
   for (int i = 0; i < ndesc; ++i) {
     t64 += rm_tiles(descs[i], 64, 64);
     t128 += rm_tiles(descs[i], 128, 128);
+    t192 += rm_tiles(descs[i], 192, 128);
     t256 += rm_tiles(descs[i], 256, 128);
     mp |= has_panels(descs[i]);
   }
   const long cus = phpc_device().cus;
-  if (mp && t128 >= 4 * cus) return device_list && g_big_config >= 0 ? g_big_config : g_big_config_host;
+  if (mp && (device_list ? t128 >= 4 * cus : t192 >= 6 * cus))
+    return device_list && g_big_config >= 0 ? g_big_config : g_big_config_host;
   if (!mp && t256 >= 2 * cus) return device_list && g_big_single >= 0 ? g_big_single : g_big_single_host;
   if (!mp && 4 * t64 > 3 * cus && t64 <= cus) return kOne;
   return t64 >= cus ? kMid : kSmall;

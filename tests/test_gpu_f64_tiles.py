@@ -61,13 +61,15 @@ def panel_sums(A, B, C0, panel):
 # the tiles' edges, and an odd n whose last 16-byte piece would end past its row
 @pytest.mark.parametrize("cfg", DIRECT)
 @pytest.mark.parametrize("m,k,n", [(1, 1, 1), (31, 15, 33), (65, 16, 63), (129, 32, 127), (255, 33, 257),
-                                   (64, 160, 129), (257, 161, 65), (40, 400, 31)])
+                                   (64, 160, 129), (257, 161, 65), (40, 400, 31), (191, 47, 130),
+                                   (193, 64, 127), (400, 20, 129)])
 def test_tile_and_slab_edges(cfg, m, k, n):
     run(m, k, n, cfg)
 
 
 @pytest.mark.parametrize("cfg", PANELS)
-@pytest.mark.parametrize("m,k,n,panel", [(70, 130, 65, 16), (130, 200, 129, 33), (33, 300, 257, 64), (64, 97, 40, 96)])
+@pytest.mark.parametrize("m,k,n,panel", [(70, 130, 65, 16), (130, 200, 129, 33), (33, 300, 257, 64), (64, 97, 40, 96), (193, 70, 129, 48),
+                                         (385, 33, 127, 16)])
 def test_panel_edges(cfg, m, k, n, panel):
     run(m, k, n, cfg, panel)
 
@@ -75,7 +77,8 @@ def test_panel_edges(cfg, m, k, n, panel):
 # work that the planner cuts into head tiles and a tail of smaller ones: by rows, by columns,
 # on 64x64, 256x128 and (with panels) 128x128 heads, on 256 CUs
 @pytest.mark.parametrize("m,k,n,panel", [(1023, 33, 1000, 0), (961, 130, 1024, 0), (1023, 33, 1000, 9), (1100, 35, 1001, 0), (500, 40, 2301, 0), (1100, 35, 1001, 16),
-                                         (4100, 20, 4201, 0), (4200, 20, 4101, 7)])
+                                         (4100, 20, 4201, 0), (4200, 20, 4101, 7), (6200, 33, 6301, 16),
+                                         (6301, 20, 6200, 7)])
 def test_head_and_tail(m, k, n, panel):
     run(m, k, n, -1, panel)
 
