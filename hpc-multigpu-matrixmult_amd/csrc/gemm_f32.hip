@@ -475,10 +475,13 @@ int phpc_f32_plan_tiles(F32Desc *descs, int ndesc, int id) {
   return start;
 }
 
+// A load spans a_rows rows of A and b_rows of B. Rows of A that lie too far apart become products
+// of one row, lda = k (rm_split_rows), so of A it is k that has to fit.
 bool phpc_f32_direct_ok(const F32Desc *descs, int ndesc) {
   for (int i = 0; i < ndesc; ++i)
     for (const F32RmConfig &c : kF32Rm)
-      if ((long)c.b_rows * descs[i].ldb * 4 >= 0x7fffffffL) return false;
+      if ((long)c.a_rows * descs[i].k * 4 >= 0x7fffffffL || (long)c.b_rows * descs[i].ldb * 4 >= 0x7fffffffL)
+        return false;
   return true;
 }
 
