@@ -3,6 +3,7 @@
 #pragma once
 
 #include "phpc_internal.h"
+#include "rm_edges.h"
 
 #include <algorithm>
 #include <cstring>
@@ -286,9 +287,8 @@ struct RmElem<float> {
 //      an operand read (rows k, k+1, ...) use different banks.
 // A slab with fewer than BK k rows (the end of a panel) takes 4-byte loads into the same
 // layout, each checked against k, rows and columns, so padding is exact zeros in both
-// operands. So does the last slab of a GEMM whose n is no whole number of chunks and whose B
-// rows are not 16-byte aligned: there a 16-byte load of the last columns would read past the
-// last row's end.
+// operands. So do the slabs that hold the last rows of B where a 16-byte load of the last columns
+// would read past the last row's end (rm_checked_rows).
 //
 // What bounds it. An FP64 MFMA holds its SIMD's vector pipe for 64 cycles, an FP32 one for 32,
 // and a vector instruction of any kind waits for the MFMA before it to leave: one address
@@ -405,7 +405,10 @@ __device__ __forceinline__ void rm_tile(const Desc &d, int row0, int col0) {
     const int full_panels = MP ? Kdim / w : 1;
     const int nslab = MP ? uni(full_panels * spp + (Kdim - full_panels * w + BK - 1) / BK) : spp;
     const int last_panel = MP && Kdim % w ? Kdim % w : w;
-    const bool exact_last = d.n % CH && ((reinterpret_cast<uintptr_t>(Bg) / SZ | (uintptr_t)ldb) & (CH - 1));
+    // slabs that end past k16 take 4-byte loads
+    const int checked =
+        rm_checked_rows<CH>(d.n, ldb, !((reinterpret_cast<uintptr_t>(Bg) / SZ | (uintptr_t)ldb) & (CH - 1)));
+    const int k16 = Kdim - checked;
 
     // Every 1 KiB block is addressed from its own first row (ARB or BRB rows, uniform), so one
     // lane offset serves all of an operand's blocks. A rows past m_rem lie at or beyond
@@ -443,7 +446,7 @@ __device__ __forceinline__ void rm_tile(const Desc &d, int row0, int col0) {
     };
     auto issue = [&]() {
       const int krem = min(BK, ipe - ikb);
-      if (krem == BK && !(exact_last && ikb + BK >= Kdim)) {
+      if (krem == BK && ikb + BK <= k16) {
 #pragma unroll
         for (int u = 0; u < K::PER; ++u) load_block(u, istage);
       } else {
@@ -481,7 +484,8 @@ __device__ __forceinline__ void rm_tile(const Desc &d, int row0, int col0) {
 
     // every wave must be done reading the previous tile's stages before refilling them
     slab_barrier();
-    const int last_units = last_panel % BK || exact_last ? 3 : 0;  // extra loads of a last slab in 4-byte pieces
+    // extra loads of a last slab in 4-byte pieces (one before it, with ldb < CH, is waited for longer)
+    const int last_units = last_panel % BK || checked ? 3 : 0;
 #pragma unroll 1
     for (int s0 = 0; s0 < STAGES - 1 && s0 < nslab; ++s0) issue();
 
@@ -491,7 +495,6 @@ __device__ __forceinline__ void rm_tile(const Desc &d, int row0, int col0) {
       const int later = issued - 1 - t;
       wait_units<K::PER, STAGES + 1>(later > 0 && issued == nslab ? later + last_units : later);
     };
-    const int k16 = Kdim - (exact_last ? 1 : 0);  // a slab that ends past it takes 4-byte loads
     // walk the slabs, STAGES at a time while the slabs that they issue are full ones of one
     // panel; compute(stage, steady) is a slab's work behind its barrier
     auto walk = [&](auto compute) {

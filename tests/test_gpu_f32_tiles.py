@@ -106,3 +106,22 @@ def test_many_gemms_as_one_plan(shapes, dtype):
     for (_, _, C), w in zip(items, want):
         assert torch.equal(C, w)
     plan.close()
+
+
+# rows of B shorter than a 16-byte load, B ending where its rows end: the last slab, or the last two,
+# hold rows whose loads would reach past it
+@pytest.mark.parametrize("k", [33, 34, 35, 65, 66, 97, 129, 161, 290])
+@pytest.mark.parametrize("m,n", [(1, 1), (40, 1), (5, 2), (300, 3), (2000, 1), (70000, 1)])
+def test_short_rows_of_b(m, n, k):
+    import torch
+    A, B, C0 = inputs(m, k, n, 11 * m + k + n)
+    C = C0.clone()
+    phpc.sgemm_device(A, B, C, method=phpc.SGEMM_FP32)
+    torch.cuda.synchronize()
+    assert torch.equal(C, staged(A, B, C0)), (m, k, n)
+    if n == 1:  # a column of rows of two: ldb = 2
+        wide = torch.stack([B[:, 0], torch.full_like(B[:, 0], float("nan"))], dim=1)
+        D = C0.clone()
+        phpc.sgemm_device(A, wide[:, :1], D, method=phpc.SGEMM_FP32)
+        torch.cuda.synchronize()
+        assert torch.equal(D, C), (m, k, n)
