@@ -407,7 +407,7 @@ int launch(const Bf3Work &w, const void *list_dev, int grid, hipStream_t s) {
   b.tail_start = w.tail_start;
   b.d0 = w.descs[0];
   if (b.ndesc == 2) b.d1 = w.descs[1];
-  const int G = grid > 0 ? std::min(grid, w.total) : w.total;
+  const int G = rm_grid(grid, w.total, c.threads);
   const int kt = phpc_ktime_begin(s);
   hipLaunchKernelGGL(c.fn, dim3((unsigned)G), dim3(c.threads), c.lds, s, b);
   phpc_ktime_end(kt, s);

@@ -541,7 +541,7 @@ int phpc_f32_launch_direct(const F32Work &w, const void *list_dev, int grid, hip
   b.tail_start = w.tail_start;
   b.d0 = w.descs[0];
   if (b.ndesc == 2) b.d1 = w.descs[1];
-  const int G = grid > 0 ? std::min(grid, w.total) : w.total;
+  const int G = rm_grid(grid, w.total, c.threads);
   const int kt = phpc_ktime_begin(stream);
   hipLaunchKernelGGL(c.fn, dim3(G), dim3(c.threads), c.lds_bytes, stream, b);
   phpc_ktime_end(kt, stream);

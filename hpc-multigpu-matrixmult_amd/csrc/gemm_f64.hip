@@ -503,13 +503,10 @@ int phpc_f64_launch(const F64Work &w, const void *list_dev, int grid, hipStream_
   b.tail_start = w.tail_start;
   b.d0 = w.descs[0];
   if (b.ndesc == 2) b.d1 = w.descs[1];
-  int G = grid;
-  if (G <= 0) {
-    // the row-major kernels leave it to the dispatcher to hand out tiles, so that a CU whose
-    // tiles end early takes the next one; the register-staged ones walk a persistent grid
-    G = ce.lds_bytes ? w.total : occupancy(w.config, w.mp, w.vec2) * phpc_device().cus;
-    if (G > w.total) G = w.total;
-  }
+  // the row-major kernels leave it to the dispatcher to hand out tiles, so that a CU whose
+  // tiles end early takes the next one; the register-staged ones walk a persistent grid
+  if (grid <= 0) grid = ce.lds_bytes ? 0 : occupancy(w.config, w.mp, w.vec2) * phpc_device().cus;
+  const int G = rm_grid(grid, w.total, ce.threads);
   {
     std::lock_guard<std::mutex> lk(g_mu);
     init_kernels_locked();

@@ -19,3 +19,13 @@ RM_BOTH int rm_checked_rows(int n, long ldb, bool aligned) {
   if (over == 0 || aligned) return 0;
   return over <= ldb ? 1 : over <= 2 * ldb ? 2 : 3;
 }
+
+// Workgroups of a launch over `total` tiles: `wanted` of them, or, at 0, one per tile. HIP launches
+// fewer than 2^32 threads in one dimension, which a column of more than 2^30 rows would exceed
+// (256 rows a tile, 1024 threads): then as many as there can be, a whole number of them on each of
+// the 8 XCDs, walk the tiles.
+inline int rm_grid(int wanted, int total, int threads) {
+  const int most = (int)(0xffffffffu / (unsigned)threads / 8 * 8);
+  const int g = wanted > 0 && wanted < total ? wanted : total;
+  return g < most ? g : most;
+}

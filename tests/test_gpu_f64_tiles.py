@@ -122,3 +122,21 @@ def test_rows_of_a_far_apart(dtype, lda):
     torch.cuda.synchronize()
     plan.close()
     assert torch.equal(C, want) and torch.equal(D, want) and torch.equal(E, want)
+
+
+# a column of so many rows that a workgroup per tile would take 2^32 threads
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_more_tiles_than_one_launch_starts(dtype):
+    import torch
+    m = 2 ** 30 + 777
+    t = torch.float64 if dtype == "f64" else torch.float32
+    A, C = torch.empty(m, 1, dtype=t, device="cuda"), torch.ones(m, 1, dtype=t, device="cuda")
+    A[:, 0] = torch.arange(m, device="cuda") % 1021
+    B = torch.full((1, 1), 3.0, dtype=t, device="cuda")
+    if dtype == "f64":
+        phpc.dgemm_device(A, B, C)
+    else:
+        phpc.sgemm_device(A, B, C, method=phpc.SGEMM_FP32)
+    torch.cuda.synchronize()
+    A.mul_(3.0).add_(1.0)
+    assert torch.equal(A, C)

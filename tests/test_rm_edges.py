@@ -46,3 +46,30 @@ def run(tmp_path, text):
 
 def test_no_load_of_b_leaves_its_memory(tmp_path):
     run(tmp_path, LOADS)
+
+
+GRIDS = r'''
+#include "rm_edges.h"
+#include <cstdio>
+int main() {
+  const int totals[] = {1, 7, 255, 256, 100000, 4194303, 4194304, 8388609, 16777216, 33554433, 2147483647};
+  const int wanted[] = {0, 1, 5, 512, 4194304, 20000000, 2147483647};
+  for (int threads = 256; threads <= 1024; threads *= 2)
+    for (int total : totals)
+      for (int want : wanted) {
+        const int g = rm_grid(want, total, threads);
+        const bool capped = want > 0 && want < total ? g < want : g < total;
+        if (g < 1 || g > total || (want > 0 && g > want) || (long)g * threads >= 1L << 32 || (capped && g % 8) ||
+            (capped && (long)(g + 8) * threads < 1L << 32)) {
+          printf("total %d wanted %d threads %d: %d\n", total, want, threads, g);
+          return 1;
+        }
+      }
+  printf("ok\n");
+  return 0;
+}
+'''
+
+
+def test_launches_stay_below_two_to_the_32_threads(tmp_path):
+    run(tmp_path, GRIDS)
