@@ -386,10 +386,9 @@ int occupancy(int cfg, int mp, int vec2) {
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 bool has_panels(const GemmDesc &d) { return d.panel > 0 && d.panel < d.k; }
 
-// the planner's configurations, replaceable through phpc_set_tuning; -1: the planner's own
-// choice (config_for)
-int g_big_config = kBigPanels;  // large panel-grouped work on device-resident lists
-int g_big_single = -1;          // large single-panel work on device-resident lists
+// the planner's configurations for large work, replaceable through phpc_set_tuning
+int g_big_config = kBigPanels;  // panel-grouped, on device-resident lists
+int g_big_single = kBig;        // single-panel, on device-resident lists
 int g_big_single_host = kBig;
 int g_big_config_host = kBigPanels;
 int g_group_m = 8;
@@ -441,8 +440,9 @@ int config_for(const GemmDesc *descs, int ndesc, bool device_list) {
   }
   const long cus = phpc_device().cus;
   if (mp && (device_list ? t128 >= 4 * cus : t192 >= 6 * cus))
-    return device_list && g_big_config >= 0 ? g_big_config : g_big_config_host;
-  if (!mp && t256 >= 2 * cus) return device_list && g_big_single >= 0 ? g_big_single : g_big_single_host;
+    // key 0 may hold a configuration without panel-grouped variants
+    return !device_list ? g_big_config_host : kConfigs[g_big_config].panels ? g_big_config : kBigPanels;
+  if (!mp && t256 >= 2 * cus) return device_list ? g_big_single : g_big_single_host;
   if (!mp && 4 * t64 > 3 * cus && t64 <= cus) return kOne;
   return t64 >= cus ? kMid : kSmall;
 }
@@ -553,14 +553,15 @@ int phpc_f64_grouped(const GemmDesc *descs, int ndesc, int grid, int config_id, 
 }
 
 // Tuning knobs for the autotuner: 0 = config for large panel-grouped problems on device
-// descriptors, 1 = tile-row swizzle width, 2 = XCD-contiguous tile order on/off, 3 = config
-// for large single-panel problems on device descriptors, 4 = the same through host
-// descriptors, 5 = large panel-grouped problems through host descriptors.
+// descriptors (one without panel-grouped variants leaves the default), 1 = tile-row swizzle
+// width, 2 = XCD-contiguous tile order on/off, 3 = config for large single-panel problems on
+// device descriptors, 4 = the same through host descriptors, 5 = large panel-grouped problems
+// through host descriptors.
 extern "C" int phpc_set_tuning(int key, int value) {
   switch (key) {
     case 0:
     case 3:
-      if (value < 0 || value >= 10) return phpc_set_error(PHPC_ERR_ARG, "config %d out of range", value);
+      if (value < 0 || value >= kNumConfigs) return phpc_set_error(PHPC_ERR_ARG, "config %d out of range", value);
       (key == 0 ? g_big_config : g_big_single) = value;
       break;
     case 1:

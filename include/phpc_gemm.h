@@ -85,16 +85,17 @@ int phpc_dgemm_vendor_device(const double *dA, long lda, const double *dB, long 
  */
 int phpc_set_launch_policy(int honor_grid, int config_id, int grid);
 int phpc_num_configs(void);
-/* Tuning knobs used by the autotuner: key 0 = FP64 config for large panel-grouped
- * problems on device-resident descriptor lists (plans fall back to it), key 1 = tile-row
- * swizzle width (1..64), key 2 = XCD-contiguous tile order (0/1), key 3 = FP64 config for
- * large single-panel problems on device-resident descriptor lists (keys 0 and 3 take configs
- * 0-9), key 4 / key 5 = FP64 config for large single-panel / panel-grouped problems, key 6 =
- * FP32 products through phpc_sgemm_device on the direct-to-LDS FP32 kernels (1, default) or
- * on the register-staged ones (0); 0 also keeps FP32 plans created without autotuning off
- * configuration 3; key 7 = FP32 configuration of plans created without autotuning (-1,
- * default = 3; 0-2 = register-staged 64x64, 128x64, 128x128; 3 = the direct-to-LDS kernels
- * on tiles picked by the work; all give the same bits); key 8 = configuration of 3 x BF16 (PHPC_F32X3) plans
+/* Tuning knobs used by the autotuner: key 0 / key 3 = FP64 config for large panel-grouped /
+ * single-panel problems on device-resident descriptor lists, that is plans created without
+ * autotuning (defaults 16 and 11; a config without panel-grouped variants leaves key 0's
+ * default in force), key 4 / key 5 = FP64 config for large single-panel / panel-grouped
+ * problems through the other entry points (defaults 11 and 16), key 1 = tile-row swizzle
+ * width (1..64), key 2 = XCD-contiguous tile order (0/1), key 6 = FP32 products through
+ * phpc_sgemm_device on the direct-to-LDS FP32 kernels (1, default) or on the register-staged
+ * ones (0); 0 also keeps FP32 plans created without autotuning off configuration 3; key 7 =
+ * FP32 configuration of plans created without autotuning (-1, default = 3; 0-2 =
+ * register-staged 64x64, 128x64, 128x128; 3 = the direct-to-LDS kernels on tiles picked by
+ * the work; all give the same bits); key 8 = configuration of 3 x BF16 (PHPC_F32X3) plans
  * created without autotuning (-1 = by work, default: 2 for fewer 64x64 tiles than CUs, 6 for at
  * least two 128x128 tiles per CU, else 4; 2 = BF16 slices cut in registers; 4, 5, 6 = BF16 slice
  * planes cut once per operand, then one grouped launch on 64x64, 256x128 or 128x128 tiles, the
