@@ -451,6 +451,7 @@ int phpc_sgemm_bf16x3_planes(const float *dA, long lda, const float *dB, long ld
 // ---------------------------------------------------------------------------
 int phpc_bf3_num_configs() { return kNumGroup; }
 bool phpc_bf3_fits(long k) { return planes_fit(k); }
+size_t phpc_bf3_plane_bytes(long rows, long k) { return plane_bytes(rows, k); }
 
 int phpc_f32x3_set_plan_config(int id) {
   if (id != -1 && id != 2 && (id < kF32X3PlanesConfig || id >= kF32X3PlanesConfig + kNumGroup))

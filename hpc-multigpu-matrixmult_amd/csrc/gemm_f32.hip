@@ -449,6 +449,33 @@ const F32RmConfig kF32Rm[] = {
 };
 std::once_flag g_rm_once;
 
+// The planes of 3 x BF16 products. Large products share one workspace, which a captured one refers
+// to from then on. Smaller ones must not move it: they have four of their own, each stream keeping
+// to one while there are no more than four, so that products on different streams run side by
+// side. Planes of more than kWayBytes an operand go to the first, so that the others together
+// stay below 3 GiB.
+struct X3Workspaces {
+  static constexpr int kWays = 4;
+  static constexpr size_t kWayBytes = 512u << 20;
+  SharedWorkspace large, way[kWays];
+  SharedWorkspace &of(hipStream_t s, size_t bytes) {
+    if (bytes > kWayBytes) return way[0];
+    std::lock_guard<std::mutex> lk(mu);
+    for (int i = 0; i < used; ++i)
+      if (user[i] == s) return way[i];
+    const int i = next;
+    next = (next + 1) % kWays;
+    used = std::max(used, i + 1);
+    user[i] = s;
+    return way[i];
+  }
+
+ private:
+  std::mutex mu;
+  hipStream_t user[kWays] = {};
+  int used = 0, next = 0;
+};
+
 }  // namespace
 
 static_assert(kF32DirectConfig == kNumF32, "the direct kernels follow the register-staged ones");
@@ -646,9 +673,9 @@ extern "C" int phpc_sgemm_device(const float *dA, long lda, const float *dB, lon
   const bool large = (long)m * n >= 2048L * 2048 && k >= 256;
   if (method == PHPC_SGEMM_BF16X3) {
     // Slice planes from one 64x64 tile per CU on: 1000^3 29 us against 40 on the in-register
-    // kernel, 1500^3 57 against 88; at 512^3, 18 against 21, the one launch that needs no shared
-    // workspace lets products on several streams run side by side. A stream being captured takes
-    // the workspace (which may grow, and waits for its last user) only where it always did.
+    // kernel, 1500^3 57 against 88; at 512^3, 18 against 21, the one launch that needs no
+    // workspace is the simpler. A stream being captured takes a workspace (which may grow, and
+    // waits for its last user) only where it always did.
     planes = large;
     if (!large && (long)((m + 63) / 64) * ((n + 63) / 64) >= phpc_device().cus && k >= 128 && phpc_bf3_fits(k)) {
       hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -659,7 +686,9 @@ extern "C" int phpc_sgemm_device(const float *dA, long lda, const float *dB, lon
   }
   if (planes) {
     // slice planes cut once, then multiplied on the direct-to-LDS pipeline
-    static SharedWorkspace ws;
+    static X3Workspaces all;
+    SharedWorkspace &ws =
+        large ? all.large : all.of((hipStream_t)stream, std::max(phpc_bf3_plane_bytes(m, k), phpc_bf3_plane_bytes(n, k)));
     std::lock_guard<std::mutex> lk(ws.mu);
     ws.after_previous((hipStream_t)stream);
     rc = phpc_sgemm_bf16x3_planes(dA, lda, dB, ldb, dC, ldc, m, k, n, (hipStream_t)stream, &ws.ws);

@@ -107,6 +107,7 @@ bool phpc_f32_vec4_ok(const F32Desc *descs, int ndesc);
 constexpr int kF32X3PlanesConfig = 4;
 int phpc_bf3_num_configs();
 bool phpc_bf3_fits(long k);  // a plane row of k fits the kernel's 32-bit offsets
+size_t phpc_bf3_plane_bytes(long rows, long k);  // of one operand's planes
 // configuration of 3 x BF16 plans created without autotuning: -1 = by work, 2 (the in-register
 // kernel) or kF32X3PlanesConfig + g
 int phpc_f32x3_set_plan_config(int id);

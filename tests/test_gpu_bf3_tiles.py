@@ -131,3 +131,54 @@ def test_captured_product_takes_no_workspace():
         check(A, B, C0, C)
         first = C.clone() if first is None else first
         assert torch.equal(C, first)
+
+
+def test_smaller_products_leave_a_captured_large_one_alone():
+    """A captured large product keeps its planes: eager products below its size, with planes larger
+    than all before, run between its replays."""
+    import torch
+    A, B, C0 = inputs(2048, 256, 2048, 1)
+    C, want = C0.clone(), C0.clone()
+    phpc.sgemm_device(A, B, want, method=phpc.SGEMM_BF16X3)  # allocates the planes
+    s = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        phpc.sgemm_device(A, B, C, method=phpc.SGEMM_BF16X3)
+    held = []
+    for rep in range(3):
+        C.copy_(C0)
+        X, Y, Z = inputs(1500, 2000 * (rep + 1), 1500, rep)
+        Z0 = Z.clone()
+        phpc.sgemm_device(X, Y, Z, method=phpc.SGEMM_BF16X3)
+        held.append(torch.full((4 << 20,), float("nan"), device="cuda"))  # would take freed planes' place
+        torch.cuda.synchronize()
+        check(X, Y, Z0, Z)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C, want)
+
+
+def test_products_on_several_streams():
+    """More streams than workspaces, two rounds, planes of several sizes, one stream's beyond the
+    size that goes to the first workspace."""
+    import torch
+    shapes = [(1500, 300, 1500), (1100, 700, 1000), (1024, 1024, 1024), (1300, 140, 1700), (1025, 2000, 1030),
+              (1500, 64000, 1500)]
+    ops = [inputs(*sh, seed=i) for i, sh in enumerate(shapes)]
+    alone = []
+    for A, B, C0 in ops:
+        C = C0.clone()
+        phpc.sgemm_device(A, B, C, method=phpc.SGEMM_BF16X3)
+        torch.cuda.synchronize()
+        alone.append(C)
+    streams = [torch.cuda.Stream() for _ in ops]
+    outs = [[C0.clone() for _, _, C0 in ops] for _ in range(2)]
+    torch.cuda.synchronize()
+    for out in outs:
+        for s, (A, B, _), C in zip(streams, ops, out):
+            phpc.sgemm_device(A, B, C, method=phpc.SGEMM_BF16X3, stream=s)
+    torch.cuda.synchronize()
+    for out in outs:
+        for C, want in zip(out, alone):
+            assert torch.equal(C, want)
