@@ -6,7 +6,7 @@
 // small ones into a second, both added to C in 64 bits at the end; the dropped ones are below
 // 2^-23 |a||b|. One kernel cuts every operand into planes; one launch then multiplies. Error
 // against 64 bits (2-norm, uniform inputs): 4096^3 3.75e-7 (3.74e-7 with one accumulator over
-// all six), 1500^3 2.1e-7 (5.9e-7 in the in-register kernel that it took before).
+// all six), 1500^3 2.1e-7 (5.9e-7 with one in the in-register kernel before).
 #include "gemm_rm.h"
 #include "phpc_internal.h"
 #include "phpc_split.h"

@@ -207,7 +207,8 @@ __global__ __launch_bounds__(256) void f32_gemm_kernel(F32Batch batch) {
 // |lo| <= 2^-16|x|; with round-to-nearest the remainder after two slices has at most 8
 // significant bits, so lo is exact for finite inputs whose slices stay normal). The six
 // products with slice indices summing to at most 2 (hi.hi, hi.mid, mid.hi, hi.lo,
-// mid.mid, lo.hi) run on the BF16 matrix cores with FP32 accumulation; the dropped
+// mid.mid, lo.hi) run on the BF16 matrix cores, hi.hi into one FP32 accumulator, the five
+// small ones into a second, both added to C in 64 bits at the end; the dropped
 // mid.lo, lo.mid and lo.lo terms are below 2^-23 |a||b|. The result carries the error
 // of an FP32 dot product: |C - exact| <= ((k + 2) 2^-24 + 2^-23) (|C0| + |A||B|).
 //
@@ -225,18 +226,21 @@ __device__ __forceinline__ uint32_t bf16_rne(float x) {
 }
 __device__ __forceinline__ float bf16_val(uint32_t h) { return __uint_as_float(h << 16); }
 
-//
-// For products too small for the slice planes of gemm_bf3.hip. waves_per_eu(2) keeps the
-// accumulators where the MFMAs take them.
-template <int BM, int BN, int VEC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f32x3_gemm_kernel(F32Batch batch) {
+// For products too small for the slice planes of gemm_bf3.hip, and where these cannot be had (a
+// stream being captured, no memory): the same products in the same order, so the same sums.
+// Bound by the cut in registers and the barriers of a slab: 1500^3 87 us, 57 on planes; 8192 x 64 x 8192 144 us, C alone 112 at a copy's rate. Tiles of 128x128 in
+// 8 waves (in 4 the two accumulators spill: 4096 x 128 x 4096 81 us against 52). waves_per_eu(2)
+// keeps the accumulators where the MFMAs take them.
+template <int BM, int BN, int WN, int VEC>
+__global__ __launch_bounds__(128 * WN) __attribute__((amdgpu_waves_per_eu(2))) void f32x3_gemm_kernel(F32Batch batch) {
+  constexpr int NT = 128 * WN;  // 2 x WN waves
   constexpr int BK = 32;
   constexpr int KP = BK + 8;  // bf16 per LDS row (80 bytes: 16-byte aligned, staggered banks)
-  constexpr int WTM = BM / 2, WTN = BN / 2;
+  constexpr int WTM = BM / 2, WTN = BN / WN;
   constexpr int TM = WTM / 32, TN = WTN / 32;
-  constexpr int AE = BM * BK / 256;  // A floats per thread
-  constexpr int BE = BN * BK / 256;  // B floats per thread
-  static_assert(BM == BN && AE % 8 == 0 && TM >= 1, "thread mapping");
+  constexpr int AE = BM * BK / NT;  // A floats per thread
+  constexpr int BE = BN * BK / NT;  // B floats per thread
+  static_assert(BM == BN && AE % 8 == 0 && TM >= 1 && TN >= 1, "thread mapping");
   __shared__ __attribute__((aligned(16))) unsigned short lds[3 * BM * KP + 3 * BN * KP];
   unsigned short *Al = lds;
   unsigned short *Bl = lds + 3 * BM * KP;
@@ -244,7 +248,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   const int tid = threadIdx.x;
   const int wave = uni(tid >> 6);
   const int lane = tid & 63;
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / WN, wn = wave % WN;
   const int G = gridDim.x, bid = blockIdx.x;
   const int slot = uni((G % 8) == 0 ? (bid % 8) * (G / 8) + bid / 8 : bid);
   // AE consecutive k of one row of A, BE of one column of B per thread
@@ -262,14 +266,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
     const long lda = d.lda, ldb = d.ldb, ldc = d.ldc;
     const float *Ag = d.A + (long)row0 * lda;
     const float *Bg = d.B + col0;
-    gfloat *Cg = (gfloat *)(d.C + (long)row0 * ldc + col0);
     const rsrc_t rA = make_rsrc(Ag, (long)min(m_rem, BM) * lda * 4);
 
-    f16v acc[TM][TN];
+    f16v big[TM][TN], small[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = f16v{};
+      for (int j = 0; j < TN; ++j) big[i][j] = small[i][j] = f16v{};
 
     float ra[AE], rb[BE];
     auto load = [&](int kb) {
@@ -344,35 +347,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
           for (int p = 0; p < 3; ++p)
             b[j][p] = __builtin_bit_cast(
                 bf8v, *(const us8v *)(Bl + p * BN * KP + (wn * WTN + j * 32 + (lane & 31)) * KP + ko));
+        // each accumulator's order is that of the planes' kernel
+        auto product = [&](f16v(&acc)[TM][TN], int p, int r) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+          for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            // small terms first
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][2], b[j][0], acc[i][j], 0, 0, 0);
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][1], b[j][1], acc[i][j], 0, 0, 0);
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][0], b[j][2], acc[i][j], 0, 0, 0);
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][1], b[j][0], acc[i][j], 0, 0, 0);
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][0], b[j][1], acc[i][j], 0, 0, 0);
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][0], b[j][0], acc[i][j], 0, 0, 0);
-          }
+            for (int j = 0; j < TN; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][p], b[j][r], acc[i][j], 0, 0, 0);
+        };
+        product(small, 0, 2);
+        product(small, 1, 1);
+        product(small, 2, 0);
+        product(big, 0, 0);
+        product(small, 0, 1);
+        product(small, 1, 0);
       }
     }
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int cc = wn * WTN + j * 32 + (lane & 31);
-        if (cc >= n_rem) continue;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int rr = wm * WTM + i * 32 + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4);
-          if (rr < m_rem) {
-            gfloat *pc = Cg + (long)rr * ldc + cc;
-            *pc = *pc + acc[i][j][r];
-          }
-        }
-      }
+    const int wrow = wm * WTM, wcol = wn * WTN;
+    if (wrow < m_rem && wcol < n_rem) {
+      const CTile<float, f16v, TM, TN, 32, 16> ct(d.C + (long)(row0 + wrow) * ldc + col0 + wcol, ldc, m_rem - wrow,
+                                                  n_rem - wcol, lane);
+      ct.update([&](float c, int i, int j, int r) {
+        return (float)((double)c + ((double)big[i][j][r] + (double)small[i][j][r]));
+      });
+    }
     __syncthreads();  // LDS is rewritten by the next tile
   }
 }
@@ -593,9 +591,10 @@ int phpc_f32x3_launch(const F32Desc *descs_dev, const F32Desc *descs_host, int n
     if (128L * d.lda * 4 >= 0x7fffffffL || 32L * d.ldb * 4 >= 0x7fffffffL)
       return phpc_set_error(PHPC_ERR_ARG, "leading dimension too large");
   }
-  static void (*const kernels[2][2])(F32Batch) = {{f32x3_gemm_kernel<64, 64, 1>, f32x3_gemm_kernel<64, 64, 4>},
-                                                  {f32x3_gemm_kernel<128, 128, 1>, f32x3_gemm_kernel<128, 128, 4>}};
+  static void (*const kernels[2][2])(F32Batch) = {{f32x3_gemm_kernel<64, 64, 2, 1>, f32x3_gemm_kernel<64, 64, 2, 4>},
+                                                  {f32x3_gemm_kernel<128, 128, 4, 1>, f32x3_gemm_kernel<128, 128, 4, 4>}};
   void (*fn)(F32Batch) = kernels[config == 2][vec4];
+  const int threads = config == 2 ? 512 : 256;
   int occ;
   {
     static int occ_cache[2][2] = {};
@@ -603,7 +602,7 @@ int phpc_f32x3_launch(const F32Desc *descs_dev, const F32Desc *descs_host, int n
     int &cached = occ_cache[config == 2][vec4];
     if (cached == 0) {
       int n = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(fn), 256, 0) != hipSuccess ||
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(fn), threads, 0) != hipSuccess ||
           n < 1)
         n = 1;
       cached = n;
@@ -618,7 +617,7 @@ int phpc_f32x3_launch(const F32Desc *descs_dev, const F32Desc *descs_host, int n
   int G = grid > 0 ? grid : occ * phpc_device().cus;
   if (G > total_tiles) G = total_tiles;
   if (G < 1) G = 1;
-  hipLaunchKernelGGL(fn, dim3(G), dim3(256), 0, stream, b);
+  hipLaunchKernelGGL(fn, dim3(G), dim3(threads), 0, stream, b);
   PHPC_HIP(hipGetLastError());
   return PHPC_OK;
 }

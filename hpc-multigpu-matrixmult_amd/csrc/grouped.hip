@@ -76,7 +76,7 @@ int plan_upload(phpc_plan *p, int id, hipStream_t s) {
     return PHPC_OK;
   } else {
     // the in-register 3 x BF16 kernel takes 128x128 tiles (config 2's) from one a CU on, else
-    // 64x64 (config 0's): 512^3 21 us against 47
+    // 64x64 (config 0's): 512^3 23 us, 50 on 128x128 tiles of 4 waves
     p->total_tiles = phpc_f32_plan_tiles(p->d32.data(), p->count, p->dtype == PHPC_F32X3 ? 2 : id);
     p->x3_tile = 2;
     if (p->dtype == PHPC_F32X3 && p->total_tiles < phpc_device().cus) {

@@ -99,7 +99,7 @@ int phpc_num_configs(void);
  * created without autotuning (-1 = by work, default: 2 for fewer 64x64 tiles than CUs, 6 for at
  * least two 128x128 tiles per CU, else 4; 2 = BF16 slices cut in registers; 4, 5, 6 = BF16 slice
  * planes cut once per operand, then one grouped launch on 64x64, 256x128 or 128x128 tiles, the
- * plan keeping the planes; configurations 4, 5 and 6 give the same bits). */
+ * plan keeping the planes; all give the same bits). */
 int phpc_set_tuning(int key, int value);
 /* Describe configuration `id`: macro tile bm x bn, threads per workgroup. */
 int phpc_config_info(int id, int *bm, int *bn, int *threads);

@@ -182,3 +182,35 @@ def test_products_on_several_streams():
     for out in outs:
         for C, want in zip(out, alone):
             assert torch.equal(C, want)
+
+
+# one call, one result: the in-register kernel (64x64 and 128x128 tiles, 16-byte and 4-byte loads)
+# sums as the planes' does
+@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (31, 15, 33), (65, 33, 127), (128, 200, 64), (300, 1000, 500),
+                                   (1025, 130, 1023), (2048, 96, 2048), (2101, 161, 2303)])
+def test_in_register_bits_are_the_planes(m, k, n):
+    import torch
+    A, B, C0 = inputs(m, k, n, 5 * m + n)
+    out = []
+    for cfg in (2, 4):
+        C = C0.clone()
+        run_plan(cfg, [(A, B, C)])
+        out.append(C.view(torch.int32))
+    assert torch.equal(*out)
+
+
+@pytest.mark.parametrize("m,k,n", [(1100, 300, 1000), (2000, 257, 2001)])
+def test_captured_bits_are_the_eager(m, k, n):
+    import torch
+    A, B, C0 = inputs(m, k, n, m)
+    want, C = C0.clone(), C0.clone()
+    phpc.sgemm_device(A, B, want, method=phpc.SGEMM_BF16X3)
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        phpc.sgemm_device(A, B, C, method=phpc.SGEMM_BF16X3)
+    for _ in range(3):
+        C.copy_(C0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C.view(torch.int32), want.view(torch.int32))
