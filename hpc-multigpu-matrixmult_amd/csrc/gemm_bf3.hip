@@ -463,15 +463,24 @@ int phpc_f32x3_set_plan_config(int id) {
 int phpc_f32x3_pick_plan_config(const F32Desc *descs, int ndesc) {
   if (g_f32x3_plan_cfg >= 0) return g_f32x3_plan_cfg;
   // The in-register kernel where the items give fewer 64x64 tiles than CUs (one launch instead
-  // of two); else planes, on 128x128 tiles with a 64x64 tail from two a CU on: 512 products
-  // log-uniform in [64, 4096] 7.4 ms, 8.3 on 64x64 tiles, 7.8 on 256x128.
+  // of two), and where most of the work is in items of no more than 256 rows or columns, whose
+  // planes are little used (512 of 256 x 128 x 256 123 us against 174, 24 of 100 x 1024 x 8192 408
+  // against 693; 100 of [64, 1024] 186 against 143, 64 of 1000 x 256 x 1000 344 against 308); else
+  // planes, on 128x128 tiles with a 64x64 tail from two a CU on: 512 products log-uniform in [64,
+  // 4096] 7.4 ms, 8.3 on 64x64 tiles, 7.8 on 256x128.
   long t64 = 0, t128 = 0;
+  double all = 0, narrow = 0;
+  bool ok = true;
   for (int i = 0; i < ndesc; ++i) {
-    t64 += rm_tiles(descs[i], 64, 64);
-    t128 += rm_tiles(descs[i], 128, 128);
+    const F32Desc &d = descs[i];
+    t64 += rm_tiles(d, 64, 64);
+    t128 += rm_tiles(d, 128, 128);
+    all += (double)d.m * d.n * d.k;
+    if (std::min(d.m, d.n) <= 256) narrow += (double)d.m * d.n * d.k;
+    ok &= phpc_f32x3_in_register_ok(d);
   }
   const long cus = phpc_device().cus;
-  return t64 < cus ? 2 : kF32X3PlanesConfig + (t128 >= 2 * cus ? kT128 : kT64);
+  return t64 < cus || (ok && 2 * narrow > all) ? 2 : kF32X3PlanesConfig + (t128 >= 2 * cus ? kT128 : kT64);
 }
 
 int Bf3Planes::build(const F32Desc *descs, int ndesc, int gcfg) {

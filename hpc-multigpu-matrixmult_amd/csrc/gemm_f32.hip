@@ -582,15 +582,57 @@ bool phpc_f32_vec4_ok(const F32Desc *descs, int ndesc) {
   return true;
 }
 
-// FP32-accurate 3 x BF16 kernel on the tiles of configuration 0 (64 x 64) or 2 (128 x 128).
-int phpc_f32x3_launch(const F32Desc *descs_dev, const F32Desc *descs_host, int ndesc, int total_tiles, int config,
-                      bool vec4, int grid, hipStream_t stream) {
-  if (ndesc <= 0 || total_tiles <= 0) return PHPC_OK;
-  for (int i = 0; i < ndesc; ++i) {
-    const F32Desc &d = descs_host[i];
-    if (128L * d.lda * 4 >= 0x7fffffffL || 32L * d.ldb * 4 >= 0x7fffffffL)
-      return phpc_set_error(PHPC_ERR_ARG, "leading dimension too large");
+namespace {
+// The in-register 3 x BF16 kernel's tiles: configuration 0's (64x64) or 2's (128x128). A CU holds
+// four workgroups of 64x64 or one of 128x128. Measured at k = 512, by tiles a CU: 64x64 24 us for
+// one, 29 for two, 36 for three, 46 for four, 80 for five; 128x128 36 for one (as for fewer), 67
+// for two, 100 for three. So 128x128 from more than three 64x64 tiles a CU on, where it does not
+// take more than 4 / 3 of the rounds (64 x 512 x 100000, four rounds of 128x128 for two of 64x64:
+// 123 us against 86; 100 x 512 x 40000, two each: 68 against 82).
+int x3_tile(const std::vector<F32Desc> &descs) {
+  long t64 = 0, t128 = 0;
+  for (const F32Desc &d : descs) {
+    t64 += rm_tiles(d, 64, 64);
+    t128 += rm_tiles(d, 128, 128);
   }
+  const long cus = phpc_device().cus;
+  return t64 > 3 * cus && 3 * ((t128 + cus - 1) / cus) <= 4 * ((t64 + 4 * cus - 1) / (4 * cus)) ? 2 : 0;
+}
+}  // namespace
+
+// 128x128 tiles in whole rounds, and what would leave their last round nearly empty in a second
+// launch of its own tiles (100 x 4096 x 40000, 313 tiles of 128x128: 445 us, 380 so).
+void phpc_f32x3_prepare(const F32Desc *descs, int ndesc, F32X3Work *w) {
+  w->descs.assign(descs, descs + ndesc);
+  w->vec4 = phpc_f32_vec4_ok(descs, ndesc);
+  std::vector<F32Desc> tail;
+  w->config[0] = x3_tile(w->descs);
+  if (w->config[0] == 2) rm_split_tail(w->descs, 128, 128, phpc_device().cus, tail, 3);
+  w->config[1] = x3_tile(tail);
+  w->head = (int)w->descs.size();
+  w->tiles[0] = phpc_f32_plan_tiles(w->descs.data(), w->head, w->config[0]);
+  w->tiles[1] = phpc_f32_plan_tiles(tail.data(), (int)tail.size(), w->config[1]);
+  w->descs.insert(w->descs.end(), tail.begin(), tail.end());
+}
+
+bool phpc_f32x3_in_register_ok(const F32Desc &d) { return 128L * d.lda * 4 < 0x7fffffffL && 32L * d.ldb * 4 < 0x7fffffffL; }
+
+// Whether a 3 x BF16 product that could take either is faster on slice planes, which cost 16 bytes
+// of traffic an element of A and B where the in-register kernel reads 4 once a tile: from k = 512
+// on with more than 256 rows and columns (1000 x 512 x 1000 23 us against 24, 512 x 4096 x 2000 77
+// against 141; at k = 256 18 against 16), and on narrower ones from k = 1024 on while the planes
+// stay in the last-level cache (128 x 1024 x 8192 37 us against 42; 128 x 512 x 8192 28 against 25,
+// 128 x 4096 x 8192 164 against 138, 32 x 4096 x 40000 590 against 275).
+bool phpc_f32x3_planes_pay(const F32Desc &d) {
+  return std::min(d.m, d.n) > 256 ? d.k >= 512 : d.k >= 1024 && ((long)d.m + d.n) * d.k <= 16L << 20;
+}
+
+namespace {
+int x3_launch(const F32Desc *descs_dev, const F32Desc *descs_host, int ndesc, int total_tiles, int config, bool vec4,
+              int grid, hipStream_t stream) {
+  if (ndesc <= 0 || total_tiles <= 0) return PHPC_OK;
+  for (int i = 0; i < ndesc; ++i)
+    if (!phpc_f32x3_in_register_ok(descs_host[i])) return phpc_set_error(PHPC_ERR_ARG, "leading dimension too large");
   static void (*const kernels[2][2])(F32Batch) = {{f32x3_gemm_kernel<64, 64, 2, 1>, f32x3_gemm_kernel<64, 64, 2, 4>},
                                                   {f32x3_gemm_kernel<128, 128, 4, 1>, f32x3_gemm_kernel<128, 128, 4, 4>}};
   void (*fn)(F32Batch) = kernels[config == 2][vec4];
@@ -620,6 +662,14 @@ int phpc_f32x3_launch(const F32Desc *descs_dev, const F32Desc *descs_host, int n
   hipLaunchKernelGGL(fn, dim3(G), dim3(threads), 0, stream, b);
   PHPC_HIP(hipGetLastError());
   return PHPC_OK;
+}
+}  // namespace
+
+int phpc_f32x3_launch(const F32X3Work &w, const F32Desc *descs_dev, int grid, hipStream_t stream) {
+  const int n = (int)w.descs.size();
+  if (int rc = x3_launch(descs_dev, w.descs.data(), w.head, w.tiles[0], w.config[0], w.vec4, grid, stream)) return rc;
+  return x3_launch(descs_dev ? descs_dev + w.head : nullptr, w.descs.data() + w.head, n - w.head, w.tiles[1], w.config[1],
+                   w.vec4, grid, stream);
 }
 
 // Launch the grouped kernel over device-resident descriptors (planned for config id).
@@ -666,17 +716,17 @@ extern "C" int phpc_sgemm_device(const float *dA, long lda, const float *dB, lon
   d.m = m;
   d.n = n;
   d.k = k;
-  const bool vec4 = phpc_f32_vec4_ok(&d, 1);
   int rc = PHPC_OK;
   bool planes = false;
   const bool large = (long)m * n >= 2048L * 2048 && k >= 256;
   if (method == PHPC_SGEMM_BF16X3) {
-    // Slice planes from one 64x64 tile per CU on: 1000^3 29 us against 40 on the in-register
-    // kernel, 1500^3 57 against 88; at 512^3, 18 against 21, the one launch that needs no
-    // workspace is the simpler. A stream being captured takes a workspace (which may grow, and
-    // waits for its last user) only where it always did.
+    // Slice planes from one 64x64 tile per CU on, where they pay or rows lie too far apart for the
+    // in-register kernel; at 512^3, 18 us against 23, the one launch that needs no workspace is the
+    // simpler. A stream being captured takes a workspace (which may grow, and waits for its last
+    // user) only where it always did.
     planes = large;
-    if (!large && (long)((m + 63) / 64) * ((n + 63) / 64) >= phpc_device().cus && k >= 128 && phpc_bf3_fits(k)) {
+    if (!large && rm_tiles(d, 64, 64) >= phpc_device().cus && (phpc_f32x3_planes_pay(d) || !phpc_f32x3_in_register_ok(d)) &&
+        phpc_bf3_fits(k)) {
       hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
       const hipError_t e = hipStreamIsCapturing((hipStream_t)stream, &st);
       if (e != hipSuccess) (void)hipGetLastError();
@@ -696,9 +746,9 @@ extern "C" int phpc_sgemm_device(const float *dA, long lda, const float *dB, lon
     if (!planes) (void)hipGetLastError();  // the allocation's, before the launch below asks for its own
   }
   if (method == PHPC_SGEMM_BF16X3 && !planes) {
-    const int cfg = (long)((m + 127) / 128) * ((n + 127) / 128) >= phpc_device().cus ? 2 : 0;
-    const int tiles = phpc_f32_plan_tiles(&d, 1, cfg);
-    rc = phpc_f32x3_launch(nullptr, &d, 1, tiles, cfg, vec4, 0, (hipStream_t)stream);
+    F32X3Work w;
+    phpc_f32x3_prepare(&d, 1, &w);
+    rc = phpc_f32x3_launch(w, nullptr, 0, (hipStream_t)stream);
   } else if (method != PHPC_SGEMM_BF16X3) {
     if (g_f32_direct && phpc_f32_direct_ok(&d, 1)) {
       F32Work w;
@@ -721,7 +771,7 @@ extern "C" int phpc_sgemm_device(const float *dA, long lda, const float *dB, lon
       const long work = (long)((m + 127) / 128) * ((n + 127) / 128);
       const int cfg = work >= 2L * phpc_device().cus ? 2 : 0;
       const int tiles = phpc_f32_plan_tiles(&d, 1, cfg);
-      rc = phpc_f32_launch(nullptr, &d, 1, tiles, cfg, vec4, 0, (hipStream_t)stream);
+      rc = phpc_f32_launch(nullptr, &d, 1, tiles, cfg, phpc_f32_vec4_ok(&d, 1), 0, (hipStream_t)stream);
     }
   }
   return rc ? rc : phpc_set_error(PHPC_OK, nullptr);

@@ -19,12 +19,12 @@ struct phpc_plan {
   size_t descs_cap = 0;
   int config = 0;
   bool vec = false;
-  int x3_tile = 2;  // 3 x BF16 on the in-register kernel: its tiles (0: 64x64, 2: 128x128)
   int total_tiles = 0;
   int grid = 0;
   double tuned_ms = 0.0;
   F64Work w64;  // FP64: the items numbered for the configuration, as descs_dev holds them
   F32Work w32;  // FP32 on the direct kernels: likewise
+  F32X3Work wx3;  // 3 x BF16 on the in-register kernel: likewise
   // 3 x BF16 plans on slice planes (configurations kF32X3PlanesConfig + g): the planes,
   // the cut list and the level launch's items
   Bf3Planes planes;
@@ -74,15 +74,13 @@ int plan_upload(phpc_plan *p, int id, hipStream_t s) {
     p->total_tiles = p->planes.work.total;
     p->config = id;
     return PHPC_OK;
+  } else if (p->dtype == PHPC_F32X3) {
+    phpc_f32x3_prepare(p->d32.data(), p->count, &p->wx3);
+    p->total_tiles = p->wx3.tiles[0] + p->wx3.tiles[1];
+    bytes = sizeof(F32Desc) * p->wx3.descs.size();
+    src = p->wx3.descs.data();
   } else {
-    // the in-register 3 x BF16 kernel takes 128x128 tiles (config 2's) from one a CU on, else
-    // 64x64 (config 0's): 512^3 23 us, 50 on 128x128 tiles of 4 waves
-    p->total_tiles = phpc_f32_plan_tiles(p->d32.data(), p->count, p->dtype == PHPC_F32X3 ? 2 : id);
-    p->x3_tile = 2;
-    if (p->dtype == PHPC_F32X3 && p->total_tiles < phpc_device().cus) {
-      p->x3_tile = 0;
-      p->total_tiles = phpc_f32_plan_tiles(p->d32.data(), p->count, 0);
-    }
+    p->total_tiles = phpc_f32_plan_tiles(p->d32.data(), p->count, id);
     p->vec = phpc_f32_vec4_ok(p->d32.data(), p->count);
     bytes = sizeof(F32Desc) * p->count;
     src = p->d32.data();
@@ -113,8 +111,7 @@ int launch(phpc_plan *p, hipStream_t s) {
     return phpc_f32_launch_direct(p->w32, p->descs_dev, p->grid, s);
   if (p->dtype == PHPC_F32X3 && p->config >= kF32X3PlanesConfig) return p->planes.run(s, p->grid);
   if (p->dtype == PHPC_F32X3)
-    return phpc_f32x3_launch((const F32Desc *)p->descs_dev, p->d32.data(), p->count, p->total_tiles, p->x3_tile, p->vec,
-                             p->grid, s);
+    return phpc_f32x3_launch(p->wx3, (const F32Desc *)p->descs_dev, p->grid, s);
   return phpc_f32_launch((const F32Desc *)p->descs_dev, p->d32.data(), p->count, p->total_tiles, p->config, p->vec,
                          p->grid, s);
 }

@@ -155,8 +155,19 @@ struct Bf3Planes {
   ~Bf3Planes() { release(); }
 };
 
-int phpc_f32x3_launch(const F32Desc *descs_dev, const F32Desc *descs_host, int ndesc, int total_tiles, int config,
-                      bool vec4, int grid, hipStream_t stream);
+bool phpc_f32x3_planes_pay(const F32Desc &d);
+bool phpc_f32x3_in_register_ok(const F32Desc &d);  // its 32-bit buffer offsets reach A's and B's rows
+// Launches of the in-register 3 x BF16 kernel: the first `head` GEMMs on the tiles of config[0] (0:
+// 64x64, 2: 128x128), the rest in a second launch on those of config[1]. One GEMM travels with its
+// launch; otherwise the caller holds a copy of descs on the device.
+struct F32X3Work {
+  std::vector<F32Desc> descs;
+  int head = 0;
+  int config[2] = {}, tiles[2] = {};
+  bool vec4 = false;
+};
+void phpc_f32x3_prepare(const F32Desc *descs, int ndesc, F32X3Work *w);
+int phpc_f32x3_launch(const F32X3Work &w, const F32Desc *descs_dev, int grid, hipStream_t stream);
 int phpc_f32_launch(const F32Desc *descs_dev, const F32Desc *descs_host, int ndesc, int total_tiles, int id, bool vec4,
                     int grid, hipStream_t stream);
 

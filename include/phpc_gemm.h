@@ -96,8 +96,8 @@ int phpc_num_configs(void);
  * FP32 configuration of plans created without autotuning (-1, default = 3; 0-2 =
  * register-staged 64x64, 128x64, 128x128; 3 = the direct-to-LDS kernels on tiles picked by
  * the work; all give the same bits); key 8 = configuration of 3 x BF16 (PHPC_F32X3) plans
- * created without autotuning (-1 = by work, default: 2 for fewer 64x64 tiles than CUs, 6 for at
- * least two 128x128 tiles per CU, else 4; 2 = BF16 slices cut in registers; 4, 5, 6 = BF16 slice
+ * created without autotuning (-1 = by work, default: 2 for fewer 64x64 tiles than CUs or mostly
+ * items of no more than 256 rows or columns, 6 for at least two 128x128 tiles per CU, else 4; 2 = BF16 slices cut in registers; 4, 5, 6 = BF16 slice
  * planes cut once per operand, then one grouped launch on 64x64, 256x128 or 128x128 tiles, the
  * plan keeping the planes; all give the same bits). */
 int phpc_set_tuning(int key, int value);

@@ -214,3 +214,33 @@ def test_captured_bits_are_the_eager(m, k, n):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(C.view(torch.int32), want.view(torch.int32))
+
+
+# either side of the rule between planes and the in-register kernel, with 128x128 tiles in whole
+# rounds and the rest apart (by columns, by rows)
+@pytest.mark.parametrize("m,k,n", [(100, 70, 40000), (20000, 65, 200), (256, 1024, 8192), (256, 2100, 8192),
+                                   (257, 511, 4100), (257, 512, 4100), (2047, 130, 2047)])
+def test_products_beside_the_rule(m, k, n):
+    import torch
+    A, B, C0 = inputs(m, k, n, m + k)
+    C, D = C0.clone(), C0.clone()
+    phpc.sgemm_device(A, B, C, method=phpc.SGEMM_BF16X3)
+    torch.cuda.synchronize()
+    check(A, B, C0, C)
+    run_plan(4, [(A, B, D)])
+    assert torch.equal(C.view(torch.int32), D.view(torch.int32))
+
+
+@pytest.mark.parametrize("shapes", [[(100, 40, 40000)], [(90, 33, 300), (2000, 64, 2100), (200, 50, 5000)],
+                                    [(i % 90 + 1, 20 + i, 70) for i in range(300)]])
+def test_in_register_plan_in_two_launches(shapes):
+    import torch
+    ops = [inputs(*s, seed=i) for i, s in enumerate(shapes)]
+    outs = []
+    for cfg in (2, 4):
+        items = [(A, B, C.clone()) for A, B, C in ops]
+        run_plan(cfg, items)
+        outs.append([C for _, _, C in items])
+    for (A, B, C0), C, D in zip(ops, *outs):
+        check(A, B, C0, C)
+        assert torch.equal(C.view(torch.int32), D.view(torch.int32))
