@@ -1376,7 +1376,7 @@ int phpc_dgemm_split_ws(const double *dA, long lda, const double *dB, long ldb, 
     if (info) {
       info->slices = L;
       info->products = L;
-      info->launches = 8;
+      info->launches = 9;  // zeroing, four of statistics, two of residues, products, reconstruction
       // exact scaling leaves the two roundings of C += 2^(e_i + f_j - 2p) C'
       info->error_estimate = exact_scaling ? std::ldexp(1.0, -52) : crt_error_estimate(pbits, mra, mrb, k);
       info->method = 1;
@@ -1465,7 +1465,7 @@ int phpc_dgemm_split_ws(const double *dA, long lda, const double *dB, long ldb, 
   if (info) {
     info->slices = s_use;
     info->products = s_use * (s_use + 1) / 2;
-    info->launches = launches + 6;
+    info->launches = launches + 7;  // zeroing, four of statistics, two of slices
     info->error_estimate = est;
     info->method = method;
     info->int_bits = bits * s_use;

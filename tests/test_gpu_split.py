@@ -455,3 +455,20 @@ def test_crt_large_problem_kernel_ragged_k_matches_restatement(k, L):
     torch.cuda.synchronize()
     want = O.crt_gemm(A, B, C0.copy(), info.int_bits, L)
     assert np.array_equal(bits(dC.cpu().numpy()), bits(want))
+
+
+@pytest.mark.parametrize("method,slices,k,launches", [("crt", 0, 300, 9), ("slices", 6, 300, 6 + 7),
+                                                      ("slices", 8, 20000, 8 + 1 + 7), ("fp8", 5, 300, 5 + 7)])
+def test_launches_issued(method, slices, k, launches):
+    """Zeroing, four kernels of statistics, two of residues or slices; then the residue products and
+    the reconstruction, or a launch a level (at k = 20000 the largest of 8 takes two)."""
+    import torch
+    A, B = O.uniform((16, k), 4), O.uniform((k, 24), 5)
+    dC = torch.zeros((16, 24), dtype=torch.float64, device="cuda")
+    kind = {"crt": phpc.SPLIT_CRT, "slices": phpc.SPLIT_SLICES, "fp8": phpc.SPLIT_FP8}[method]
+    try:
+        info = phpc.dgemm_split_device(dev(A), dev(B), dC, slices=slices, method=kind)
+        torch.cuda.synchronize()
+    finally:
+        phpc.lib().phpc_split_set_method(phpc.SPLIT_CRT)
+    assert info.launches == launches
