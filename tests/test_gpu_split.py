@@ -458,10 +458,11 @@ def test_crt_large_problem_kernel_ragged_k_matches_restatement(k, L):
 
 
 @pytest.mark.parametrize("method,slices,k,launches", [("crt", 0, 300, 9), ("slices", 6, 300, 6 + 7),
-                                                      ("slices", 8, 20000, 8 + 1 + 7), ("fp8", 5, 300, 5 + 7)])
+                                                      ("slices", 8, 20000, 8 + 2 + 7), ("fp8", 5, 300, 5 + 7)])
 def test_launches_issued(method, slices, k, launches):
     """Zeroing, four kernels of statistics, two of residues or slices; then the residue products and
-    the reconstruction, or a launch a level (at k = 20000 the largest of 8 takes two)."""
+    the reconstruction, or a launch a level (at k = 20000, 20096 padded, an int32 sum holds six
+    slices, so the levels of seven and eight take two)."""
     import torch
     A, B = O.uniform((16, k), 4), O.uniform((k, 24), 5)
     dC = torch.zeros((16, 24), dtype=torch.float64, device="cuda")
