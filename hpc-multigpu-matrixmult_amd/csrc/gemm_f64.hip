@@ -522,6 +522,22 @@ int phpc_f64_grouped(const GemmDesc *descs, int ndesc, int grid, int config_id, 
   F64Work w;
   if (int rc = phpc_f64_prepare(descs, ndesc, config_id, false, &w)) return rc;
   if (w.list.empty()) return phpc_f64_launch(w, nullptr, grid, stream);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
+  if (capture == hipStreamCaptureStatusActive) {
+    // A replay would read what the buffer below holds by then: as many GEMMs a launch as it carries.
+    const std::vector<GemmDesc> all = w.descs;
+    for (size_t i = 0, n; i < all.size(); i += n) {
+      n = std::min<size_t>(2, all.size() - i);
+      if (int rc = phpc_f64_prepare(&all[i], (int)n, w.config, false, &w)) return rc;
+      if (!w.list.empty()) {  // two and their tails
+        n = 1;
+        if (int rc = phpc_f64_prepare(&all[i], 1, w.config, false, &w)) return rc;
+      }
+      if (int rc = phpc_f64_launch(w, nullptr, grid, stream)) return rc;
+    }
+    return PHPC_OK;
+  }
   // More GEMMs than travel with the launch: their list goes through one process-wide device
   // buffer. Callers on other streams may still have a launch queued that reads it, so the
   // buffer is rewritten only after the previous user's launch has finished (g_desc_done).

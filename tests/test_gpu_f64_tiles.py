@@ -140,3 +140,46 @@ def test_more_tiles_than_one_launch_starts(dtype):
     torch.cuda.synchronize()
     A.mul_(3.0).add_(1.0)
     assert torch.equal(A, C)
+
+
+# GEMMs that go through the shared descriptor buffer in eager calls: captured, their launches carry
+# them, and replays do not depend on what eager calls put into that buffer meanwhile
+@pytest.mark.parametrize("what", ["far_rows", "ranks", "ranks_with_tails"])
+def test_captured_lists(what):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(4)
+
+    def ints(*s):
+        return torch.randint(-8, 9, s, generator=g, device="cuda").double()
+
+    if what == "far_rows":
+        m, k, n, lda = 5, 37, 130, 34_000_000
+        A, B, C0 = ints(m, k), ints(k, n), ints(m, n)
+        far = torch.empty((m - 1) * lda + k, dtype=torch.float64, device="cuda").as_strided((m, k), (lda, 1))
+        far.copy_(A)
+    else:
+        N = 200 if what == "ranks" else 2700
+        A, B, C0 = ints(N, N), ints(N, N), ints(N, N)
+
+    def call(C, stream=None):
+        if what == "far_rows":
+            phpc.dgemm_device(far, B, C, stream=stream)
+        else:
+            phpc.summa_device(A, B, C, 3, 2, panel=97, mode=phpc.SUMMA_FUSED, stream=stream)
+
+    want = C0 + (A.cpu() @ B.cpu()).cuda()  # integers: exact in any order
+    C, D = C0.clone(), C0.clone()
+    call(D)
+    s, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=s):
+        call(C, s)
+    assert torch.equal(D, want)
+    X, Y, Z = ints(77, 77), ints(77, 77), ints(77, 77)
+    for _ in range(3):
+        C.copy_(C0)
+        phpc.summa_device(X, Y, Z, 7, 7, mode=phpc.SUMMA_FUSED)  # 49 GEMMs through the buffer
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C, want)
