@@ -514,22 +514,26 @@ int phpc_f32_prepare(const F32Desc *descs, int ndesc, F32Work *w) {
   w->descs.clear();
   w->total = w->tail_start = 0;
   long t64 = 0, t128 = 0;
+  int kmax = 0;
   for (int i = 0; i < ndesc; ++i) {
     if (descs[i].m <= 0 || descs[i].n <= 0 || descs[i].k <= 0) continue;
     w->descs.push_back(descs[i]);
     t64 += rm_tiles(descs[i], 64, 64);
     t128 += rm_tiles(descs[i], 128, 64);
+    kmax = std::max(kmax, descs[i].k);
   }
   const long cus = phpc_device().cus;
   // 128x64 tiles from four a CU on (two rounds of the two resident ones): 3000^3, 4.4 a CU, 404
-  // us against 416 on 64x64, but 2500^3, 3.1 a CU, 265 against 249. 32x32 tiles where 64x64 ones
-  // would leave CUs empty: 256^3 5.4 us against 9.5. From three quarters of them to one 64x64
-  // tile per CU, those in 8 waves on 64-deep slabs: 1000^3 21.9 us against 24.1 in 4 waves and
-  // 22.6 on 32x32, 1024 x 4096 x 1024 66 against 70 and 75; 800^3, 0.66 a CU, 17.6 against 15.2.
-  w->config = t128 >= 4 * cus                    ? kF32Big
-              : 4 * t64 > 3 * cus && t64 <= cus ? kF32One
-              : t64 >= cus                      ? kF32Mid
-                                                : kF32Small;
+  // us against 416 on 64x64, but 2500^3, 3.1 a CU, 265 against 249. 64x64 in 4 waves above one a CU
+  // (1.06 a CU, k = 1000: 27 us against 30 on 32x32). Up to one 64x64 tile a CU 32x32 tiles, which
+  // leave no CU empty (256^3 5.4 us against 9.5); but more than three quarters of one and k >= 1000,
+  // 64x64 in 8 waves on 64-deep slabs (0.76, 0.88 and 1.0 a CU: k = 3000 53 us each against 58, 59
+  // and 60 on 32x32; k = 1500 30.8, 30.9 and 31.5 against 32.2, 33.3 and 33.5; k = 700 19.8, 19.9 and 20.2
+  // against 18.0, 18.9 and 18.6; 0.70, k = 3000: 53 against 47).
+  w->config = t128 >= 4 * cus                     ? kF32Big
+              : t64 > cus                         ? kF32Mid
+              : 4 * t64 > 3 * cus && kmax >= 1000 ? kF32One
+                                                  : kF32Small;
   const F32RmConfig &c = kF32Rm[w->config];
   if (!phpc_f32_direct_ok(w->descs.data(), (int)w->descs.size()))
     return phpc_set_error(PHPC_ERR_ARG, "leading dimension too large");

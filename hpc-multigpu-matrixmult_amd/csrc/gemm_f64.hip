@@ -413,29 +413,37 @@ namespace {
 
 // Planner: by how many tiles the work gives the CUs. Measured on MI355X, with the neighbouring
 // choices:
-//   fewer 64x64 tiles than CUs: 32x32 tiles (512^3: 8.6 us against 20.4 on 64x64, N = 256:
-//     6.2 against 12.7), whose workgroups share a CU five at a time;
-//   from three quarters of them to one 64x64 tile per CU, those in 16 waves on 32-deep slabs,
-//     which hide each other's barriers where no second workgroup does (1024 x 4096 x 1024: 123
-//     us against 138 in 4 waves and 139 on 32x32; 1024^3 37.5 against 39.7 and 37.3;
-//     600 x 3000 x 900, 0.6 a CU, 92 against 79 on 32x32);
-//   then 64x64 tiles in 4 waves with a 32x32 tail (2048^3: 68 TFLOP/s against 54 on 32x32 alone);
+//   up to one 64x64 tile per CU: 32x32 tiles (512^3: 8.6 us against 20.4 on 64x64, N = 256:
+//     6.2 against 12.7), whose workgroups share a CU five at a time; but more than three quarters
+//     of a tile per CU and k >= 900, those in 16 waves on 32-deep slabs, which hide each other's
+//     barriers where no second workgroup does (0.76, 0.88 and 1.0 a CU: k = 3000 92, 92 and 94 us
+//     against 98, 100 and 103 on 32x32; k = 1300 45.7, 46.2 and 46.5 against 48.1, 48.4 and 49.6; k =
+//     400 21.5, 20.8 and 21.2 against 19.9, 19.2 and 19.4; 0.70, k = 3000: 92 against 79);
+//   then 64x64 tiles in 4 waves with a 32x32 tail (1.06 a CU, k = 3000: 120 us, 128 on 32x32 alone;
+//     2048^3: 68 TFLOP/s against 54); with panels from one a CU (1024^3 in panels of 256: 46 us
+//     against 54);
 //   from two 256x128 tiles per CU on, those (4096^3: 73.2 against 68; 16384^3: 74.8 against 65
-//     on 64x64). With panels, from six 192x128 tiles per CU on (four of 128x128 in a list), those:
-//     the largest whose waves have room for accumulators and the carried C (16384^3 in panels of
-//     256 122.9 ms against 127.8 on 128x128 in 16 waves and 126.4 on 64x64; 6000^3, 5.9 a CU, 6.26
-//     against 6.47 and 6.28; 5000^3, 4.2 a CU, 3.81 against 3.83 and 3.69; 10000^3 on 3 x 3 ranks
-//     as a plan 29.4, 31.0 on 128x128 in 8 waves). They load less of L2 per output than any
-//     smaller tile, which counts where launches of several streams meet on the GPU: the plan
-//     29.7 against 31.4 there, and 35 on 64x64.
+//     on 64x64);
+//   with panels, from six 192x128 tiles per CU on, those: the largest whose waves have room for
+//     accumulators and the carried C (16384^3 in panels of 256 122.9 ms against 127.8 on 128x128 in
+//     16 waves and 126.4 on 64x64; 6000^3, 5.9 a CU, 6.26 against 6.47 and 6.28; 5000^3, 4.2 a CU,
+//     3.81 against 3.83 and 3.69);
+//   lists with panels take them from four 128x128 tiles per CU on. Alone, 64x64 tiles are faster
+//     up to some ten of 192x128 a CU, but a plan's launches meet others on the GPU, where tiles
+//     that load less of L2 per output lose less (ranks of N = 4000, 4800, 7000, 8000 and 10000, 2.7 to
+//     17 a CU, three plans in turn: 1.92, 3.28, 10.7, 14.5, 29.5 ms a launch against 2.09, 3.45,
+//     11.3, 16.9 and 34.4 on 64x64; alone 2.05, 3.50, 10.9, 14.7 and 29.5 against 1.94, 3.19, 10.2, 14.9
+//     and 30.1).
 int config_for(const GemmDesc *descs, int ndesc, bool device_list) {
   long t64 = 0, t128 = 0, t192 = 0, t256 = 0;
+  int k = 0;
   bool mp = false;
   for (int i = 0; i < ndesc; ++i) {
     t64 += rm_tiles(descs[i], 64, 64);
     t128 += rm_tiles(descs[i], 128, 128);
     t192 += rm_tiles(descs[i], 192, 128);
     t256 += rm_tiles(descs[i], 256, 128);
+    k = std::max(k, descs[i].k);
     mp |= has_panels(descs[i]);
   }
   const long cus = phpc_device().cus;
@@ -443,8 +451,8 @@ int config_for(const GemmDesc *descs, int ndesc, bool device_list) {
     // key 0 may hold a configuration without panel-grouped variants
     return !device_list ? g_big_config_host : kConfigs[g_big_config].panels ? g_big_config : kBigPanels;
   if (!mp && t256 >= 2 * cus) return device_list ? g_big_single : g_big_single_host;
-  if (!mp && 4 * t64 > 3 * cus && t64 <= cus) return kOne;
-  return t64 >= cus ? kMid : kSmall;
+  if (t64 > cus || (mp && t64 == cus)) return kMid;
+  return !mp && 4 * t64 > 3 * cus && k >= 900 ? kOne : kSmall;
 }
 
 }  // namespace

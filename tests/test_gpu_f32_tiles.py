@@ -125,3 +125,27 @@ def test_short_rows_of_b(m, n, k):
         phpc.sgemm_device(A, wide[:, :1], D, method=phpc.SGEMM_FP32)
         torch.cuda.synchronize()
         assert torch.equal(D, C), (m, k, n)
+
+
+# beside the lines of the tile rule below one 64x64 tile per CU (256): k, and the tiles
+@pytest.mark.parametrize("m,k,n", [(1023, 999, 1000), (1023, 1000, 1000), (961, 1027, 1024), (800, 1000, 960),
+                                   (769, 1065, 1023), (1025, 1001, 1023)])
+def test_about_one_tile_per_cu(m, k, n):
+    import torch
+    A, B, C0 = inputs(m, k, n, m + k)
+    _, dA = on_view(A, float("nan"))
+    _, dB = on_view(B, float("nan"))
+    C = C0.clone()
+    phpc.sgemm_device(dA, dB, C, method=phpc.SGEMM_FP32)
+    torch.cuda.synchronize()
+    assert torch.equal(C, staged(A, B, C0))
+    x, y, z = (t.double() for t in (A, B, C0))
+    want = z.clone()
+    phpc.dgemm_device(x, y, z)
+    phpc.set_launch_policy(0, 2, 0)  # register-staged
+    try:
+        phpc.dgemm_device(x, y, want)
+        torch.cuda.synchronize()
+    finally:
+        phpc.set_launch_policy(0, -1, 0)
+    assert torch.equal(z, want)
