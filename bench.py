@@ -1,7 +1,7 @@
 """Benchmark: FP64 SUMMA on one MI355X (N = 16384, emulated 4 x 4 grid, k-panel 256).
 
 One step = one SUMMA pass C += A*B over the 64 panels for all 16 emulated ranks, run by
-the plain FP64-MFMA path (one persistent grouped launch). Inputs are uniform[-1,1) from
+the plain FP64-MFMA path (one grouped launch). Inputs are uniform[-1,1) from
 fixed seeds and resident in HBM before the timed region starts. Prints one JSON line.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W]
@@ -175,7 +175,7 @@ def grouped_bench(phpc, seed=21):
     out["fp64_n10000_grid3x3"] = {"tflops": round(2.0 * N ** 3 / (ms * 1e-3) / 1e12, 3), "ms": round(ms, 3),
                                   "blocks": "3334/3333/3333", "panel": N // 3, "config": info["config"],
                                   "tiles": info["tiles"], "err_cw_max_sampled": cw, "err_nw_sampled": nw,
-                                  "launch": "one persistent panel-grouped launch for all 9 rank blocks and all "
+                                  "launch": "one panel-grouped launch for all 9 rank blocks and all "
                                             "k panels (3333, 3333, 3333, 1), hipGraph replay"}
     plan.close()
     del A, B, C, items
@@ -230,7 +230,7 @@ def grouped_bench(phpc, seed=21):
         if dtype == phpc.F32X3:
             launch = ("one batched kernel cutting every A and B into BF16 slice planes + one launch of all "
                       "six products for all 512 GEMMs" if info["config"] >= 4 else
-                      "one persistent 3 x BF16 kernel for all 512 GEMMs")
+                      "the in-register 3 x BF16 kernel for all 512 GEMMs")
         else:
             launch = ("one direct-to-LDS launch for all 512 GEMMs (operands read in place)" if info["config"] == 3
                       else "one persistent kernel for all 512 GEMMs")

@@ -1,7 +1,7 @@
 // FP32 grouped GEMM on gfx950 matrix cores: C += A*B for a list of independent row-major FP32
 // GEMMs of any shapes, one launch. Two families: the direct kernels (gemm_rm.h,
 // v_mfma_f32_16x16x4f32), and the register-staged ones below (v_mfma_f32_32x32x2f32), for tuning
-// and for leading dimensions of B that do not fit the direct kernels' 32-bit offsets. Both sum
+// and for rows of B too far apart and rows of A too long for the direct kernels' 32-bit offsets. Both sum
 // each output as one FMA chain in k order: the same bits.
 //
 // The register-staged kernels: a BM x BN macro tile per workgroup, 4 waves in a

@@ -249,25 +249,20 @@ struct RmElem;
 template <>
 struct RmElem<double> {
   typedef double acc_t __attribute__((ext_vector_type(4)));
-  typedef double __attribute__((address_space(1))) global_t;
   static constexpr int CYCLES = 64;  // of a SIMD per MFMA
   static __device__ __forceinline__ acc_t mfma(double a, double b, acc_t c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
-  // row of accumulator r in lane group g
-  static __device__ __forceinline__ int row(int r, int g) { return 4 * r + g; }
   // B slot rotation of k row k (chunks per row cpb): see the LDS layout below
   static constexpr __device__ __forceinline__ int swz_b(int k, int) { return (k & 1) << 3; }
 };
 template <>
 struct RmElem<float> {
   typedef float acc_t __attribute__((ext_vector_type(4)));
-  typedef float __attribute__((address_space(1))) global_t;
   static constexpr int CYCLES = 32;
   static __device__ __forceinline__ acc_t mfma(float a, float b, acc_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
-  static __device__ __forceinline__ int row(int r, int g) { return 4 * g + r; }
   static constexpr __device__ __forceinline__ int swz_b(int k, int cpb) {
     return cpb >= 16 ? (k & 3) << 2 : ((k >> 1) & 1) << 2;
   }
@@ -361,7 +356,6 @@ __device__ __forceinline__ void rm_tile(const Desc &d, int row0, int col0) {
   using K = RmShape<E, BM, BN, WM, WN, BK, STAGES>;
   using X = RmElem<E>;
   using acc_t = typename X::acc_t;
-  using global_t = typename X::global_t;
   constexpr int SZ = K::SZ, CH = K::CH;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int tid = threadIdx.x;

@@ -140,10 +140,9 @@ extern "C" int phpc_plan_create(int dtype, const phpc_gemm_item *items, int coun
     if (it.m == 0 || it.n == 0 || it.k == 0) continue;
     live.push_back(it);
   }
-  // Items in decreasing k: a tile's time grows with k, and the persistent workgroups take
-  // tiles round-robin from the flat list, so tiles of similar cost then share each round
-  // and the workgroups finish together (on log-uniform k, the slowest of 512 workgroups
-  // would otherwise carry about 18% more than the mean). Outputs do not depend on the order.
+  // Items in decreasing k: a tile's time grows with k, and tiles start in the list's order (a
+  // workgroup each, or in rounds of the persistent kernels), so that the long ones start first
+  // and short ones fill the end. Outputs do not depend on the order.
   std::stable_sort(live.begin(), live.end(),
                    [](const phpc_gemm_item &a, const phpc_gemm_item &b) { return a.k > b.k; });
   p->count = (int)live.size();

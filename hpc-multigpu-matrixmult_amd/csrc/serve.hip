@@ -6,8 +6,8 @@
 // operand arena, a single device allocation sized to the memory budget that is
 // sub-allocated at admission, so no driver allocation sits on the request path. Requests too small to fill the GPU on
 // their own (fewer output tiles than compute units) are batched: requests of the
-// head's kind and load width that are waiting join its launch, one persistent grouped
-// kernel over all their tiles. Large requests run alone, since they fill the GPU by
+// head's kind and load width that are waiting join its launch, one grouped
+// launch over all their tiles. Large requests run alone, since they fill the GPU by
 // themselves. Workers run concurrently, so a batch being prepared or finished overlaps
 // the one computing. Latency is measured from submission to completion.
 #include "phpc_internal.h"

@@ -400,10 +400,10 @@ __device__ __forceinline__ int i8_swz(int r) {
   return (r * CPR / SD) & (CPR - 1);
 }
 
-// F8 = false: int8 operands, int32 sums (level or residue epilogue). F8 = true: FP8-E4M3
+// F8 = false: int8 operands, int32 sums, FP64 level epilogue. F8 = true: FP8-E4M3
 // operands (16 per chunk); the chunks of two k steps make one lane's 32 bytes of
 // v_mfma_scale_f32_32x32x64_f8f6f4 at unit scales (A and B take the same bytes, so the sum
-// runs over the same 64 k), FP32 sums that stay exact integers below 2^24, FP64 level epilogue.
+// runs over the same 64 k), FP32 sums that stay exact integers below 2^24, the same epilogue.
 // The byte layout and the pipeline are the same.
 // The operands of one level product as the tile code reads them (wave-uniform values):
 // read once per product.

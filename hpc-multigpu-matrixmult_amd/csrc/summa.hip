@@ -5,7 +5,7 @@
 // column j (row t % p) broadcast it (:63-89); every rank then runs the local update
 // C_ij += A(R_i, t) * B(t, C_j) (:93). On one GPU every rank sees the whole of A and B
 // in HBM, so:
-//   FUSED     one persistent grouped launch covers all p*q rank blocks; each tile walks
+//   FUSED     one grouped launch covers all p*q rank blocks; each tile walks
 //             the panels in order, summing each panel from zero and adding it to the C
 //             value carried in registers, i.e. exactly the sequence of per-step updates;
 //   STEPWISE  per panel, the non-owners' receive buffers are produced by a strided ->

@@ -344,13 +344,16 @@ def num_configs():
     return lib().phpc_num_configs()
 
 
-TUNE_F32_TRANSPOSED_A = 6
+TUNE_F32_DIRECT = 6
+TUNE_F32_TRANSPOSED_A = TUNE_F32_DIRECT  # its name while that path read a transposed copy of A
 TUNE_F32_PLAN_CONFIG = 7
 
 
 def set_tuning(key, value):
-    """One tuning knob (phpc_set_tuning): keys 0-5 pick FP64 configs, key 6 switches
-    FP32 products between the direct-to-LDS kernels (1) and the register-staged ones (0), key 7 sets the FP32 configuration of plans created without autotuning (-1 = by work)."""
+    """One tuning knob (phpc_set_tuning): keys 0-5 pick FP64 configs, tile order and swizzle, key 6
+    switches FP32 products between the direct-to-LDS kernels (1) and the register-staged ones
+    (0), keys 7 and 8 set the FP32 and the 3 x BF16 configuration of plans created without
+    autotuning (-1 = by work)."""
     check(lib().phpc_set_tuning(key, value))
 
 

@@ -81,7 +81,7 @@ int phpc_dgemm_vendor_device(const double *dA, long lda, const double *dB, long 
  * Launch policy for the FP64 kernels:
  *   honor_grid : 1 -> use grid_width*grid_height workgroups where the caller passes them
  *   config_id  : -1 -> planner's choice; else a fixed tile configuration (0..n-1)
- *   grid       : > 0 -> fixed persistent workgroup count; 0 -> planner's choice
+ *   grid       : > 0 -> fixed workgroup count, which walk the tiles; 0 -> planner's choice
  */
 int phpc_set_launch_policy(int honor_grid, int config_id, int grid);
 int phpc_num_configs(void);

@@ -1,6 +1,6 @@
 /*
- * libphpc — grouped GEMM plans: many independent row-major GEMMs (FP64 or FP32) in ONE
- * persistent launch, with autotuned tiles and optional hipGraph capture.
+ * libphpc — grouped GEMM plans: many independent row-major GEMMs (FP64 or FP32) in one
+ * launch, with autotuned tiles and optional hipGraph capture.
  *
  * No single counterpart in the reference. Its closest relative is the per-rank local
  * GEMM of the SUMMA loop (src/phpc_summa.c:93), which the reference issues as one call
@@ -41,12 +41,14 @@ typedef struct phpc_plan *phpc_plan_t;
  * (planner rule, or the fastest measured one with PHPC_PLAN_AUTOTUNE; tuned choices are
  * cached per shape list for the life of the process). */
 int phpc_plan_create(int dtype, const phpc_gemm_item *items, int count, int flags, void *stream, phpc_plan_t *plan);
-/* One persistent launch computing every item, stream-ordered. */
+/* One launch computing every item, stream-ordered (3 x BF16: the cut of the operands and the
+ * product, or up to two launches of the in-register kernel). */
 int phpc_plan_launch(phpc_plan_t plan, void *stream);
 /* Same launch replayed from a hipGraph captured on the first call (stream must not be
  * NULL: the capture needs a created stream). */
 int phpc_plan_graph_launch(phpc_plan_t plan, void *stream);
-/* config: tile configuration index; tiles: total tiles; grid: persistent workgroups;
+/* config: tile configuration index; tiles: total tiles; grid: workgroups (0: the
+ * configuration's own count);
  * tuned_ms: best time measured by the autotuner (0 if not tuned). */
 int phpc_plan_info(phpc_plan_t plan, int *config, int *tiles, int *grid, double *tuned_ms);
 void phpc_plan_destroy(phpc_plan_t plan);

@@ -3,7 +3,7 @@
  * at any time. Their operands live in an HBM arena sized to the memory budget; a
  * request is admitted (FIFO) when a worker slot is free and its operands fit. Workers
  * run concurrently on their own HIP streams. Requests too small to fill the GPU alone
- * are batched with waiting requests of the same kind into one persistent grouped
+ * are batched with waiting requests of the same kind into one grouped
  * launch; large requests run alone.
  *
  * No counterpart in the reference (its driver runs one GEMM per program run,

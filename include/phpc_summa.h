@@ -31,13 +31,13 @@ int phpc_grid_dims(phpc_grid_t grid, int dims[2]);
 int phpc_grid_set_panel(phpc_grid_t grid, int panel);
 int phpc_grid_get_panel(phpc_grid_t grid);
 /* Execution mode of phpc_gemm_summa_cuda / phpc_summa_device:
- *   PHPC_SUMMA_FUSED    one persistent launch over all ranks, walking the panels with
+ *   PHPC_SUMMA_FUSED    one launch over all ranks, walking the panels with
  *                       each rank's C tile kept in registers (default)
  *   PHPC_SUMMA_STEPWISE per panel: pack the broadcast panels (strided -> packed, as the
  *                       MPI_Type_vector sends do), then one grouped local-update launch
  *   PHPC_SUMMA_VENDOR   the STEPWISE schedule with rocBLAS dgemm as the local GEMM
  *                       (phpc_summa_device only)
- *   PHPC_SUMMA_CHAINED  one persistent launch, one FMA chain per output over all panels
+ *   PHPC_SUMMA_CHAINED  one launch, one FMA chain per output over all panels
  *                       (C is not rounded between panels): the arithmetic of a single
  *                       local-GEMM call over the full k; the fastest FP64 schedule
  *   PHPC_SUMMA_SPLIT    every rank's update over the full k by the split-precision CRT
@@ -88,7 +88,7 @@ int phpc_gemm_summa(gemm_t f, phpc_grid_t grid, const double *A, const double *B
 /* ---------------- device-resident extensions ---------------- */
 
 /* SUMMA on device pointers (N x N, row-major, ld = N), stream-ordered, any mode above.
- * panel 0 = N / lcm(p, q). wg > 0 fixes the persistent grid. */
+ * panel 0 = N / lcm(p, q). wg > 0 fixes the workgroup count. */
 int phpc_summa_device(int p, int q, int panel, int mode, const double *dA, const double *dB, double *dC, int N,
                       int wg, void *stream);
 
