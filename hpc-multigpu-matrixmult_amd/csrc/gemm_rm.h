@@ -406,8 +406,8 @@ __device__ __forceinline__ void rm_tile(const Desc &d, int row0, int col0) {
 
     // Every 1 KiB block is addressed from its own first row (ARB or BRB rows, uniform), so one
     // lane offset serves all of an operand's blocks. A rows past m_rem lie at or beyond
-    // num_records and read zero (k rides in the scalar offset, which the range check leaves
-    // out); B chunks past n_rem go out of range here.
+    // num_records and read zero (k rides in the scalar offset, which the range check adds: within
+    // a row of lda >= k it stays below); B chunks past n_rem go out of range here.
     rsrc_t rA[K::PA];
 #pragma unroll
     for (int u = 0; u < K::PA; ++u) {

@@ -492,8 +492,8 @@ __device__ __forceinline__ void level_tile(const LevelArgs &args, const LevelOps
       for (int u = 0; u < K::PER; ++u) {
         const int blk = wave + u * K::NW;
         const bool isA = u < PA;
-        // the range check applies to the lane offset (past num_records reads zero); k
-        // rides in soffset
+        // past num_records reads zero; k rides in soffset, which the range check adds and
+        // which stays within a row
         const uint32_t go = isA ? ga0 + (uint32_t)u * gstep_a : gb0 + (uint32_t)(u - PA) * gstep_b;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(isA ? rA : rB, (lds_void *)(stage + blk * 1024), 16, go,
                                                   kb, 0, 0);
